@@ -26,28 +26,30 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Wall", "-Wno-unus
 DEVICE = ["--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
           "-fno-gpu-rdc"]
 
-SOURCES = [
-    ("dn_kernels.hip", True),
-    ("dn_core.cpp", False),
-    ("dn_setup.cpp", False),
-    ("dn_dropin.cpp", False),
-    ("dn_fwi.cpp", False),
-    ("dn_io.cpp", False),
-    ("dn_unet.hip", True),
-    ("dn_unet.cpp", False),
-    ("dn_gradproc.hip", True),
-    ("dn_stf.hip", True),
-    ("dn_misfit.hip", True),
-    ("dn_misfit_noalloc.hip", True),
+# (source, flags[, object name]); the tile step is compiled once per stencil
+# half-order, so that the objects build in parallel
+SOURCES = [("dn_tile.hip", ["-DDN_TILE_K=%d" % k], "dn_tile_k%d" % k) for k in (4, 6, 5, 3, 2, 1)] + [
+    ("dn_kernels.hip", []),
+    ("dn_core.cpp", []),
+    ("dn_setup.cpp", []),
+    ("dn_dropin.cpp", []),
+    ("dn_fwi.cpp", []),
+    ("dn_io.cpp", []),
+    ("dn_unet.hip", []),
+    ("dn_unet.cpp", []),
+    ("dn_gradproc.hip", []),
+    ("dn_stf.hip", []),
+    ("dn_misfit.hip", []),
+    ("dn_misfit_noalloc.hip", []),
 ]
 
 
-def compile_one(src, device, objdir):
+def compile_one(src, flags, objdir, name=None):
     path = os.path.join(CSRC, src)
-    obj = os.path.join(objdir, src + ".o")
+    obj = os.path.join(objdir, (name or src) + ".o")
     # host translation units include the HIP runtime and are compiled as HIP
     # as well (for gfx950 only) so no default offload target sneaks in
-    cmd = [HIPCC] + COMMON + ["-x", "hip"] + DEVICE
+    cmd = [HIPCC] + COMMON + ["-x", "hip"] + DEVICE + flags
     cmd += ["-c", path, "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
@@ -63,11 +65,10 @@ def compile_one(src, device, objdir):
 def build(jobs=8, verbose=True):
     if not os.path.exists(HIPCC):
         raise RuntimeError("hipcc not found at %s" % HIPCC)
-    srcs = [(s, d) for s, d in SOURCES if os.path.exists(os.path.join(CSRC, s))]
     objdir = tempfile.mkdtemp(prefix="dnbuild_")
     try:
         with ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
-            objs = list(ex.map(lambda sd: compile_one(sd[0], sd[1], objdir), srcs))
+            objs = list(ex.map(lambda t: compile_one(t[0], t[1], objdir, *t[2:]), SOURCES))
         tmp = LIB + ".tmp"
         cmd = [HIPCC, "-shared", "-fPIC", "--offload-arch=gfx950", "-o", tmp] + objs
         r = subprocess.run(cmd, capture_output=True, text=True)

@@ -211,7 +211,7 @@ static void free_batch(dn_ctx *c)
     dfree_t(c->d_seis); dfree_t(c->d_resid); dfree_t(c->d_snap); dfree_t(c->d_snap16); dfree_t(c->d_snap_scale);
     dfree_t(c->d_stage); dfree_t(c->d_stage_max);
     dfree_t(c->d_Ws); dfree_t(c->d_Wr); dfree_t(c->d_gu_shot); dfree_t(c->d_grho_shot); dfree_t(c->d_part);
-    dfree_t(c->d_shot_map);
+    dfree_t(c->d_shot_map); dfree_t(c->d_slots);
     c->cur_map.clear();   // the shot map must be uploaded again into the new workspace
     c->batch_cap = 0;
     c->batch_nt_max = 0;
@@ -766,6 +766,7 @@ int dn_ensure_batch(dn_ctx *c, int want, bool gradient)
     HIPCHK(c, dalloc(&c->d_grho_shot, S * nxny));
     HIPCHK(c, dalloc(&c->d_part, S * c->ntr * 2));
     HIPCHK(c, dalloc(&c->d_shot_map, S));
+    HIPCHK(c, dalloc(&c->d_slots, S));
     c->batch_has_snap = gradient;
     if (gradient) {
         const size_t ns = (size_t)dn_nsnap(c);
@@ -830,6 +831,24 @@ static int choose_rows(const dn_ctx *c, int nshots, int nstrips)
     return best;
 }
 
+// Rows per wave of the tile step, 0 for the strip step.  Tiles (64 columns x
+// 8 rows per wave) are faster than strips at every size measured; the strips
+// run where the caller asks for a shape of theirs (rows per segment, two shots
+// per wave, a workgroup layout) and with BOUNDARY 1 on grids so narrow that a
+// tile's columns would wrap twice.  One row per wave halves the work in a
+// workgroup's chain but recomputes 2K-1 rows for 8 instead of 16: it wins
+// while the 16-row tiles would leave CUs without a workgroup.  Microseconds
+// per step with 1 / 2 rows: 400x120 (56 tiles of 16 rows) 5.4 / 7.0,
+// 440x177x3 (252) 8.8 / 9.1, 392x563x2 (504) 11.7 / 11.7, 3366x220 (742)
+// 17.1 / 16.7, 1200x300x8 (2888) 44.8 / 43.1.
+static int choose_tile(const dn_ctx *c, int nshots)
+{
+    if (c->rows_req > 0 || c->two_shots || c->sg > 1) return 0;
+    if (c->g.periodic && c->g.nx < 2 * kWave) return 0;
+    const long long tiles16 = (long long)nshots * ((c->g.nx + kWave - 1) / kWave) * ((c->g.ny + 15) / 16);
+    return tiles16 <= 256 ? 1 : 2;
+}
+
 void dn_fill_step_common(dn_ctx *c, StepArgs &a, int n)
 {
     const Geo &g = c->g;
@@ -852,6 +871,16 @@ void dn_fill_step_common(dn_ctx *c, StepArgs &a, int n)
     a.nblocks_sg8 = (a.nblocks_sg + 7) / 8;
     a.nblocks2 = (n >= 2 && c->two_shots) ? ((n + 1) / 2) * a.ngroups * a.nsegs : 0;
     a.nblocks2_8 = (a.nblocks2 + 7) / 8;
+    a.tl_rw = choose_tile(c, n);
+    if (a.tl_rw > 0) {
+        a.tl_w = kWave;
+        a.tl_h = 8 * a.tl_rw;
+        a.tl_ny = (g.ny + a.tl_h - 1) / a.tl_h;
+        a.tl_nblk = n * ((g.nx + a.tl_w - 1) / a.tl_w) * a.tl_ny;
+        a.tl_nblk8 = (a.tl_nblk + 7) / 8;
+        a.tl_mshots = 0xffffffffu / (unsigned)n;
+        a.tl_mny = 0xffffffffu / (unsigned)a.tl_ny;
+    }
     a.DT = c->p.dt;
     a.DH = c->p.dh;
     a.dhi = (c->p.L > 0) ? (float)(1.0 / (double)c->p.dh) : c->p.dt / c->p.dh;
@@ -860,12 +889,6 @@ void dn_fill_step_common(dn_ctx *c, StepArgs &a, int n)
     a.hcy6 = c->hc[5];  // update_v_PML.c:469 (Q6)
     a.pml = c->pml;
     a.bfield = c->d_b;
-    a.uip = c->d_uip;
-    a.ujp = c->d_ujp;
-    a.fipjp = c->d_fipjp;
-    a.fcoef = c->d_f;
-    a.dip = c->d_dip;
-    a.dcoef = c->d_d;
     a.spk = c->d_spk;
     for (int l = 0; l < kMaxL; ++l) {
         a.bip[l] = c->bip[l];
@@ -877,6 +900,7 @@ void dn_fill_step_common(dn_ctx *c, StepArgs &a, int n)
     a.pvx = c->d_pvx;
     a.pvy = c->d_pvy;
     a.shot_map = c->d_shot_map;
+    a.slots = c->d_slots;
     a.status = c->d_status;
     a.shot_nt = c->d_shot_nt;
     a.src_off = c->d_src_off;
@@ -919,7 +943,7 @@ static int enqueue_steps(dn_ctx *c, StepArgs &a, int n, bool adjoint, bool pack_
     for (int k = 0; k < count; ++k) {
         const int nt = nt0 + k;
         a.nt = nt;
-        a.nt_base = nt_base;
+        a.nt_base = nt_base ? nt_base : c->d_ntbase + 1;   // the second word stays zero
         a.vy_in = c->d_vy[cur];
         a.sxy_in = c->d_sxy[cur];
         a.syz_in = c->d_syz[cur];
@@ -1001,8 +1025,18 @@ int dn_run_pass(dn_ctx *c, const std::vector<int> &shots, bool adjoint, bool sto
     int ntmax = 0;
     for (int s = 0; s < n; ++s) ntmax = std::max(ntmax, c->shot_nt[shots[s]]);
     if (c->nt_limit > 0) ntmax = std::min(ntmax, c->nt_limit);
+    if (!c->d_ntbase) {
+        HIPCHK(c, hipMalloc((void **)&c->d_ntbase, 256));
+        HIPCHK(c, launch_fill_u32((unsigned int *)c->d_ntbase, 64, 0u, c->stream));
+    }
     if (c->cur_map != shots) {
         HIPCHK(c, hipMemcpyAsync(c->d_shot_map, shots.data(), n * sizeof(int), hipMemcpyHostToDevice, c->stream));
+        c->h_slots.assign(n, ShotSlot{});
+        for (int s = 0; s < n; ++s) {
+            const int S = shots[s], l0 = c->src_off[S], l1 = c->src_off[S + 1];
+            c->h_slots[s] = ShotSlot{S, c->shot_nt[S], l0, l1, l1 > l0 ? c->src_i[l0] : 0, l1 > l0 ? c->src_j[l0] : 0, {0, 0}};
+        }
+        HIPCHK(c, hipMemcpyAsync(c->d_slots, c->h_slots.data(), n * sizeof(ShotSlot), hipMemcpyHostToDevice, c->stream));
         c->cur_map = shots;
     }
     if (dn_zero_state(c, n)) return -1;
@@ -1049,7 +1083,6 @@ int dn_run_pass(dn_ctx *c, const std::vector<int> &shots, bool adjoint, bool sto
     const int nchunks = (CH > 0 && ntmax >= 2 * CH) ? ntmax / CH : 0;
     hipGraphExec_t exec = nullptr;
     if (nchunks > 0) {
-        if (!c->d_ntbase) HIPCHK(c, hipMalloc((void **)&c->d_ntbase, 256));
         if (get_graph(c, a, n, adjoint, store, record, pack_mode, nsnap, CH, corr_res, fwd_extra, &exec)) return -1;
     }
     HIPCHK(c, launch_fill_u32((unsigned int *)c->d_status, 4, 0u, c->stream));
@@ -1420,10 +1453,12 @@ extern "C" int dn_forward_fields(dn_ctx *c, int shot, int nsteps, float *vy, flo
     if (!c || shot < 0 || shot >= c->nshots || nsteps < 1) return dn_fail(c, "dn_forward_fields: bad arguments");
     if (dn_ensure_batch(c, 1, false)) return -1;
     const int saved = c->shot_nt[shot];
+    c->cur_map.clear();   // the batch slots carry the record lengths
     c->shot_nt[shot] = std::min(nsteps, saved);
     HIPCHK(c, hipMemcpy(c->d_shot_nt + shot, &c->shot_nt[shot], sizeof(int), hipMemcpyHostToDevice));
     const int rc = dn_run_pass(c, std::vector<int>{shot}, false, false, false);
     c->shot_nt[shot] = saved;
+    c->cur_map.clear();
     HIPCHK(c, hipMemcpy(c->d_shot_nt + shot, &saved, sizeof(int), hipMemcpyHostToDevice));
     if (rc) return rc;
     const int cur = c->cur_final;

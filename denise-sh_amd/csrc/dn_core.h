@@ -68,6 +68,8 @@ struct dn_ctx {
     float *d_Ws = nullptr, *d_Wr = nullptr, *d_gu_shot = nullptr, *d_grho_shot = nullptr;
     double *d_part = nullptr;
     int *d_shot_map = nullptr;
+    dn::ShotSlot *d_slots = nullptr; // the batch slots' records of the tile step
+    std::vector<dn::ShotSlot> h_slots;
     std::vector<int> cur_map;        // absolute shot of each batch slot in the last pass
     std::vector<double> shot_l2, shot_energy;   // per-shot misfit sums of the last residual pass
     int cur_final = 0;

@@ -13,7 +13,7 @@ constexpr int kMaxL = 4;       // relaxation mechanisms supported
 // Zero frame around the interior of every padded field.  The fused step
 // reads up to 2K-1 rows above/below the interior, 2K-1 columns left of it
 // and 63 right of it (the last strip's wave), K <= 6.
-constexpr int kPadX = 16;      // columns left of i = 1 (64-byte aligned rows)
+constexpr int kPadX = 32;      // columns left of i = 1 (rows start on a 128-byte line)
 constexpr int kPadR = 64;      // columns right of i = nx (at least)
 constexpr int kPadY = 12;      // rows above j = 1 and below j = ny
 
@@ -63,12 +63,57 @@ struct PmlVec {
     const float *Kx, *ax, *bx, *Kxh, *axh, *bxh, *Ky, *ay, *by, *Kyh, *ayh, *byh;
 };
 
+// A batch slot of the tile step: what a workgroup needs of its shot in one
+// scalar load (the strips read shot_map, shot_nt and src_off one after the other)
+struct ShotSlot {
+    int shot, nt;                  // absolute shot, its time steps
+    int src0, src1;                // its sources src0..src1-1
+    int si, sj;                    // position of the first
+    int pad[2];
+};
+
 // Arguments of the fused time-step kernel (one launch advances every active
-// shot of a batch by one time step).
+// shot of a batch by one time step).  What a workgroup reads first stands
+// first: its scalar loads then share cache lines and wait once.
 struct StepArgs {
-    Geo g;
+    const ShotSlot *slots;         // [nshots] tile step
+    const int *nt_base;            // device step counter added to nt (graph replay; otherwise a zero)
+    int nt;                        // current step, 1-based (offset within a graph chunk)
     int nshots;                    // shots in this launch
     int nshots_all;                // shots of the context (bound of shot_map entries)
+    int tl_rw;                     // tile step: rows per wave; 0: the strip step
+    int tl_w, tl_h;                // columns and rows of a tile
+    int tl_ny;                     // tiles in a column of tiles
+    int tl_nblk, tl_nblk8;         // tiles of all shots, and per XCD slice
+    unsigned tl_mshots, tl_mny;    // (2^32 - 1) / nshots, (2^32 - 1) / tl_ny
+    Geo g;
+    // per-shot dynamic state; shot stride = plane (2*L*plane for rq)
+    const float *vy_in, *sxy_in, *syz_in;
+    // static model fields (shared by all shots), padded layout
+    const float *__restrict__ bfield;   // 1/rho (0 where rho < 1e-20)
+    // the stress coefficients packed per cell, read by the fused step
+    // with one wide load instead of one load per field: elastic one float2
+    // plane {uip, ujp}; viscoelastic one float4 plane {fipjp, f, dip[0],
+    // d[0]} followed by L-1 float2 planes {dip[l], d[l]}
+    const float *__restrict__ spk;
+    // the relaxation memory variables r[L], q[L] of a shot, interleaved per
+    // cell so that one wide access moves a cell's pairs: float4 planes
+    // {r[l], q[l], r[l+1], q[l+1]} for l = 0, 2, ..., then a float2 plane
+    // {r[L-1], q[L-1]} when L is odd
+    float *rq;
+    const int *rec_row;                     // [ny+1] -> offset into rec_tab, or -1
+    const int *rec_tab;                     // rows of [nx+1]: receiver index or -1 (shared by all shots)
+    PmlVec pml;
+    const float *psx_in;                    // psi_sxy_x [s][ny][2fw] (ping-pong)
+    const float *psy_in;                    // psi_syy_y [s][2fw][nx] (ping-pong)
+    float *psx_out, *psy_out;
+    float *pvx, *pvy;                       // psi_vyx [s][ny][2fw], psi_vyy [s][2fw][nx]
+    float *vy_out, *sxy_out, *syz_out;
+    float DT, DH, dhi, dthalbe;
+    float hc[7];
+    float hcy6;                    // coefficient used for the 6th y-term of update_v (Q6: hc[5])
+    float bip[kMaxL], bjm[kMaxL], cip[kMaxL], cjm[kMaxL];
+    // strip step
     int ow, nstrips, R, nsegs;     // strip width (owned columns), strips, rows per segment, segments
     int ngroups;                   // workgroups of kStripsPerGroup adjacent strips per segment row
     int nblocks, nblocks8;         // real workgroups and workgroups per XCD slice (one shot per wave)
@@ -77,44 +122,13 @@ struct StepArgs {
                                    // shot; 2, 4, 8 = kStripsPerGroup / sg adjacent strips of sg
                                    // consecutive shots (one shot per wave)
     int nblocks_sg, nblocks_sg8;   // workgroups in a layout with sg > 1
-    float DT, DH, dhi, dthalbe;
-    float hc[7];
-    float hcy6;                    // coefficient used for the 6th y-term of update_v (Q6: hc[5])
-    PmlVec pml;
-    // static model fields (shared by all shots), padded layout
-    const float *__restrict__ bfield;   // 1/rho (0 where rho < 1e-20)
-    const float *__restrict__ uip;      // elastic
-    const float *__restrict__ ujp;
-    const float *__restrict__ fipjp;    // visco
-    const float *__restrict__ fcoef;
-    const float *__restrict__ dip;      // [L][plane]
-    const float *__restrict__ dcoef;    // [L][plane]
-    // the same stress coefficients packed per cell, read by the fused step
-    // with one wide load instead of one load per field: elastic one float2
-    // plane {uip, ujp}; viscoelastic one float4 plane {fipjp, f, dip[0],
-    // d[0]} followed by L-1 float2 planes {dip[l], d[l]}
-    const float *__restrict__ spk;
-    float bip[kMaxL], bjm[kMaxL], cip[kMaxL], cjm[kMaxL];
-    // per-shot dynamic state; shot stride = plane (2*L*plane for rq)
-    const float *vy_in, *sxy_in, *syz_in;
-    float *vy_out, *sxy_out, *syz_out;
-    // the relaxation memory variables r[L], q[L] of a shot, interleaved per
-    // cell so that one wide access moves a cell's pairs: float4 planes
-    // {r[l], q[l], r[l+1], q[l+1]} for l = 0, 2, ..., then a float2 plane
-    // {r[L-1], q[L-1]} when L is odd
-    float *rq;
-    const float *psx_in;  float *psx_out;   // psi_sxy_x [s][ny][2fw] (ping-pong)
-    const float *psy_in;  float *psy_out;   // psi_syy_y [s][2fw][nx] (ping-pong)
-    float *pvx, *pvy;                       // psi_vyx [s][ny][2fw], psi_vyy [s][2fw][nx]
     // shot tables (absolute shot index of batch slot s: shot_map[s])
     const int *shot_map;
     const int *shot_nt;                     // [all shots] time steps of each shot
     const int *src_off, *src_i, *src_j;     // sources of shot s: src_off[s]..src_off[s+1]-1
     const float *src_sig;                   // [nsrc_total][nt_max]
     int nt_max;
-    // receivers (shared by all shots)
-    const int *rec_row;                     // [ny+1] -> offset into rec_tab, or -1
-    const int *rec_tab;                     // rows of [nx+1]: receiver index or -1
+    // receivers
     int ntr;
     float *seis;                            // forward: [s][ntr][nt_max]
     const float *resid;                     // adjoint: [s][ntr][nt_max] time-reversed residual
@@ -134,8 +148,6 @@ struct StepArgs {
     float *wacc;                            // Ws (forward) or Wr (adjoint) [s][ny][nx]
     float *grad_u, *grad_rho;               // adjoint [s][ny][nx]; forward with hess: H_mu, H_rho sums
     int hess;                               // forward: accumulate the pseudo-Hessian (hess_save.c, hessian.c)
-    int nt;                                 // current step, 1-based (offset within a graph chunk if nt_base)
-    const int *nt_base;                     // graph replay: device step counter added to nt, or null
     // latched by the kernel: [0] the first step after which vy at the probe
     // cell (NY/2, NX/2) is NaN (denise.c:1183-1185 checks that cell before
     // every step; 0: none), [1] that shot + 1, [2] nonzero: a shot-map
@@ -147,6 +159,10 @@ struct StepArgs {
 // extra: the step may store snapshots / sum the pseudo-Hessian (forward) or
 // correlate with the stored snapshots (adjoint) for some shot of the launch
 hipError_t launch_step(const StepArgs &a, int K, bool visco, bool adjoint, bool extra, hipStream_t st);
+
+// the same step on two-dimensional tiles (dn_tile.hip, one object per K);
+// a.tl_* must be set
+template <int K> hipError_t launch_tile_k(const StepArgs &a, int L, bool adjoint, bool extra, hipStream_t st);
 
 struct ModelPrepArgs {
     Geo g;

@@ -141,7 +141,7 @@ __global__ __launch_bounds__(kWave * kStripsPerGroup) void k_step(const StepArgs
         strip = live ? grp * kStripsPerGroup + wv : a.nstrips - 1;
     }
     const Geo &g = a.g;
-    const int nt = a.nt_base ? (*a.nt_base + a.nt) : a.nt;
+    const int nt = *a.nt_base + a.nt;
 
     // the wave's shots: batch slot, absolute shot, record length, active
     int sl[NSH], Sx[NSH], NTs[NSH];
@@ -775,10 +775,26 @@ static hipError_t launch_step_k(const StepArgs &a, int L, bool adjoint, bool ext
     }
 }
 
+template <> hipError_t launch_tile_k<1>(const StepArgs &a, int L, bool adjoint, bool extra, hipStream_t st);
+template <> hipError_t launch_tile_k<2>(const StepArgs &a, int L, bool adjoint, bool extra, hipStream_t st);
+template <> hipError_t launch_tile_k<3>(const StepArgs &a, int L, bool adjoint, bool extra, hipStream_t st);
+template <> hipError_t launch_tile_k<4>(const StepArgs &a, int L, bool adjoint, bool extra, hipStream_t st);
+template <> hipError_t launch_tile_k<5>(const StepArgs &a, int L, bool adjoint, bool extra, hipStream_t st);
+template <> hipError_t launch_tile_k<6>(const StepArgs &a, int L, bool adjoint, bool extra, hipStream_t st);
+
 hipError_t launch_step(const StepArgs &a, int K, bool visco, bool adjoint, bool extra, hipStream_t st)
 {
     const int L = visco ? a.g.L : 0;
     if (visco != (a.g.L > 0)) return hipErrorInvalidValue;
+    if (a.tl_rw > 0) switch (K) {
+        case 1: return launch_tile_k<1>(a, L, adjoint, extra, st);
+        case 2: return launch_tile_k<2>(a, L, adjoint, extra, st);
+        case 3: return launch_tile_k<3>(a, L, adjoint, extra, st);
+        case 4: return launch_tile_k<4>(a, L, adjoint, extra, st);
+        case 5: return launch_tile_k<5>(a, L, adjoint, extra, st);
+        case 6: return launch_tile_k<6>(a, L, adjoint, extra, st);
+        default: return hipErrorInvalidValue;
+        }
     switch (K) {
     case 1: return launch_step_k<1>(a, L, adjoint, extra, st);
     case 2: return launch_step_k<2>(a, L, adjoint, extra, st);

@@ -250,7 +250,10 @@ int dn_set_observed(dn_ctx *ctx, const float *obs);
 int dn_set_time_filt(dn_ctx *ctx, int time_filt, float fc_start, float fc, int order);
 
 /* Maximum number of shots advanced together (0 = automatic from free HBM)
- * and rows per workgroup segment of the time-step kernel (0 = automatic). */
+ * and rows per workgroup segment of the time-step kernel (0 = automatic: the
+ * step on two-dimensional tiles; a number of rows asks for the step on strips
+ * of columns, as two shots per wave or a workgroup layout do).  Results are
+ * identical. */
 int dn_set_batch(dn_ctx *ctx, int max_shots_per_batch, int rows_per_segment);
 /* by_record_length 1 (default): a gradient whose shots have uneven record
  * lengths and take several batches forms the batches by decreasing length
@@ -306,8 +309,8 @@ int dn_set_group_layout(dn_ctx *ctx, int mode);
 
 /* Tile-shape autotuner: on the batch the gradient runs (as many of the
  * first nshots shots as share a batch with their snapshots stored), times
- * nsteps forward steps for each candidate rows-per-segment (0: the cost
- * model's choice, then fixed heights), then one or two shots per wave, the
+ * nsteps forward steps for each candidate rows-per-segment (0: the automatic
+ * choice, then strips of fixed heights), then one or two shots per wave, the
  * workgroup layouts (at the cost model's, half, equal and double the rows)
  * and graph replay (kept unless eager launches are more than 2 % faster),
  * each the faster of two timed passes; keeps the fastest setting and
