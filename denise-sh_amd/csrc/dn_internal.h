@@ -183,7 +183,7 @@ hipError_t launch_hessian_finish(int nshots, int nx, int ny, const Geo &g, const
                                  const float *hr_shot, const float *vs_pad, const float *rho_pad, float *hu,
                                  float *hr, int first, int last, hipStream_t st);
 
-// per-shot residual (calc_res / calc_energy): one thread per trace
+// per-shot residual (calc_res / calc_energy)
 hipError_t launch_residual(int nshots, int nshots_all, int ntr, int nt_max, const int *shot_map, const int *shot_nt,
                            const float *syn, const float *obs, float *resid, double *part, float DT,
                            const unsigned char *flags, hipStream_t st);

@@ -930,47 +930,133 @@ hipError_t launch_model_prep(const ModelPrepArgs &a, hipStream_t st)
 
 // ---------------------------------------------------------------------------
 // Residual and misfit (calc_res.c:150-257 LNORM 2 / GRAD_FORM 2, Q7, and
-// calc_energy.c:53-61).  One thread per (shot, trace); per-trace FP64 partial
-// sums are written in place and reduced on the host in a fixed order.
+// calc_energy.c:53-61), with per-trace FP64 partial sums reduced on the host
+// in a fixed order.  flags [nshots_all][ntr] (or null): bit 0 leaves the
+// trace out of the residual and L2 (trace kill or offset mute,
+// calc_res.c:99-113), bit 1 out of the energy (trace kill as
+// calc_energy.c:23-49 reads the kill file).
+//
+// The sums of a trace (L2, the running float sum of the observed samples and
+// the energy) are serial chains over its samples; the bytes are 12 per
+// sample.  A workgroup takes 16 traces in chunks of 256 samples: all threads
+// load (one chunk ahead), form the residual and the squares with coalesced
+// accesses, and three waves run the three chains from LDS, 16 traces side by
+// side, the energy one chunk behind the running sum.  One thread per trace
+// with its own strided loads waited a memory latency per sample: 394 traces
+// of 12000 samples took 3195 us, now 287 us (96 traces of 1500: 442 -> 50 us).
 // ---------------------------------------------------------------------------
-// flags [nshots_all][ntr] (or null): bit 0 leaves the trace out of the
-// residual and L2 (trace kill or offset mute, calc_res.c:99-113), bit 1 out
-// of the energy (trace kill as calc_energy.c:23-49 reads the kill file)
-__global__ void k_residual(int nshots, int nshots_all, int ntr, int nt_max, const int *shot_map, const int *shot_nt,
-                           const float *syn, const float *obs, float *resid, double *part, float DT,
-                           const unsigned char *flags)
+constexpr int kResTraces = 16, kResChunk = 256;   // one sample per thread and trace
+
+__global__ __launch_bounds__(256) void k_residual(int nshots, int nshots_all, int ntr, int nt_max, const int *shot_map,
+                                                  const int *shot_nt, const float *syn, const float *obs,
+                                                  float *resid, double *part, float DT, const unsigned char *flags)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nshots * ntr) return;
-    const int s = t / ntr, r = t % ntr;
-    const int S = shot_map[s];
-    if (S < 0 || S >= nshots_all) {
-        part[2 * (long long)t] = 0.0;
-        part[2 * (long long)t + 1] = 0.0;
-        return;
+    constexpr int NE = kResTraces;                     // elements per thread: one sample of every trace
+    __shared__ float so[kResTraces][kResChunk + 1];    // observed samples, then their running sum
+    __shared__ double sd[kResTraces][kResChunk + 1];   // squared residuals
+    __shared__ double se[kResTraces][kResChunk + 1];   // squared running sums of the chunk before
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int t0 = blockIdx.x * kResTraces, ntot = nshots * ntr;
+    const int js = threadIdx.x;                        // the thread's sample of a chunk
+    int ns[NE];
+    bool res[NE], nrg[NE];
+    const float *sy[NE], *ob[NE];
+    float *df[NE];
+    int nmax = 0;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+        const int t = t0 + e;
+        ns[e] = 0;
+        res[e] = nrg[e] = false;
+        sy[e] = syn;
+        ob[e] = obs;
+        df[e] = nullptr;
+        if (t < ntot) {
+            const int s = t / ntr, r = t % ntr, S = shot_map[s];
+            if (S >= 0 && S < nshots_all) {
+                const unsigned fl = flags ? flags[(long long)S * ntr + r] : 0u;
+                ns[e] = shot_nt[S];
+                res[e] = !(fl & 1u);
+                nrg[e] = !(fl & 2u);
+                sy[e] = syn + (long long)t * nt_max;
+                ob[e] = obs + ((long long)S * ntr + r) * nt_max;
+                df[e] = resid + (long long)t * nt_max;
+            }
+        }
+        nmax = max(nmax, ns[e]);
     }
-    const int ns = shot_nt[S];
-    const float *sy = syn + (long long)t * nt_max;
-    const float *ob = obs + ((long long)S * ntr + r) * nt_max;
-    float *df = resid + (long long)t * nt_max;
-    const unsigned fl = flags ? flags[(long long)S * ntr + r] : 0u;
-    const bool res = !(fl & 1u), nrg = !(fl & 2u);
-    double l2 = 0.0, en = 0.0;
-    float intseis = 0.0f;
-    for (int j = 1; j <= ns; ++j) {
-        // calc_res.c:152 sets obs[1] = syn[1] for the traces it covers
-        const float o = (j == 1 && res) ? sy[0] : ob[j - 1];
-        const float d = res ? sy[j - 1] - o : 0.0f;
-        df[ns - j] = d;                                 // time reversal, calc_res.c:224
-        l2 += (double)d * (double)d;
-        if (nrg) {
-            intseis = intseis + o;                      // calc_energy.c:59-60
-            en += (double)(intseis * intseis * DT * DT);
+    float vs[NE], vo[NE];
+    auto load = [&](int c0) {
+        // past the end a valid sample is read again, unused: a load under a
+        // condition would be waited for at once
+#pragma unroll
+        for (int e = 0; e < NE; ++e) {
+            const int k = max(min(c0 + js, ns[e] - 1), 0);
+            vs[e] = sy[e][k];
+            vo[e] = ob[e][k];
+        }
+    };
+    double acc = 0.0;        // wave 0: l2, wave 2: energy of trace `lane`
+    float run = 0.0f;        // wave 1: running sum of the observed samples
+    load(0);
+    for (int c0 = 0; c0 < nmax + kResChunk; c0 += kResChunk) {
+        const int j = c0 + js;
+#pragma unroll
+        for (int e = 0; e < NE; ++e) {
+            const int r = e;
+            const bool in = j < ns[e];
+            // calc_res.c:152 sets obs[1] = syn[1] for the traces it covers
+            const float o = (j == 0 && res[e]) ? vs[e] : vo[e];
+            const float d = res[e] ? vs[e] - o : 0.0f;
+            if (in) df[e][ns[e] - 1 - j] = d;                  // time reversal, calc_res.c:224
+            so[r][js] = (in && nrg[e]) ? o : 0.0f;
+            sd[r][js] = in ? (double)d * (double)d : 0.0;
+        }
+        __syncthreads();
+        load(c0 + kResChunk);
+        if (lane < kResTraces) {
+            // sixteen samples are read before the chain uses them and before
+            // it writes
+            if (wave == 1) {
+                for (int k = 0; k < kResChunk; k += 16) {
+                    float v[16];
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) v[q] = so[lane][k + q];
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) {
+                        run = run + v[q];                      // calc_energy.c:59-60
+                        v[q] = run;
+                    }
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) so[lane][k + q] = v[q];
+                }
+            } else if (wave == 0 || (wave == 2 && c0 > 0)) {
+                const double *sv = wave == 0 ? sd[lane] : se[lane];
+                for (int k = 0; k < kResChunk; k += 16) {
+                    double v[16];
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) v[q] = sv[k + q];
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) acc += v[q];
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < NE; ++e) {
+            const int r = e;
+            const float p = so[r][js];
+            se[r][js] = (j < ns[e] && nrg[e]) ? (double)(p * p * DT * DT) : 0.0;
         }
     }
-    for (int j = ns; j < nt_max; ++j) df[j] = 0.0f;
-    part[2 * (long long)t] = l2;
-    part[2 * (long long)t + 1] = en;
+#pragma unroll
+    for (int e = 0; e < NE; ++e)
+        if (df[e])
+            for (int j = ns[e] + js; j < nt_max; j += kResChunk) df[e][j] = 0.0f;
+    if (lane < kResTraces && t0 + lane < ntot) {
+        if (wave == 0) part[2 * (long long)(t0 + lane)] = acc;
+        if (wave == 2) part[2 * (long long)(t0 + lane) + 1] = acc;
+    }
 }
 
 hipError_t launch_residual(int nshots, int nshots_all, int ntr, int nt_max, const int *shot_map, const int *shot_nt,
@@ -978,8 +1064,8 @@ hipError_t launch_residual(int nshots, int nshots_all, int ntr, int nt_max, cons
                            const unsigned char *flags, hipStream_t st)
 {
     const int n = nshots * ntr;
-    hipLaunchKernelGGL(k_residual, dim3((n + 63) / 64), dim3(64), 0, st, nshots, nshots_all, ntr, nt_max, shot_map,
-                       shot_nt, syn, obs, resid, part, DT, flags);
+    hipLaunchKernelGGL(k_residual, dim3((n + kResTraces - 1) / kResTraces), dim3(256), 0, st, nshots, nshots_all, ntr,
+                       nt_max, shot_map, shot_nt, syn, obs, resid, part, DT, flags);
     return hipGetLastError();
 }
 

@@ -1,0 +1,35 @@
+"""The chunked residual, smooth2 and Gaussian kernels at the edges of their
+chunks, row groups and pair tables, bit for bit against the oracle."""
+import sys
+
+import numpy as np
+import pytest
+
+from common import oracle, product
+from test_gpu_misfit import oracle_residual
+
+pytestmark = pytest.mark.gpu
+
+O32 = oracle("f32")
+
+
+def say(*a):
+    print(*a)
+    sys.stdout.flush()
+
+
+def bits(a):
+    return np.ascontiguousarray(a, np.float32).view(np.uint32)
+
+
+@pytest.mark.parametrize("ntr,ns", [(1, 127), (15, 128), (16, 129), (17, 256), (33, 257), (50, 64), (2, 1000)])
+def test_residual_chunks(ntr, ns):
+    say("residual", ntr, ns)
+    rng = np.random.default_rng(ntr + ns)
+    syn = rng.standard_normal((ntr, ns)).astype(np.float32)
+    obs = (syn + 0.3 * rng.standard_normal((ntr, ns))).astype(np.float32)
+    diff, l2, en, ob = product().calc_res(syn, obs, 1e-4)
+    rdiff, rl2, ren, rob = oracle_residual(syn, obs, float(np.float32(1e-4)))
+    assert np.array_equal(diff, rdiff) and np.array_equal(ob, rob)
+    # the sums of a trace run in sample order; only the order over traces differs
+    assert abs(l2 - rl2) <= 1e-12 * abs(rl2) and abs(en - ren) <= 1e-12 * abs(ren)
