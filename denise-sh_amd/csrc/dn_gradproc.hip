@@ -114,53 +114,215 @@ __global__ __launch_bounds__(256) void k_gauss_filt_var(int nx, int ny, const fl
     out[t] = conv / P.sum;
 }
 
-// x substitutions of smooth2: thread j (1..ny-1) solves the system of grid
-// row j over v[0..nx-1][j], v[0][j] = 0 (the zero column), in place on
-// g[j-1][0..nx-2]; e, d: the factored x matrix (tripd's e[k-1] and d[k])
-__global__ void k_smooth2_x(int nx, int ny, float *__restrict__ g, const float *__restrict__ e,
-                            const float *__restrict__ d, float v0)
+// Substitutions of smooth2.  Each system is a serial chain (a multiply and a
+// subtraction per unknown, forward then backward); the divisions of the
+// backward sweep are not part of it.  A thread that walks its system straight
+// from memory waits a load per unknown: 2000 x 400 took 931 us for x (rows,
+// uncoalesced) and 157 us for z.  Here the values come many unknowns ahead:
+// 86 and 38 us.
+//
+// 16 n unknowns of a chain in LDS: b[q] = b[q] - e[q] b[q-1], sixteen read
+// before the first is written
+template <int SB, int SE> __device__ __forceinline__ void chain16(int n, float *b, const float *e, float &prev)
 {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    if (j > ny - 1) return;
-    float *row = g + (size_t)(j - 1) * nx;   // v[ix][j] = row[ix - 1] for ix >= 1
-    float prev = v0;                         // b[0]
-    for (int k = 1; k < nx; ++k) {
-        const float b = row[k - 1] - e[k - 1] * prev;
-        row[k - 1] = b;
-        prev = b;
-    }
-    float bk = prev / d[nx - 1];             // b[n-1]
-    row[nx - 2] = bk;
-    for (int k = nx - 1; k >= 2; --k) {      // b[k-1] for k-1 >= 1; b[0] is not kept
-        const float b = row[k - 2] / d[k - 1] - e[k - 1] * bk;
-        row[k - 2] = b;
-        bk = b;
+    for (int k = 0; k < n; ++k) {
+        float v[16], w[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            v[q] = b[q * SB];
+            w[q] = e[q * SE];
+        }
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            prev = v[q] - w[q] * prev;
+            v[q] = prev;
+        }
+#pragma unroll
+        for (int q = 0; q < 16; ++q) b[q * SB] = v[q];
+        b += 16 * SB;
+        e += 16 * SE;
     }
 }
 
-// z substitutions of smooth2: thread i (1..nx-1) solves the system of grid
-// column i over v[i][1..ny-1] (n = ny - 1), its first right-hand side plus
-// r1 w v[i][0] (v[i][0] = v0 = 0, the zero row after its x smoothing)
-__global__ void k_smooth2_z(int nx, int ny, float *__restrict__ g, const float *__restrict__ e,
-                            const float *__restrict__ d, float r1w, float v0)
+// x: a workgroup takes kS2Rows grid rows in chunks of kS2Chunk columns
+// through LDS: all threads load (one chunk ahead), divide and store with
+// coalesced accesses, lane r of the first wave runs row r's chain.  Row j
+// (1..ny-1) is solved over v[0..nx-1][j], v[0][j] = 0 (the zero column), in
+// place on g[j-1][0..nx-2]; e, d: the factored x matrix (tripd's e[k-1], d[k]).
+constexpr int kS2Rows = 16, kS2Chunk = 512;
+
+__global__ __launch_bounds__(256) void k_smooth2_x(int nx, int ny, float *__restrict__ g, const float *__restrict__ e,
+                                                   const float *__restrict__ d, float v0)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    if (i > nx - 1) return;
-    float *col = g + (i - 1);                // v[i][iz + 1] = col[iz * nx]
-    const int n = ny - 1;
-    float prev = col[0] + (r1w * v0);
-    col[0] = prev;
-    for (int k = 1; k < n; ++k) {
-        const float b = col[(size_t)k * nx] - e[k - 1] * prev;
-        col[(size_t)k * nx] = b;
-        prev = b;
+    constexpr int NC = kS2Chunk / 256;       // columns per thread
+    __shared__ float buf[kS2Rows][kS2Chunk + 1];
+    __shared__ float se[kS2Chunk];
+    const int m = nx - 1;                    // unknowns of a row
+    const int row0 = blockIdx.x * kS2Rows, rows = min(kS2Rows, ny - 1 - row0);
+    const int lane = threadIdx.x;            // chain of row `lane`
+    float v[kS2Rows][NC], ev[NC], dv[NC];
+    // chunk [c0, c0 + kS2Chunk) of the unknowns; e and d at unknown + off.
+    // Past the ends the last row or column is read again, unused: a load under
+    // a condition would be waited for at once.
+    auto load = [&](int c0, int off) {
+#pragma unroll
+        for (int q = 0; q < NC; ++q) {
+            const int c = min(c0 + q * 256 + (int)threadIdx.x, m - 1);
+            ev[q] = e[c + off];
+            dv[q] = d[c + off];
+#pragma unroll
+            for (int r = 0; r < kS2Rows; ++r) v[r][q] = g[(size_t)(row0 + min(r, rows - 1)) * nx + c];
+        }
+    };
+    auto stage = [&](bool divide) {
+#pragma unroll
+        for (int q = 0; q < NC; ++q) {
+            const int col = q * 256 + (int)threadIdx.x;
+            se[col] = ev[q];
+#pragma unroll
+            for (int r = 0; r < kS2Rows; ++r) buf[r][col] = divide ? v[r][q] / dv[q] : v[r][q];
+        }
+    };
+    auto store = [&](int c0) {
+#pragma unroll
+        for (int q = 0; q < NC; ++q) {
+            const int col = q * 256 + (int)threadIdx.x, c = c0 + col;
+#pragma unroll
+            for (int r = 0; r < kS2Rows; ++r)
+                if (c < m && r < rows) g[(size_t)(row0 + r) * nx + c] = buf[r][col];
+        }
+    };
+    const int nch = (m + kS2Chunk - 1) / kS2Chunk;
+    float prev = v0;                         // b[0]
+    load(0, 0);
+    for (int n = 0; n < nch; ++n) {
+        const int c0 = n * kS2Chunk, len = min(kS2Chunk, m - c0);
+        stage(false);
+        __syncthreads();
+        if (n + 1 < nch) load(c0 + kS2Chunk, 0);
+        if (lane < rows) {
+            if (len >= 16) chain16<1, 1>(len / 16, &buf[lane][0], &se[0], prev);
+            for (int k = len / 16 * 16; k < len; ++k) {
+                prev = buf[lane][k] - se[k] * prev;
+                buf[lane][k] = prev;
+            }
+        }
+        __syncthreads();
+        store(c0);
     }
-    float bk = prev / d[n - 1];
-    col[(size_t)(n - 1) * nx] = bk;
-    for (int k = n - 1; k >= 1; --k) {
-        const float b = col[(size_t)(k - 1) * nx] / d[k - 1] - e[k - 1] * bk;
-        col[(size_t)(k - 1) * nx] = b;
-        bk = b;
+    // backward: b[m-1] = prev / d[nx-1], then b[k] = row[k] / d[k+1] - e[k+1] b[k+1]
+    // (each thread reads back only what it stored itself)
+    load((nch - 1) * kS2Chunk, 1);
+    for (int n = nch - 1; n >= 0; --n) {
+        const int c0 = n * kS2Chunk, len = min(kS2Chunk, m - c0);
+        __syncthreads();
+        stage(true);
+        __syncthreads();
+        if (n > 0) load(c0 - kS2Chunk, 1);
+        if (lane < rows) {
+            int k = len - 1;
+            if (n == nch - 1) prev = buf[lane][k--];
+            for (; (k + 1) % 16 != 0; --k) {
+                prev = buf[lane][k] - se[k] * prev;
+                buf[lane][k] = prev;
+            }
+            if (k >= 0) chain16<-1, -1>((k + 1) / 16, &buf[lane][k], &se[k], prev);
+        }
+        __syncthreads();
+        store(c0);
+    }
+}
+
+// z: column i (1..nx-1) is solved over v[i][1..ny-1] (n = ny - 1), its first
+// right-hand side plus r1 w v[i][0] (v[i][0] = v0 = 0, the zero row after its
+// x smoothing).  A workgroup takes 64 columns in chunks of kS2Rowz rows the
+// same way: four waves load, divide and store, the first runs the chains.
+constexpr int kS2Rowz = 128;
+
+__global__ __launch_bounds__(256) void k_smooth2_z(int nx, int ny, float *__restrict__ g, const float *__restrict__ e,
+                                                   const float *__restrict__ d, float r1w, float v0)
+{
+    constexpr int NR = kS2Rowz / 4;          // rows per thread: wave, wave + 4, ...
+    __shared__ float buf[kS2Rowz][64];
+    __shared__ float se[kS2Rowz];
+    const int n = ny - 1;                    // unknowns of a column
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int ci = blockIdx.x * 64 + lane;   // column i - 1
+    const bool in = ci < nx - 1;
+    const int cl = min(ci, nx - 2);
+    float v[NR], dv[NR], ev = 0.0f;
+    // rows [k0, k0 + kS2Rowz) (past the ends as above); e at row + off
+    auto load = [&](int k0, int off) {
+        ev = e[min(max(k0 + (int)threadIdx.x + off, 0), n - 1)];
+#pragma unroll
+        for (int q = 0; q < NR; ++q) {
+            const int r = min(k0 + wave + 4 * q, n - 1);
+            v[q] = g[(size_t)r * nx + cl];
+            dv[q] = d[r];
+        }
+    };
+    auto store = [&](int k0) {
+#pragma unroll
+        for (int q = 0; q < NR; ++q) {
+            const int r = k0 + wave + 4 * q;
+            if (in && r < n) g[(size_t)r * nx + ci] = buf[wave + 4 * q][lane];
+        }
+    };
+    const int nch = (n + kS2Rowz - 1) / kS2Rowz;
+    float prev = 0.0f;
+    load(0, -1);
+    for (int c = 0; c < nch; ++c) {
+        const int k0 = c * kS2Rowz, len = min(kS2Rowz, n - k0);
+#pragma unroll
+        for (int q = 0; q < NR; ++q) buf[wave + 4 * q][lane] = v[q];
+        if ((int)threadIdx.x < kS2Rowz) se[threadIdx.x] = ev;
+        __syncthreads();
+        if (c + 1 < nch) load(k0 + kS2Rowz, -1);
+        if (wave == 0) {
+            int k = 0;
+            if (c == 0) {
+                prev = buf[0][lane] + (r1w * v0);
+                buf[0][lane] = prev;
+                k = 1;
+            }
+            for (; k < len && k % 16 != 0; ++k) {
+                prev = buf[k][lane] - se[k] * prev;
+                buf[k][lane] = prev;
+            }
+            if (k + 16 <= len) {
+                const int n16 = (len - k) / 16;
+                chain16<64, 1>(n16, &buf[k][lane], &se[k], prev);
+                k += 16 * n16;
+            }
+            for (; k < len; ++k) {
+                prev = buf[k][lane] - se[k] * prev;
+                buf[k][lane] = prev;
+            }
+        }
+        __syncthreads();
+        store(k0);
+    }
+    // b[n-1] = prev / d[n-1], then b[k] = col[k] / d[k] - e[k] b[k+1]
+    load((nch - 1) * kS2Rowz, 0);
+    for (int c = nch - 1; c >= 0; --c) {
+        const int k0 = c * kS2Rowz, len = min(kS2Rowz, n - k0);
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < NR; ++q) buf[wave + 4 * q][lane] = v[q] / dv[q];
+        if ((int)threadIdx.x < kS2Rowz) se[threadIdx.x] = ev;
+        __syncthreads();
+        if (c > 0) load(k0 - kS2Rowz, 0);
+        if (wave == 0) {
+            int k = len - 1;
+            if (c == nch - 1) prev = buf[k--][lane];
+            for (; (k + 1) % 16 != 0; --k) {
+                prev = buf[k][lane] - se[k] * prev;
+                buf[k][lane] = prev;
+            }
+            if (k >= 0) chain16<-64, -1>((k + 1) / 16, &buf[k][lane], &se[k], prev);
+        }
+        __syncthreads();
+        store(k0);
     }
 }
 
@@ -581,9 +743,10 @@ hipError_t run_smooth2(int nx, int ny, const Smooth2Plan &P, std::vector<float> 
             return e;
     }
     const float *ex = *buf, *dx = ex + nx, *ez = dx + nx, *dz = ez + (ny - 1);
-    hipLaunchKernelGGL(k_smooth2_x, dim3((unsigned)((ny - 1 + 63) / 64)), dim3(64), 0, st, nx, ny, g, ex, dx, 0.0f);
+    hipLaunchKernelGGL(k_smooth2_x, dim3((unsigned)((ny - 1 + kS2Rows - 1) / kS2Rows)), dim3(256), 0, st, nx, ny, g, ex, dx,
+                       0.0f);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_smooth2_z, dim3((unsigned)((nx - 1 + 63) / 64)), dim3(64), 0, st, nx, ny, g, ez, dz, P.r1,
+    hipLaunchKernelGGL(k_smooth2_z, dim3((unsigned)((nx - 1 + 63) / 64)), dim3(256), 0, st, nx, ny, g, ez, dz, P.r1,
                        0.0f);
     return hipGetLastError();
 }

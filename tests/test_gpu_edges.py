@@ -33,3 +33,11 @@ def test_residual_chunks(ntr, ns):
     assert np.array_equal(diff, rdiff) and np.array_equal(ob, rob)
     # the sums of a trace run in sample order; only the order over traces differs
     assert abs(l2 - rl2) <= 1e-12 * abs(rl2) and abs(en - ren) <= 1e-12 * abs(ren)
+
+
+@pytest.mark.parametrize("nx,ny", [(2, 3), (129, 17), (130, 18), (128, 16), (257, 34), (145, 66), (100, 97), (64, 98)])
+def test_smooth2_chunks(nx, ny):
+    say("smooth2", nx, ny)
+    g = np.random.default_rng(nx * ny).standard_normal((ny, nx)).astype(np.float32)
+    for wd in (1.5, 11.0):
+        assert np.array_equal(bits(product().smooth2(g, wd)), bits(O32.smooth2(g, wd)))
