@@ -16,9 +16,9 @@
 //
 // Gaussian smoothing.  Each cell's half widths (hx, hz) follow its local
 // wavelength vs / FC_END; its kernel weights exp(-ii^2/sx - jj^2/sz) depend
-// only on (hx, hz).  The host turns the vs model into a per-cell index of
-// the distinct (hx, hz) pairs and builds one weight table per pair with the
-// same float operands, the double exp() rounded to float and the same
+// only on (hx, hz).  The device turns the vs model into a per-cell index of
+// the distinct (hx, hz) pairs; the host builds one weight table per pair with
+// the same float operands, the double exp() rounded to float and the same
 // sequential float sum as the reference, so the weights and their sums are
 // bit-identical to it.  The device then sums gradient x weight per cell in
 // the reference's order (x offset outer, y offset inner; unfused float
@@ -112,6 +112,83 @@ __global__ __launch_bounds__(256) void k_gauss_filt_var(int nx, int ny, const fl
         }
     }
     out[t] = conv / P.sum;
+}
+
+// gauss_filt_var.c:160-200 per cell on the device: the half widths of every
+// cell (the float operations of make_gauss_plan), the distinct pairs in a
+// small hash table (cell [ny][nx] gets the slot, -1 copies) and the largest
+// half width of every tile.  flags: nonzero if the host has to make the plan
+// (a size out of range, or more pairs than the table takes).
+constexpr int kPairSlots = 1024;            // distinct pairs taken: below half of it
+constexpr unsigned kNoPair = 0xffffffffu;
+
+__global__ __launch_bounds__(256) void k_gauss_plan(int nx, int ny, const float *__restrict__ vel, int pitch, float DH,
+                                                    float WD_DAMP, float WD_DAMP1, float FC_END, unsigned *keys,
+                                                    int *flags, int *__restrict__ cell, int *__restrict__ tile_half)
+{
+    __shared__ int hm[kTileY];
+    const int i = blockIdx.x * kTileX + threadIdx.x, j = blockIdx.y * kTileY + threadIdx.y;
+    int h = 0, slot = -1;
+    unsigned key = kNoPair;
+    if (i < nx && j < ny) {
+        const float lam = vel[(size_t)j * pitch + i] / FC_END;
+        const float rx = (WD_DAMP1 * lam) / DH, rz = (WD_DAMP * lam) / DH;
+        if (!(fabsf(rz) < 1e7f) || !(fabsf(rx) < 1e7f)) {
+            flags[0] = 1;
+        } else {
+            int fx = (int)roundf(rx), fz = (int)roundf(rz);
+            if (fz > 0) {
+                if (!(fx % 2)) fx += 1;
+                if (!(fz % 2)) fz += 1;
+                if (fx < 6) fx = 6;
+                if (fz < 6) fz = 6;
+                const int hx = abs(fx) / 2, hz = abs(fz) / 2;
+                h = max(hx, hz);
+                if (h > kMaxHalf)
+                    flags[0] = 1;
+                else
+                    key = ((unsigned)hx << 16) | (unsigned)hz;
+            }
+        }
+    }
+    // one lane of the wave looks a pair up for all lanes that have it: with a
+    // look-up per cell the table's cache line was the limit (248 us at
+    // 1200 x 300, now 12 us)
+    unsigned long long left = __ballot(key != kNoPair);
+    while (left) {
+        const int first = (int)__builtin_ctzll(left);
+        const unsigned ku = (unsigned)__builtin_amdgcn_readlane((int)key, first);
+        int found = 0;
+        if ((int)threadIdx.x == first) {   // threadIdx.x is the lane (kTileX is a wave)
+            unsigned q = (ku * 2654435761u) >> 22;   // 10 bits
+            int n = 0;
+            for (; n < kPairSlots; ++n, q = (q + 1) % kPairSlots) {
+                // a key never changes once set, so an old empty entry is
+                // settled by the exchange
+                unsigned k = keys[q];
+                if (k == kNoPair) k = atomicCAS(&keys[q], kNoPair, ku);
+                if (k == kNoPair || k == ku) break;
+            }
+            if (n == kPairSlots) flags[0] = 1;
+            found = (int)q;
+        }
+        found = __builtin_amdgcn_readlane(found, first);
+        if (key == ku) slot = found;
+        left &= ~__ballot(key == ku);
+    }
+    if (i < nx && j < ny) cell[(size_t)j * nx + i] = slot;
+    for (int o = 32; o > 0; o >>= 1) h = max(h, __shfl_xor(h, o, 64));
+    if (threadIdx.x == 0) hm[threadIdx.y] = h;
+    __syncthreads();
+    if (threadIdx.x == 0 && threadIdx.y == 0)
+        tile_half[blockIdx.y * gridDim.x + blockIdx.x] = max(max(hm[0], hm[1]), max(hm[2], hm[3]));
+}
+
+__global__ void k_gauss_plan_clear(unsigned *keys, int *flags)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < kPairSlots) keys[t] = kNoPair;
+    if (t == 0) flags[0] = 0;
 }
 
 // Substitutions of smooth2.  Each system is a serial chain (a multiply and a
@@ -343,7 +420,33 @@ struct GaussPlan {
     std::vector<float> w;        // weight tables, concatenated
     std::vector<int> tile_half;  // per 64x4 tile: largest half width
     int tiles_x = 0, tiles_y = 0;
+    int hmax = 0;                // largest half width
+    bool on_device = false;      // cell and tile_half are on the device already
 };
+
+// weight table of one pair (hx, hz) appended to P.w; exp() once per
+// (|ii|, |jj|), as the operands are squares
+void add_pair_weights(GaussPlan &P, int hx, int hz, GPair &out)
+{
+    const size_t woff = P.w.size();
+    const float sigx = (float)(hx / 2), sigz = (float)(hz / 2);
+    const float sx = (float)(2.0 * sigx * sigx), sz = (float)(2.0 * sigz * sigz);
+    std::vector<float> q((size_t)(hx + 1) * (hz + 1));
+    for (int ii = 0; ii <= hx; ++ii)
+        for (int jj = 0; jj <= hz; ++jj) {
+            const float a = (float)(ii * ii) / sx, b = (float)(jj * jj) / sz;
+            q[(size_t)ii * (hz + 1) + jj] = (float)::exp((double)(-a - b));
+        }
+    float sum = 0.0f;
+    for (int ii = -hx; ii <= hx; ++ii)
+        for (int jj = -hz; jj <= hz; ++jj) {
+            const float k = q[(size_t)std::abs(ii) * (hz + 1) + std::abs(jj)];
+            P.w.push_back(k);
+            sum += k;
+        }
+    out = GPair{hx, hz, (int)woff, sum};
+    P.hmax = std::max(P.hmax, std::max(hx, hz));
+}
 
 // gauss_filt_var.c:160-200 per cell; float operands as in the reference
 bool make_gauss_plan(int nx, int ny, float DH, float WD_DAMP, float WD_DAMP1, float FC_END, const float *vel,
@@ -381,17 +484,8 @@ bool make_gauss_plan(int nx, int ny, float DH, float WD_DAMP, float WD_DAMP1, fl
                 err = "smooth_grad: Gaussian weight tables above 2^28 entries";
                 return false;
             }
-            const float sigx = (float)(hx / 2), sigz = (float)(hz / 2);
-            const float sx = (float)(2.0 * sigx * sigx), sz = (float)(2.0 * sigz * sigz);
-            float sum = 0.0f;
-            for (int ii = -hx; ii <= hx; ++ii)
-                for (int jj = -hz; jj <= hz; ++jj) {
-                    const float a = (float)(ii * ii) / sx, b = (float)(jj * jj) / sz;
-                    const float k = (float)::exp((double)(-a - b));
-                    P.w.push_back(k);
-                    sum += k;
-                }
-            P.pairs.push_back(GPair{hx, hz, (int)woff, sum});
+            P.pairs.push_back(GPair{});
+            add_pair_weights(P, hx, hz, P.pairs.back());
             it = index.emplace(key, id).first;
         }
         P.cell[t] = it->second;
@@ -459,6 +553,7 @@ int make_gauss_fixed_plan(int nx, int ny, float DH, float WD_DAMP, float FC_END,
     P.tiles_x = (nx + kTileX - 1) / kTileX;
     P.tiles_y = (ny + kTileY - 1) / kTileY;
     P.tile_half.assign((size_t)P.tiles_x * P.tiles_y, hfs);
+    P.hmax = hfs;
     return 0;
 }
 
@@ -518,7 +613,8 @@ struct GaussDev {
     int *cell = nullptr, *tile_half = nullptr;
     GPair *pairs = nullptr;
     float *w = nullptr, *tmp = nullptr;
-    size_t cap_cell = 0, cap_tiles = 0, cap_pairs = 0, cap_w = 0, cap_tmp = 0;
+    unsigned *keys = nullptr;    // kPairSlots keys, then the flag word
+    size_t cap_cell = 0, cap_tiles = 0, cap_pairs = 0, cap_w = 0, cap_tmp = 0, cap_keys = 0;
     void release()
     {
         (void)hipFree(cell);
@@ -526,6 +622,7 @@ struct GaussDev {
         (void)hipFree(pairs);
         (void)hipFree(w);
         (void)hipFree(tmp);
+        (void)hipFree(keys);
         *this = GaussDev{};
     }
 };
@@ -546,13 +643,14 @@ hipError_t upload_plan(const GaussPlan &P, GaussDev &D, size_t n, hipStream_t st
 {
     hipError_t e;
     if ((e = grow(&D.cell, D.cap_cell, n)) != hipSuccess) return e;
-    if ((e = grow(&D.tile_half, D.cap_tiles, P.tile_half.size())) != hipSuccess) return e;
+    if ((e = grow(&D.tile_half, D.cap_tiles, (size_t)P.tiles_x * P.tiles_y)) != hipSuccess) return e;
     if ((e = grow(&D.pairs, D.cap_pairs, P.pairs.size())) != hipSuccess) return e;
     if ((e = grow(&D.w, D.cap_w, P.w.size())) != hipSuccess) return e;
     if ((e = grow(&D.tmp, D.cap_tmp, n)) != hipSuccess) return e;
-    if ((e = hipMemcpyAsync(D.cell, P.cell.data(), n * sizeof(int), hipMemcpyHostToDevice, st)) != hipSuccess)
+    if (P.on_device) {
+    } else if ((e = hipMemcpyAsync(D.cell, P.cell.data(), n * sizeof(int), hipMemcpyHostToDevice, st)) != hipSuccess)
         return e;
-    if ((e = hipMemcpyAsync(D.tile_half, P.tile_half.data(), P.tile_half.size() * sizeof(int),
+    else if ((e = hipMemcpyAsync(D.tile_half, P.tile_half.data(), P.tile_half.size() * sizeof(int),
                             hipMemcpyHostToDevice, st)) != hipSuccess)
         return e;
     if (!P.pairs.empty()) {
@@ -567,15 +665,50 @@ hipError_t upload_plan(const GaussPlan &P, GaussDev &D, size_t n, hipStream_t st
     return hipSuccess;
 }
 
+// The plan from a vs model on the device (rows of `pitch` floats): cell and
+// tile_half stay there.  Returns 1 where the host has to make the plan.
+hipError_t make_gauss_plan_device(int nx, int ny, float DH, float WD_DAMP, float WD_DAMP1, float FC_END,
+                                  const float *vel, int pitch, GaussDev &D, GaussPlan &P, bool &ok, hipStream_t st)
+{
+    ok = false;
+    P.tiles_x = (nx + kTileX - 1) / kTileX;
+    P.tiles_y = (ny + kTileY - 1) / kTileY;
+    hipError_t e;
+    if ((e = grow(&D.cell, D.cap_cell, (size_t)nx * ny)) != hipSuccess) return e;
+    if ((e = grow(&D.tile_half, D.cap_tiles, (size_t)P.tiles_x * P.tiles_y)) != hipSuccess) return e;
+    if ((e = grow(&D.keys, D.cap_keys, kPairSlots + 1)) != hipSuccess) return e;
+    int *flags = (int *)(D.keys + kPairSlots);
+    hipLaunchKernelGGL(k_gauss_plan_clear, dim3(kPairSlots / 256), dim3(256), 0, st, D.keys, flags);
+    hipLaunchKernelGGL(k_gauss_plan, dim3(P.tiles_x, P.tiles_y), dim3(kTileX, kTileY), 0, st, nx, ny, vel, pitch, DH,
+                       WD_DAMP, WD_DAMP1, FC_END, D.keys, flags, D.cell, D.tile_half);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    std::vector<unsigned> h(kPairSlots + 1);
+    if ((e = hipMemcpyAsync(h.data(), D.keys, h.size() * sizeof(unsigned), hipMemcpyDeviceToHost, st)) != hipSuccess)
+        return e;
+    if ((e = hipStreamSynchronize(st)) != hipSuccess) return e;
+    size_t used = 0, total = 0;
+    for (int q = 0; q < kPairSlots; ++q)
+        if (h[q] != kNoPair) {
+            ++used;
+            total += (size_t)(2 * (h[q] >> 16) + 1) * (2 * (h[q] & 0xffffu) + 1);
+        }
+    if (h[kPairSlots] != 0 || used >= kPairSlots / 2 || total > (size_t)1 << 28) return hipSuccess;
+    P.pairs.assign(kPairSlots, GPair{0, 0, 0, 1.0f});
+    for (int q = 0; q < kPairSlots; ++q)
+        if (h[q] != kNoPair) add_pair_weights(P, (int)(h[q] >> 16), (int)(h[q] & 0xffffu), P.pairs[q]);
+    if (P.w.empty()) P.pairs.clear();
+    P.on_device = true;
+    ok = true;
+    return hipSuccess;
+}
+
 // filters the device plane g [ny][nx] in place (through D.tmp)
 hipError_t run_gauss(int nx, int ny, const GaussPlan &P, GaussDev &D, float *g, hipStream_t st)
 {
     const size_t n = (size_t)nx * ny;
     hipError_t e = hipMemcpyAsync(D.tmp, g, n * sizeof(float), hipMemcpyDeviceToDevice, st);
     if (e != hipSuccess) return e;
-    int hmax = 0;
-    for (int h : P.tile_half) hmax = std::max(hmax, h);
-    const size_t want = (size_t)(kTileX + 2 * hmax) * (kTileY + 2 * hmax);
+    const size_t want = (size_t)(kTileX + 2 * P.hmax) * (kTileY + 2 * P.hmax);
     const size_t lds = std::min<size_t>(want, kLdsFloats) * sizeof(float);
     hipLaunchKernelGGL(k_gauss_filt_var, dim3(P.tiles_x, P.tiles_y), dim3(kTileX, kTileY), lds, st, nx, ny,
                        D.tmp, g, D.cell, D.pairs, D.w, D.tile_half);
@@ -839,10 +972,15 @@ int dn_smooth_grad_device(dn_ctx *c, int spatfilter, float wd_damp, float wd_dam
         if (rc < 0) return dn_fail(c, "%s", err.c_str());
         if (rc > 0) return 0;
     } else {
-        std::vector<float> vel;
-        if (vs_host(c, vel)) return -1;
-        if (!make_gauss_plan(g.nx, g.ny, c->p.dh, wd_damp, wd_damp1, fc_end, vel.data(), P, err))
-            return dn_fail(c, "%s", err.c_str());
+        bool ok = false;
+        HIPCHK(c, make_gauss_plan_device(g.nx, g.ny, c->p.dh, wd_damp, wd_damp1, fc_end, c->d_vs + gidx(g, 1, 1),
+                                         g.pitch, gp(c)->gd, P, ok, c->stream));
+        if (!ok) {
+            std::vector<float> vel;
+            if (vs_host(c, vel)) return -1;
+            if (!make_gauss_plan(g.nx, g.ny, c->p.dh, wd_damp, wd_damp1, fc_end, vel.data(), P, err))
+                return dn_fail(c, "%s", err.c_str());
+        }
     }
     dn_gradproc_state *s = gp(c);
     const size_t n = (size_t)g.nx * g.ny;
@@ -919,10 +1057,14 @@ extern "C" int dn_gauss_filt_var(int nx, int ny, float dh, float wd_damp, float 
     if (sa_init(S)) return -1;
     GaussPlan P;
     std::string err;
-    if (!make_gauss_plan(nx, ny, dh, wd_damp, wd_damp1, fc_end, vel, P, err))
-        return dn_fail(nullptr, "%s", err.c_str());
     const size_t n = (size_t)nx * ny;
     SACHK(grow(&S.g, S.cap_g, n));
+    // the model passes through the gradient's buffer
+    bool ok = false;
+    SACHK(hipMemcpyAsync(S.g, vel, n * sizeof(float), hipMemcpyHostToDevice, S.st));
+    SACHK(make_gauss_plan_device(nx, ny, dh, wd_damp, wd_damp1, fc_end, S.g, nx, S.gd, P, ok, S.st));
+    if (!ok && !make_gauss_plan(nx, ny, dh, wd_damp, wd_damp1, fc_end, vel, P, err))
+        return dn_fail(nullptr, "%s", err.c_str());
     SACHK(upload_plan(P, S.gd, n, S.st));
     SACHK(hipMemcpyAsync(S.g, grad, n * sizeof(float), hipMemcpyHostToDevice, S.st));
     SACHK(run_gauss(nx, ny, P, S.gd, S.g, S.st));

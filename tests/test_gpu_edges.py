@@ -41,3 +41,28 @@ def test_smooth2_chunks(nx, ny):
     g = np.random.default_rng(nx * ny).standard_normal((ny, nx)).astype(np.float32)
     for wd in (1.5, 11.0):
         assert np.array_equal(bits(product().smooth2(g, wd)), bits(O32.smooth2(g, wd)))
+
+
+@pytest.mark.parametrize("name,ny,nx,wd,wd1,fc,lo,hi", [
+    ("a jump at every cell", 20, 130, 0.3, 0.25, 20.0, 60.0, 500.0),
+    ("more pairs than the table takes", 70, 130, 1.1, 0.9, 5.0, 20.0, 600.0),
+    ("one pair", 9, 65, 0.3, 0.3, 25.0, 200.0, 200.0),
+])
+def test_gauss_pairs(name, ny, nx, wd, wd1, fc, lo, hi):
+    say("gauss_filt_var", name)
+    rng = np.random.default_rng(4)
+    vel = rng.uniform(lo, hi, (ny, nx)).astype(np.float32)
+    g = rng.standard_normal((ny, nx)).astype(np.float32)
+    got = product().gauss_filt_var(g, vel, 0.25, wd, wd1, fc)
+    assert np.array_equal(bits(got), bits(O32.gauss_filt_var(g, vel, 0.25, wd, wd1, fc)))
+
+
+def test_gauss_out_of_range_is_refused():
+    dn = product()
+    vel = np.full((20, 70), 200.0, np.float32)
+    vel[7, 33] = np.nan
+    with pytest.raises(dn.DeniseError):
+        dn.gauss_filt_var(np.ones((20, 70), np.float32), vel, 0.25, 0.3, 0.3, 25.0)
+    vel[7, 33] = 1e6
+    with pytest.raises(dn.DeniseError):
+        dn.gauss_filt_var(np.ones((20, 70), np.float32), vel, 0.25, 0.3, 0.3, 25.0)
