@@ -35,6 +35,7 @@ const LSpec kLayers[] = {
     {80, 32, 80, 1}, {32, 32, 32, 1}, {48, 16, 48, 1}, {16, 16, 16, 1}, {16, 16, 16, 0},
 };
 constexpr int kNL = sizeof(kLayers) / sizeof(kLayers[0]);
+constexpr int kLossParts = 256;   // workgroups of the loss kernel
 
 template <typename T> hipError_t dal(T **p, size_t n) { return hipMalloc((void **)p, std::max<size_t>(n, 1) * sizeof(T)); }
 template <typename T> void dfr(T *&p)
@@ -55,7 +56,6 @@ struct dn_unet {
     // activation buffers for one (n, H, W)
     int bn = 0, bH = 0, bW = 0;
     uint16_t *x = nullptr, *a[kNL] = {nullptr}, *p1 = nullptr, *p2 = nullptr, *p3 = nullptr;
-    uint16_t *c8 = nullptr, *c10 = nullptr, *c12 = nullptr;
     uint16_t *d[kNL + 1] = {nullptr}, *dc8 = nullptr, *dc10 = nullptr, *dc12 = nullptr, *dp1 = nullptr,
              *dp2 = nullptr, *dp3 = nullptr;
     float *out32 = nullptr, *xin = nullptr, *tgt = nullptr, *yout = nullptr, *part = nullptr, *bpart = nullptr;
@@ -74,7 +74,7 @@ static void free_buffers(dn_unet *u)
     dfr(u->x);
     for (int l = 0; l < kNL; ++l) dfr(u->a[l]);
     for (int l = 0; l <= kNL; ++l) dfr(u->d[l]);
-    dfr(u->p1); dfr(u->p2); dfr(u->p3); dfr(u->c8); dfr(u->c10); dfr(u->c12);
+    dfr(u->p1); dfr(u->p2); dfr(u->p3);
     dfr(u->dc8); dfr(u->dc10); dfr(u->dc12); dfr(u->dp1); dfr(u->dp2); dfr(u->dp3);
     dfr(u->out32); dfr(u->xin); dfr(u->tgt); dfr(u->yout); dfr(u->part); dfr(u->bpart); dfr(u->lpart);
     u->bn = u->bH = u->bW = 0;
@@ -104,16 +104,13 @@ static int ensure_buffers(dn_unet *u, int n, int H, int W)
     UCHK(dal(&u->p1, P1 * 16));
     UCHK(dal(&u->p2, P2 * 32));
     UCHK(dal(&u->p3, P3 * 48));
-    UCHK(dal(&u->c8, P2 * 112));
-    UCHK(dal(&u->c10, P1 * 80));
-    UCHK(dal(&u->c12, P0 * 48));
     UCHK(dal(&u->dc8, P2 * 112));
     UCHK(dal(&u->dc10, P1 * 80));
     UCHK(dal(&u->dc12, P0 * 48));
     UCHK(dal(&u->dp1, P1 * 16));
     UCHK(dal(&u->dp2, P2 * 32));
     UCHK(dal(&u->dp3, P3 * 48));
-    UCHK(dal(&u->out32, P0 * 16));
+    UCHK(dal(&u->out32, P0));
     UCHK(dal(&u->xin, P0 * 3));
     UCHK(dal(&u->tgt, P0));
     UCHK(dal(&u->yout, P0));
@@ -125,7 +122,7 @@ static int ensure_buffers(dn_unet *u, int n, int H, int W)
     }
     UCHK(dal(&u->part, plen));
     UCHK(dal(&u->bpart, blen));
-    UCHK(dal(&u->lpart, 256));
+    UCHK(dal(&u->lpart, kLossParts));
     u->part_len = plen;
     u->bn = n;
     u->bH = H;
@@ -141,7 +138,9 @@ static int cast_all(dn_unet *u)
     return 0;
 }
 
-static int conv(dn_unet *u, int l, int n, int H, int W, const uint16_t *x, uint16_t *y16, float *y32)
+// layer l; with up, its input is [up-sampled up | x]
+static int conv(dn_unet *u, int l, int n, int H, int W, const uint16_t *x, uint16_t *y16, float *y1 = nullptr,
+                const uint16_t *up = nullptr)
 {
     ConvArgs c{};
     c.n = n;
@@ -154,7 +153,8 @@ static int conv(dn_unet *u, int l, int n, int H, int W, const uint16_t *x, uint1
     c.bias = u->w32 + u->boff[l];
     c.relu = kLayers[l].relu;
     c.y16 = y16;
-    c.y32 = y32;
+    c.y1 = y1;
+    c.up = up;
     UCHK(launch_conv3x3(c, u->stream));
     return 0;
 }
@@ -177,7 +177,8 @@ static int conv_bwd(dn_unet *u, int l, int n, int H, int W, const uint16_t *dy, 
     return 0;
 }
 
-static int wgrad(dn_unet *u, int l, int n, int H, int W, const uint16_t *x, const uint16_t *dy)
+static int wgrad(dn_unet *u, int l, int n, int H, int W, const uint16_t *x, const uint16_t *dy,
+                 const uint16_t *up = nullptr)
 {
     WgradArgs w{};
     w.n = n;
@@ -186,6 +187,7 @@ static int wgrad(dn_unet *u, int l, int n, int H, int W, const uint16_t *x, cons
     w.Ci = kLayers[l].ci;
     w.Co = kLayers[l].co;
     w.x = x;
+    w.up = up;
     w.dy = dy;
     w.chunk_rows = wgrad_chunk_rows(n, H);
     w.part = u->part;
@@ -194,27 +196,22 @@ static int wgrad(dn_unet *u, int l, int n, int H, int W, const uint16_t *x, cons
     return 0;
 }
 
-// forward of the packed input u->x; result in u->out32 (channel 0)
-static int forward_dev(dn_unet *u, int n, int H, int W)
+// forward of the packed input u->x; result in y [n][H][W]
+static int forward_dev(dn_unet *u, int n, int H, int W, float *y)
 {
     const int H1 = H / 2, W1 = W / 2, H2 = H / 4, W2 = W / 4, H3 = H / 8, W3 = W / 8;
-    if (conv(u, 0, n, H, W, u->x, u->a[0], nullptr) || conv(u, 1, n, H, W, u->a[0], u->a[1], nullptr)) return -1;
-    UCHK(launch_pool(n, H, W, 16, u->a[1], u->p1, u->stream));
-    if (conv(u, 2, n, H1, W1, u->p1, u->a[2], nullptr) || conv(u, 3, n, H1, W1, u->a[2], u->a[3], nullptr)) return -1;
-    UCHK(launch_pool(n, H1, W1, 32, u->a[3], u->p2, u->stream));
-    if (conv(u, 4, n, H2, W2, u->p2, u->a[4], nullptr) || conv(u, 5, n, H2, W2, u->a[4], u->a[5], nullptr)) return -1;
-    UCHK(launch_pool(n, H2, W2, 48, u->a[5], u->p3, u->stream));
-    if (conv(u, 6, n, H3, W3, u->p3, u->a[6], nullptr) || conv(u, 7, n, H3, W3, u->a[6], u->a[7], nullptr)) return -1;
-    UCHK(launch_upcat(n, H2, W2, 64, 48, u->a[7], u->a[5], u->c8, u->stream));
-    if (conv(u, 8, n, H2, W2, u->c8, u->a[8], nullptr) || conv(u, 9, n, H2, W2, u->a[8], u->a[9], nullptr)) return -1;
-    UCHK(launch_upcat(n, H1, W1, 48, 32, u->a[9], u->a[3], u->c10, u->stream));
-    if (conv(u, 10, n, H1, W1, u->c10, u->a[10], nullptr) || conv(u, 11, n, H1, W1, u->a[10], u->a[11], nullptr))
-        return -1;
-    UCHK(launch_upcat(n, H, W, 32, 16, u->a[11], u->a[1], u->c12, u->stream));
-    if (conv(u, 12, n, H, W, u->c12, u->a[12], nullptr) || conv(u, 13, n, H, W, u->a[12], u->a[13], nullptr))
-        return -1;
-    if (conv(u, 14, n, H, W, u->a[13], nullptr, u->out32)) return -1;
-    return 0;
+    uint16_t **a = u->a;
+    if (conv(u, 0, n, H, W, u->x, a[0]) || conv(u, 1, n, H, W, a[0], a[1])) return -1;
+    UCHK(launch_pool(n, H, W, 16, a[1], u->p1, u->stream));
+    if (conv(u, 2, n, H1, W1, u->p1, a[2]) || conv(u, 3, n, H1, W1, a[2], a[3])) return -1;
+    UCHK(launch_pool(n, H1, W1, 32, a[3], u->p2, u->stream));
+    if (conv(u, 4, n, H2, W2, u->p2, a[4]) || conv(u, 5, n, H2, W2, a[4], a[5])) return -1;
+    UCHK(launch_pool(n, H2, W2, 48, a[5], u->p3, u->stream));
+    if (conv(u, 6, n, H3, W3, u->p3, a[6]) || conv(u, 7, n, H3, W3, a[6], a[7])) return -1;
+    if (conv(u, 8, n, H2, W2, a[5], a[8], nullptr, a[7]) || conv(u, 9, n, H2, W2, a[8], a[9])) return -1;
+    if (conv(u, 10, n, H1, W1, a[3], a[10], nullptr, a[9]) || conv(u, 11, n, H1, W1, a[10], a[11])) return -1;
+    if (conv(u, 12, n, H, W, a[1], a[12], nullptr, a[11]) || conv(u, 13, n, H, W, a[12], a[13])) return -1;
+    return conv(u, 14, n, H, W, a[13], nullptr, y);
 }
 
 // backward from d[kNL] (gradient of the head output) into u->g
@@ -225,15 +222,15 @@ static int backward_dev(dn_unet *u, int n, int H, int W)
     // head and dec1
     if (wgrad(u, 14, n, H, W, u->a[13], d[14]) || conv_bwd(u, 14, n, H, W, d[14], u->a[13], d[13])) return -1;
     if (wgrad(u, 13, n, H, W, u->a[12], d[13]) || conv_bwd(u, 13, n, H, W, d[13], u->a[12], d[12])) return -1;
-    if (wgrad(u, 12, n, H, W, u->c12, d[12]) || conv_bwd(u, 12, n, H, W, d[12], nullptr, u->dc12)) return -1;
+    if (wgrad(u, 12, n, H, W, u->a[1], d[12], u->a[11]) || conv_bwd(u, 12, n, H, W, d[12], nullptr, u->dc12)) return -1;
     UCHK(launch_up_bwd(n, H, W, 32, 48, u->dc12, u->a[11], d[11], u->stream));
     // dec2
     if (wgrad(u, 11, n, H1, W1, u->a[10], d[11]) || conv_bwd(u, 11, n, H1, W1, d[11], u->a[10], d[10])) return -1;
-    if (wgrad(u, 10, n, H1, W1, u->c10, d[10]) || conv_bwd(u, 10, n, H1, W1, d[10], nullptr, u->dc10)) return -1;
+    if (wgrad(u, 10, n, H1, W1, u->a[3], d[10], u->a[9]) || conv_bwd(u, 10, n, H1, W1, d[10], nullptr, u->dc10)) return -1;
     UCHK(launch_up_bwd(n, H1, W1, 48, 80, u->dc10, u->a[9], d[9], u->stream));
     // dec3
     if (wgrad(u, 9, n, H2, W2, u->a[8], d[9]) || conv_bwd(u, 9, n, H2, W2, d[9], u->a[8], d[8])) return -1;
-    if (wgrad(u, 8, n, H2, W2, u->c8, d[8]) || conv_bwd(u, 8, n, H2, W2, d[8], nullptr, u->dc8)) return -1;
+    if (wgrad(u, 8, n, H2, W2, u->a[5], d[8], u->a[7]) || conv_bwd(u, 8, n, H2, W2, d[8], nullptr, u->dc8)) return -1;
     UCHK(launch_up_bwd(n, H2, W2, 64, 112, u->dc8, u->a[7], d[7], u->stream));
     // mid
     if (wgrad(u, 7, n, H3, W3, u->a[6], d[7]) || conv_bwd(u, 7, n, H3, W3, d[7], u->a[6], d[6])) return -1;
@@ -260,12 +257,11 @@ static int check_shape(int n, int H, int W)
     return 0;
 }
 
-static int loss_dev(dn_unet *u, long long P, bool grad, double *loss)
+// sum of the loss partials (synchronises the stream)
+static int read_loss(dn_unet *u, long long P, double *loss)
 {
-    const int nb = 256;
-    UCHK(launch_mse(P, u->out32, u->tgt, grad ? u->d[14] : nullptr, u->lpart, nb, u->stream));
-    std::vector<double> h(nb);
-    UCHK(hipMemcpyAsync(h.data(), u->lpart, nb * sizeof(double), hipMemcpyDeviceToHost, u->stream));
+    double h[kLossParts];
+    UCHK(hipMemcpyAsync(h, u->lpart, sizeof(h), hipMemcpyDeviceToHost, u->stream));
     UCHK(hipStreamSynchronize(u->stream));
     double s = 0.0;
     for (double v : h) s += v;
@@ -353,8 +349,7 @@ int dn_unet_forward_device(dn_unet *u, int n, int H, int W, const float *x_dev, 
 {
     if (check_shape(n, H, W) || ensure_buffers(u, n, H, W)) return -1;
     UCHK(launch_pack_input(n, H, W, x_dev, u->x, u->stream));
-    if (forward_dev(u, n, H, W)) return -1;
-    UCHK(launch_extract((long long)n * H * W, u->out32, y_dev, u->stream));
+    if (forward_dev(u, n, H, W, y_dev)) return -1;
     UCHK(hipStreamSynchronize(u->stream));
     return 0;
 }
@@ -377,10 +372,11 @@ static int loss_grad_common(dn_unet *u, int n, int H, int W, const float *x, con
     UCHK(hipMemcpyAsync(u->xin, x, P * 3 * sizeof(float), hipMemcpyHostToDevice, u->stream));
     UCHK(hipMemcpyAsync(u->tgt, t, P * sizeof(float), hipMemcpyHostToDevice, u->stream));
     UCHK(launch_pack_input(n, H, W, u->xin, u->x, u->stream));
-    if (forward_dev(u, n, H, W)) return -1;
-    if (loss_dev(u, (long long)P, true, loss)) return -1;
+    if (forward_dev(u, n, H, W, u->out32)) return -1;
+    UCHK(launch_mse((long long)P, u->out32, u->tgt, u->d[14], u->lpart, kLossParts, u->stream));
+    // the loss is read behind the backward pass, which does not need it
     if (backward_dev(u, n, H, W)) return -1;
-    return 0;
+    return read_loss(u, (long long)P, loss);
 }
 
 extern "C" int dn_unet_loss_grad(dn_unet *u, int n, int H, int W, const float *x, const float *t, double *loss,

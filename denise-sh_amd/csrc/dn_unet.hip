@@ -37,112 +37,247 @@ __device__ __forceinline__ f4v mfma32(u8v a, u8v b, f4v c)
 // tap; one MFMA takes 4 groups: lane quarter kq = lane / 16 supplies group
 // 4i + kq, A = W[tap][co = lane % 16][8 channels] and B = X[pixel lane % 16
 // + shift][8 channels] (16 bytes each), and receives D[4kq + r][lane % 16],
-// r = 0..3.  Groups past the last tap are zero.
-// Workgroup: 4 waves over 256 consecutive pixels of one image row (64 per
-// wave, 4 pixel tiles) and a group of up to 64 output channels (blockIdx.z,
-// up to 4 channel tiles): 16 accumulator tiles per wave.  The weights of one
-// kernel row (3 taps x 64 channels x CI) are staged in LDS once and read by
-// all four waves; the input comes with one 16-byte load per lane and
-// operand, the three taps of a row re-reading a pixel through L1.
+// r = 0..3.  The weights of groups past the last tap are zero.
+//
+// The layers move 2 (CI + Co) bytes per pixel for 18 CI Co operations: at 16
+// channels 72 operations per byte, so the bytes bound them, if enough loads
+// are in flight.  A wave owns 16 NT columns and up to 16 NM output channels
+// and walks down a strip of rows: each input row is loaded once, while the
+// row before it is multiplied, and enters the accumulators of the three
+// output rows it belongs to, in the order ky = 0, 1, 2 of the sum.  All nine
+// taps' weights are staged in LDS once, so the walk has no barrier.  One row
+// per workgroup, each row's weights staged and waited for and each input row
+// loaded for three output rows, took 118 us for 16 -> 16 channels at 800 x
+// 4000 and 168 us for 80 -> 32 at half of it; now 47 us (4.4 TB/s) and 79.
+//
+// CAT: the input is the concatenation of an up-sampled tensor (CU channels at
+// half resolution, nearest) and a skip tensor, read from both where they are:
+// the concatenated copy (243 us per layer at 800 x 4000) is never written.
 // ---------------------------------------------------------------------------
-template <int CI>
-__global__ __launch_bounds__(256) void k_conv3x3(ConvArgs a)
+constexpr int cat_up(int CI) { return CI == 112 ? 64 : (CI == 80 ? 48 : 32); }
+
+// One row of a tensor as a buffer resource: an offset outside [0, bytes)
+// reads zero and stores nothing, which is the convolution's padding, without
+// a branch (behind a branch the compiler waits for every access in flight).
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+__device__ __forceinline__ rsrc_t row_rsrc(const void *p, int bytes)
 {
-    constexpr int CB = CI / 8;          // 8-channel groups per tap
-    constexpr int NG = 3 * CB;          // groups of one kernel row
-    constexpr int NKI = (NG + 3) / 4;   // MFMAs per kernel row
-    constexpr int SW = 65;              // LDS entries per group (64 channels + 1 against bank conflicts)
-    __shared__ u8v sw[NKI * 4 * SW];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, bytes, 0x00027000);
+}
+typedef unsigned int u4v __attribute__((ext_vector_type(4)));
+typedef unsigned int u2v __attribute__((ext_vector_type(2)));
+
+template <int CI, int NM, int NT, bool CAT>
+__global__ __launch_bounds__(256, 2) void k_conv3x3(ConvArgs a)
+{
+    // the input's parts: the up-sampled and the skip tensor, or one tensor
+    constexpr int C0 = CAT ? cat_up(CI) : CI, C1 = CI - C0;
+    constexpr int B0 = C0 / 8, B1 = C1 / 8;                          // 8-channel groups per tap
+    constexpr int N0 = (3 * B0 + 3) / 4, N1 = (3 * B1 + 3) / 4;      // MFMAs per kernel row
+    constexpr int NKI = N0 + N1;
+    constexpr int SW = 16 * NM + 1;     // LDS entries per group (+ 1 against bank conflicts)
+    __shared__ u8v sw[3 * NKI * 4 * SW];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int nl = lane & 15, kq = lane >> 4;
-    const int row = blockIdx.y;
-    const int img = row / a.H, y = row - img * a.H;
-    const int x0 = blockIdx.x * 256 + wave * 64;
-    const int cg = blockIdx.z * 64;
-    const int nmt = min(4, (a.Co - cg) >> 4);
-    f4v acc[4][4];
-#pragma unroll
-    for (int m = 0; m < 4; ++m)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) acc[m][t] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int ky = 0; ky < 3; ++ky) {
-        const int yy = y + ky - 1;
-        if (yy < 0 || yy >= a.H) continue;   // uniform in the workgroup
-        __syncthreads();                     // the previous kernel row's weights are consumed
-        for (int e = threadIdx.x; e < NKI * 4 * 64; e += 256) {
-            const int g = e >> 6, co = e & 63;
-            u8v v = u8v{0, 0, 0, 0, 0, 0, 0, 0};
-            if (g < NG && cg + co < a.Co) {
-                const int kx = g / CB, cb = g - kx * CB;
-                v = *(const u8v *)(a.w + ((long long)(3 * ky + kx) * a.Co + cg + co) * CI + 8 * cb);
-            }
-            sw[g * SW + co] = v;
+    const int img = blockIdx.y / a.hblocks, hb = blockIdx.y - img * a.hblocks;
+    const int y0 = (hb * 4 + wave) * a.rows, y1 = min(y0 + a.rows, a.H);   // output rows of the wave
+    const int x0 = blockIdx.x * (16 * NT);
+    const int cg = blockIdx.z * (16 * NM);
+    const int nmt = min(NM, (a.Co - cg) >> 4);
+    for (int e = threadIdx.x; e < 3 * NKI * 4 * 16 * NM; e += 256) {
+        const int co = e % (16 * NM), kg = e / (16 * NM);      // kg = ky * 4 NKI + group
+        const int ky = kg / (4 * NKI), gg = kg - ky * (4 * NKI);
+        const bool second = gg >= 4 * N0;
+        const int g = second ? gg - 4 * N0 : gg, cbs = second ? (B1 > 0 ? B1 : 1) : B0;
+        u8v v = u8v{0, 0, 0, 0, 0, 0, 0, 0};
+        if (g < 3 * cbs && cg + co < a.Co) {
+            const int kx = g / cbs, cb = g - kx * cbs;
+            v = *(const u8v *)(a.w + ((long long)(3 * ky + kx) * a.Co + cg + co) * CI + (second ? C0 : 0) + 8 * cb);
         }
-        __syncthreads();
-        const uint16_t *xrow = a.x + (long long)(img * a.H + yy) * a.W * CI;
+        sw[kg * SW + co] = v;
+    }
+    float bias[NM][4];
+#pragma unroll
+    for (int m = 0; m < NM; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int co = cg + m * 16 + 4 * kq + r;
+            bias[m][r] = (a.bias && co < a.Co) ? a.bias[co] : 0.0f;
+        }
+    __syncthreads();
+    if (y0 >= y1) return;
+
+    // input fragment i, t of row yi (a group past the last tap: zero)
+    auto load = [&](int yi, int i, int t) -> u8v {
+        if (i < N0) {
+            const int g = 4 * i + kq, kx = g / B0, cb = g - kx * B0;
+            int px = x0 + 16 * t + nl + kx - 1;
+            const uint16_t *row;
+            int w;
+            if (CAT) {
+                w = a.W >> 1;
+                px >>= 1;                                  // -1 stays -1, W becomes W / 2
+                row = a.up + (long long)(img * (a.H >> 1) + (yi >> 1)) * w * C0;
+            } else {
+                w = a.W;
+                row = a.x + (long long)(img * a.H + yi) * w * C0;
+            }
+            int off = (px * C0 + 8 * cb) * 2;
+            if (4 * N0 > 3 * B0 && g >= 3 * B0) off = -16;
+            return __builtin_bit_cast(u8v, __builtin_amdgcn_raw_buffer_load_b128(row_rsrc(row, w * C0 * 2), off, 0, 0));
+        }
+        constexpr int CC = C1 > 0 ? C1 : 8, BB = CC / 8;
+        const int g = 4 * (i - N0) + kq, kx = g / BB, cb = g - kx * BB;
+        const int px = x0 + 16 * t + nl + kx - 1;
+        const uint16_t *row = a.x + (long long)(img * a.H + yi) * a.W * CC;
+        int off = (px * CC + 8 * cb) * 2;
+        if (4 * N1 > 3 * B1 && g >= 3 * BB) off = -16;
+        return __builtin_bit_cast(u8v, __builtin_amdgcn_raw_buffer_load_b128(row_rsrc(row, a.W * CC * 2), off, 0, 0));
+    };
+    u8v b[NKI][NT];
+    f4v acc[3][NM][NT];
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[q][m][t] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+    const int ya = max(y0 - 1, 0), yb = min(y1, a.H - 1);      // input rows
+#pragma unroll
+    for (int i = 0; i < NKI; ++i)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) b[i][t] = load(ya, i, t);
+
+    const int orow = a.W * a.Co * 2;                           // bytes of an output (or mask) row
+    auto ooff = [&](int t, int m) -> int { return ((x0 + 16 * t + nl) * a.Co + cg + m * 16 + 4 * kq) * 2; };
+    auto finish = [&](int y, f4v (&ac)[NM][NT], const u2v (&mk)[NM][NT]) {
+        const long long row = (long long)(img * a.H + y) * a.W;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int m = 0; m < NM; ++m) {
+                if (m < nmt) {
+                    float v[4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        v[r] = ac[m][t][r] + bias[m][r];
+                        if (a.relu) v[r] = fmaxf(v[r], 0.0f);
+                    }
+                    if (a.mask) {
+                        if (!(u_bf2f((uint16_t)(mk[m][t].x & 0xffffu)) > 0.0f)) v[0] = 0.0f;
+                        if (!(u_bf2f((uint16_t)(mk[m][t].x >> 16)) > 0.0f)) v[1] = 0.0f;
+                        if (!(u_bf2f((uint16_t)(mk[m][t].y & 0xffffu)) > 0.0f)) v[2] = 0.0f;
+                        if (!(u_bf2f((uint16_t)(mk[m][t].y >> 16)) > 0.0f)) v[3] = 0.0f;
+                    }
+                    if (a.y16) {
+                        const u2v o = u2v{(unsigned)u_f2bf(v[0]) | ((unsigned)u_f2bf(v[1]) << 16),
+                                          (unsigned)u_f2bf(v[2]) | ((unsigned)u_f2bf(v[3]) << 16)};
+                        __builtin_amdgcn_raw_buffer_store_b64(o, row_rsrc(a.y16 + row * a.Co, orow), ooff(t, m), 0, 0);
+                    }
+                    if (a.y1 && m == 0) {   // channel 0: lanes kq 0 of the first tile
+                        const int off = (kq == 0 && cg == 0) ? (x0 + 16 * t + nl) * 4 : -4;
+                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[0]), row_rsrc(a.y1 + row, a.W * 4), off, 0, 0);
+                    }
+                }
+                ac[m][t] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+    };
+    // the ReLU mask of output row y, asked for before the next input row
+    auto masks = [&](int y, u2v (&mk)[NM][NT]) {
+        const rsrc_t rs = row_rsrc(a.mask ? a.mask + (long long)(img * a.H + max(y, 0)) * a.W * a.Co : a.w, a.mask ? orow : 0);
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+                if (m < nmt) mk[m][t] = __builtin_amdgcn_raw_buffer_load_b64(rs, ooff(t, m), 0, 0);
+    };
+    // one input row: output rows yi+1 (ky 0), yi (ky 1), yi-1 (ky 2, complete
+    // after it) in the accumulators a0, a1, a2
+    auto step = [&](int yi, f4v (&a0)[NM][NT], f4v (&a1)[NM][NT], f4v (&a2)[NM][NT]) {
+        const bool d0 = yi + 1 < y1, d1 = yi >= y0 && yi < y1, d2 = yi - 1 >= y0;   // uniform
+        const int yn = min(yi + 1, yb);
+        u2v mk[NM][NT];
+        if (a.mask) masks(yi - 1, mk);
 #pragma unroll
         for (int i = 0; i < NKI; ++i) {
-            const int g = 4 * i + kq;
-            const bool live = g < NG;
-            const int kx = live ? g / CB : 0, cb = live ? g - (g / CB) * CB : 0;
-            u8v b[4];
+            auto mult = [&](int ky, f4v (&ac)[NM][NT]) {
+                const u8v *w = sw + (ky * 4 * NKI + 4 * i + kq) * SW + nl;
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const int xx = x0 + 16 * t + nl + kx - 1;
-                b[t] = u8v{0, 0, 0, 0, 0, 0, 0, 0};
-                if (live && xx >= 0 && xx < a.W) b[t] = *(const u8v *)(xrow + (long long)xx * CI + 8 * cb);
-            }
+                for (int m = 0; m < NM; ++m)
+                    if (m < nmt) {
+                        const u8v av = w[16 * m];
 #pragma unroll
-            for (int m = 0; m < 4; ++m)
-                if (m < nmt) {
-                    const u8v av = sw[g * SW + 16 * m + nl];
+                        for (int t = 0; t < NT; ++t) ac[m][t] = mfma32(av, b[i][t], ac[m][t]);
+                    }
+            };
+            if (d0) mult(0, a0);
+            if (d1) mult(1, a1);
+            if (d2) mult(2, a2);
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) acc[m][t] = mfma32(av, b[t], acc[m][t]);
-                }
+            for (int t = 0; t < NT; ++t) b[i][t] = load(yn, i, t);
         }
+        if (d2) finish(yi - 1, a2, mk);
+    };
+    auto last = [&](int y, f4v (&ac)[NM][NT]) {               // the image's last row
+        u2v mk[NM][NT];
+        if (a.mask) masks(y, mk);
+        finish(y, ac, mk);
+    };
+    // the accumulators take turns: after a row, a2's is free for row yi+2
+    int yi = ya;
+    for (; yi + 2 <= yb; yi += 3) {
+        step(yi, acc[0], acc[1], acc[2]);
+        step(yi + 1, acc[2], acc[0], acc[1]);
+        step(yi + 2, acc[1], acc[2], acc[0]);
     }
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        const int xo = x0 + 16 * t + nl;
-        if (xo >= a.W) continue;
-        const long long pix = (long long)(img * a.H + y) * a.W + xo;
-#pragma unroll
-        for (int m = 0; m < 4; ++m)
-            if (m < nmt) {
-                const int co0 = cg + m * 16 + 4 * kq;
-                float v[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    v[r] = acc[m][t][r];
-                    if (a.bias) v[r] += a.bias[co0 + r];
-                    if (a.relu) v[r] = fmaxf(v[r], 0.0f);
-                }
-                if (a.mask) {
-                    const ushort4 mk = *(const ushort4 *)(a.mask + pix * a.Co + co0);
-                    if (!(u_bf2f(mk.x) > 0.0f)) v[0] = 0.0f;
-                    if (!(u_bf2f(mk.y) > 0.0f)) v[1] = 0.0f;
-                    if (!(u_bf2f(mk.z) > 0.0f)) v[2] = 0.0f;
-                    if (!(u_bf2f(mk.w) > 0.0f)) v[3] = 0.0f;
-                }
-                if (a.y16)
-                    *(ushort4 *)(a.y16 + pix * a.Co + co0) =
-                        make_ushort4(u_f2bf(v[0]), u_f2bf(v[1]), u_f2bf(v[2]), u_f2bf(v[3]));
-                if (a.y32) *(float4 *)(a.y32 + pix * a.Co + co0) = make_float4(v[0], v[1], v[2], v[3]);
-            }
+    if (yi <= yb) {
+        step(yi, acc[0], acc[1], acc[2]);
+        if (yi + 1 <= yb) {
+            step(yi + 1, acc[2], acc[0], acc[1]);
+            if (yb == y1 - 1) last(yb, acc[0]);
+        } else if (yb == y1 - 1) {
+            last(yb, acc[1]);
+        }
+    } else if (yb == y1 - 1) {
+        last(yb, acc[2]);
     }
+}
+
+template <int CI, int NM, int NT, bool CAT> static void conv_launch(ConvArgs a, hipStream_t st)
+{
+    // rows per wave: a strip of R rows loads R + 2; shorter where the image
+    // would leave CUs without a workgroup
+    const int cols = (a.W + 16 * NT - 1) / (16 * NT), z = (a.Co + 16 * NM - 1) / (16 * NM);
+    int R = 12;
+    while (R > 2 && (long long)cols * z * a.n * ((a.H + 4 * R - 1) / (4 * R)) < 1024) R /= 2;
+    a.rows = R;
+    a.hblocks = (a.H + 4 * R - 1) / (4 * R);
+    hipLaunchKernelGGL((k_conv3x3<CI, NM, NT, CAT>), dim3((unsigned)cols, (unsigned)(a.n * a.hblocks), (unsigned)z),
+                       dim3(256), 0, st, a);
 }
 
 hipError_t launch_conv3x3(const ConvArgs &a, hipStream_t st)
 {
     if (a.Co % 16 || a.Co < 16 || a.n < 1 || a.H < 1 || a.W < 1) return hipErrorInvalidValue;
-    dim3 grid((unsigned)((a.W + 255) / 256), (unsigned)(a.n * a.H), (unsigned)((a.Co + 63) / 64));
-    switch (a.Ci) {
-    case 16: hipLaunchKernelGGL(k_conv3x3<16>, grid, dim3(256), 0, st, a); break;
-    case 32: hipLaunchKernelGGL(k_conv3x3<32>, grid, dim3(256), 0, st, a); break;
-    case 48: hipLaunchKernelGGL(k_conv3x3<48>, grid, dim3(256), 0, st, a); break;
-    case 64: hipLaunchKernelGGL(k_conv3x3<64>, grid, dim3(256), 0, st, a); break;
-    case 80: hipLaunchKernelGGL(k_conv3x3<80>, grid, dim3(256), 0, st, a); break;
-    case 112: hipLaunchKernelGGL(k_conv3x3<112>, grid, dim3(256), 0, st, a); break;
+    if (a.up && ((a.H | a.W) & 1)) return hipErrorInvalidValue;
+    // output channel tiles per wave: all of them up to four, 5 as 3 + 2, 7 as 4 + 3
+    // (112 input channels: one, its weights would fill the LDS of a CU)
+    const int tiles = a.Co / 16, nm = a.Ci == 112 ? 1 : (tiles <= 4 ? tiles : (tiles == 5 ? 3 : 4));
+    switch ((a.up ? 10000 : 0) + a.Ci * 10 + nm) {   // the layers and their data gradients
+    case 161: conv_launch<16, 1, 4, false>(a, st); break;
+    case 162: conv_launch<16, 2, 2, false>(a, st); break;
+    case 163: conv_launch<16, 3, 2, false>(a, st); break;
+    case 321: conv_launch<32, 1, 4, false>(a, st); break;
+    case 322: conv_launch<32, 2, 2, false>(a, st); break;
+    case 323: conv_launch<32, 3, 2, false>(a, st); break;
+    case 482: conv_launch<48, 2, 2, false>(a, st); break;
+    case 483: conv_launch<48, 3, 2, false>(a, st); break;
+    case 484: conv_launch<48, 4, 2, false>(a, st); break;
+    case 643: conv_launch<64, 3, 2, false>(a, st); break;
+    case 644: conv_launch<64, 4, 2, false>(a, st); break;
+    case 10481: conv_launch<48, 1, 4, true>(a, st); break;
+    case 10802: conv_launch<80, 2, 2, true>(a, st); break;
+    case 11121: conv_launch<112, 1, 2, true>(a, st); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -156,7 +291,8 @@ hipError_t launch_conv3x3(const ConvArgs &a, hipStream_t st)
 // pixels of a row.  Per segment the output gradient dY[64 px][CO] and, for
 // each kx, the shifted input row X[y + ky - 1][x + kx - 1][CI] are staged in
 // LDS transposed ([channel][pixel], zero outside the image; one 16-byte load
-// of 8 channels per thread and item), so that a lane reads 8 consecutive
+// of 8 channels per thread and item, issued while the segment before is
+// multiplied), so that a lane reads 8 consecutive
 // pixels of one channel as one 16-byte operand: A = dY^T (co = lane % 16),
 // B = X_shift (ci = lane % 16).  The 3 x (CO/16) x (CI/16) tiles of the
 // kernel row are dealt round-robin to the waves (at most 16 each) and
@@ -182,36 +318,81 @@ __global__ __launch_bounds__(256) void k_wgrad(WgradArgs a)
 #pragma unroll
     for (int q = 0; q < 16; ++q) acc[q] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
     float bsum = 0.0f;
-    for (int r = r0; r < r1; ++r) {
-        const int img = r / a.H, y = r - img * a.H;
-        const int yy = y + ky - 1;
+    // items (pixel, 8 channels) of a segment per thread
+    constexpr int ND = (kSegPx * (CO / 8) + 255) / 256, NX = ((kSegPx + 2) * (CI / 8) + 255) / 256;
+    u8v rd[ND], rx[NX];
+    const int nseg = (a.W + kSegPx - 1) / kSegPx;
+    // the segment's loads: zero outside the row (buffer range) and, by an
+    // empty range, for a row outside the image
+    auto fetch = [&](int r, int x0) {
+        const int img = r / a.H, y = r - img * a.H, yy = y + ky - 1;
         const bool yin = yy >= 0 && yy < a.H;
-        for (int x0 = 0; x0 < a.W; x0 += kSegPx) {
+        const rsrc_t sd = row_rsrc(a.dy + (long long)r * a.W * CO, a.W * CO * 2);
+#pragma unroll
+        for (int k = 0; k < ND; ++k) {
+            const int e = (int)threadIdx.x + 256 * k, j = e / (CO / 8), c8 = e - j * (CO / 8);
+            rd[k] = __builtin_bit_cast(u8v, __builtin_amdgcn_raw_buffer_load_b128(sd, ((x0 + j) * CO + 8 * c8) * 2, 0, 0));
+        }
+        const long long xr = yin ? (long long)(img * a.H + yy) : 0;
+        if (!a.up) {
+            const rsrc_t sx_ = row_rsrc(a.x + xr * a.W * CI, yin ? a.W * CI * 2 : 0);
+#pragma unroll
+            for (int k = 0; k < NX; ++k) {
+                const int e = (int)threadIdx.x + 256 * k, jj = e / (CI / 8), c8 = e - jj * (CI / 8);
+                rx[k] = __builtin_bit_cast(
+                    u8v, __builtin_amdgcn_raw_buffer_load_b128(sx_, ((x0 + jj - 1) * CI + 8 * c8) * 2, 0, 0));
+            }
+        } else {   // up-sampled and skip channels, as in k_conv3x3: one of the two reads zero
+            constexpr int CU = cat_up(CI), CS = CI - CU > 0 ? CI - CU : 8;
+            const long long ur = yin ? (long long)(img * (a.H >> 1) + (yy >> 1)) : 0;
+            const int wu = a.W >> 1;
+            const rsrc_t su = row_rsrc(a.up + ur * wu * CU, yin ? wu * CU * 2 : 0);
+            const rsrc_t ss = row_rsrc(a.x + xr * a.W * CS, yin ? a.W * CS * 2 : 0);
+#pragma unroll
+            for (int k = 0; k < NX; ++k) {
+                const int e = (int)threadIdx.x + 256 * k, jj = e / (CI / 8), c8 = e - jj * (CI / 8);
+                const int px = x0 + jj - 1;
+                const bool up = c8 < CU / 8;
+                const u8v vu = __builtin_bit_cast(
+                    u8v, __builtin_amdgcn_raw_buffer_load_b128(su, up ? ((px >> 1) * CU + 8 * c8) * 2 : -16, 0, 0));
+                const u8v vs = __builtin_bit_cast(
+                    u8v, __builtin_amdgcn_raw_buffer_load_b128(ss, up ? -16 : (px * CS + 8 * c8 - CU) * 2, 0, 0));
+                rx[k] = vu | vs;
+            }
+        }
+    };
+    fetch(r0, 0);
+    for (int r = r0; r < r1; ++r) {
+        for (int sg = 0; sg < nseg; ++sg) {
             __syncthreads();   // the previous segment is consumed
             // dY[y][x0 + j][8c .. 8c+7] -> sdy[8c + k][j]
-            for (int e = threadIdx.x; e < kSegPx * (CO / 8); e += 256) {
-                const int j = e / (CO / 8), c8 = e - j * (CO / 8);
-                const int x = x0 + j;
-                u8v v = u8v{0, 0, 0, 0, 0, 0, 0, 0};
-                if (x < a.W) v = *(const u8v *)(a.dy + ((long long)r * a.W + x) * CO + 8 * c8);
 #pragma unroll
-                for (int k = 0; k < 8; ++k) sdy[(8 * c8 + k) * kSegPad + j] = v[k];
+            for (int n = 0; n < ND; ++n) {
+                const int e = (int)threadIdx.x + 256 * n, j = e / (CO / 8), c8 = e - j * (CO / 8);
+                if (e < kSegPx * (CO / 8))
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) sdy[(8 * c8 + k) * kSegPad + j] = rd[n][k];
             }
             // X[yy][x0 + jj - 1][8c .. 8c+7] -> sx[kx][8c + k][jj - kx]
-            for (int e = threadIdx.x; e < (kSegPx + 2) * (CI / 8); e += 256) {
-                const int jj = e / (CI / 8), c8 = e - jj * (CI / 8);
-                const int x = x0 + jj - 1;
-                u8v v = u8v{0, 0, 0, 0, 0, 0, 0, 0};
-                if (yin && x >= 0 && x < a.W) v = *(const u8v *)(a.x + ((long long)(img * a.H + yy) * a.W + x) * CI + 8 * c8);
 #pragma unroll
-                for (int kx = 0; kx < 3; ++kx) {
-                    const int j = jj - kx;
-                    if (j >= 0 && j < kSegPx)
+            for (int n = 0; n < NX; ++n) {
+                const int e = (int)threadIdx.x + 256 * n, jj = e / (CI / 8), c8 = e - jj * (CI / 8);
+                if (e < (kSegPx + 2) * (CI / 8))
 #pragma unroll
-                        for (int k = 0; k < 8; ++k) sx[(kx * CI + 8 * c8 + k) * kSegPad + j] = v[k];
-                }
+                    for (int kx = 0; kx < 3; ++kx) {
+                        const int j = jj - kx;
+                        if (j >= 0 && j < kSegPx)
+#pragma unroll
+                            for (int k = 0; k < 8; ++k) sx[(kx * CI + 8 * c8 + k) * kSegPad + j] = rx[n][k];
+                    }
             }
             __syncthreads();
+            // the next segment's loads go out before this one is multiplied
+            {
+                const bool wrap = sg + 1 == nseg;
+                const int rn = wrap ? min(r + 1, r1 - 1) : r;
+                fetch(rn, wrap ? 0 : (sg + 1) * kSegPx);
+            }
             if (ky == 0 && (int)threadIdx.x < CO)
 #pragma unroll 8
                 for (int j = 0; j < kSegPx; ++j) bsum += u_bf2f(sdy[threadIdx.x * kSegPad + j]);
@@ -255,13 +436,13 @@ __global__ void k_reduce_chunks(int nchunks, long long len, const float *part, f
          e += (long long)gridDim.x * blockDim.x) {
         float s = 0.0f;
         int c = 0;
-        for (; c + 4 <= nchunks; c += 4) {
-            const float p0 = part[(long long)c * len + e], p1 = part[(long long)(c + 1) * len + e];
-            const float p2 = part[(long long)(c + 2) * len + e], p3 = part[(long long)(c + 3) * len + e];
-            s += p0;
-            s += p1;
-            s += p2;
-            s += p3;
+        // 32 partials are read before the first is added
+        for (; c + 32 <= nchunks; c += 32) {
+            float p[32];
+#pragma unroll
+            for (int k = 0; k < 32; ++k) p[k] = part[(long long)(c + k) * len + e];
+#pragma unroll
+            for (int k = 0; k < 32; ++k) s += p[k];
         }
         for (; c < nchunks; ++c) s += part[(long long)c * len + e];
         out[e] = s;
@@ -332,79 +513,79 @@ hipError_t launch_wgrad(const WgradArgs &a, float *dw, float *db, hipStream_t st
 }
 
 // ---------------------------------------------------------------------------
-// 2x2 average pooling, nearest upsampling with channel concatenation, and
-// their adjoints with the ReLU mask of the activation they feed.
+// 2x2 average pooling and the adjoints of pooling and nearest upsampling with
+// the ReLU mask of the activation they feed.  Bytes only: one thread per 8
+// channels of a pixel (16-byte accesses), one image row per blockIdx.y, so
+// the only division is by the channel count, a constant.
 // ---------------------------------------------------------------------------
-__global__ void k_pool(int n, int H, int W, int C, const uint16_t *x, uint16_t *y)
+__device__ __forceinline__ void unpack8(const uint16_t *p, float (&f)[8])
 {
-    const int h = H / 2, w = W / 2;
-    const long long total = (long long)n * h * w * C;
-    for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < total;
-         e += (long long)gridDim.x * blockDim.x) {
-        const int c = (int)(e % C);
-        const long long q = e / C;
-        const int xo = (int)(q % w), yo = (int)((q / w) % h), im = (int)(q / ((long long)w * h));
-        const long long b = ((long long)(im * H + 2 * yo) * W + 2 * xo) * C + c;
-        const float s = (u_bf2f(x[b]) + u_bf2f(x[b + C])) + (u_bf2f(x[b + (long long)W * C]) +
-                                                             u_bf2f(x[b + (long long)W * C + C]));
-        y[e] = u_f2bf(0.25f * s);
-    }
+    const u8v v = *(const u8v *)p;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) f[k] = u_bf2f(v[k]);
+}
+
+template <int C> __global__ void k_pool(int H, int W, const uint16_t *x, uint16_t *y)
+{
+    constexpr int C8 = C / 8;
+    const int w = W / 2, e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= w * C8) return;
+    const int xo = e / C8, c = 8 * (e - xo * C8);
+    const long long row = blockIdx.y;                     // image * H/2 + y
+    const uint16_t *b = x + ((2 * row * W + 2 * xo) * C + c);
+    float p[8], q[8], r[8], t[8];
+    unpack8(b, p);
+    unpack8(b + C, q);
+    unpack8(b + (long long)W * C, r);
+    unpack8(b + (long long)W * C + C, t);
+    u8v o;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) o[k] = u_f2bf(0.25f * ((p[k] + q[k]) + (r[k] + t[k])));
+    *(u8v *)(y + (row * w + xo) * C + c) = o;
 }
 
 // dact[p][c] = (act > 0) * (0.25 * dpool[p/2][c] + dcat[p][off + c])
-__global__ void k_pool_bwd(int n, int H, int W, int C, const uint16_t *dpool, const uint16_t *dcat, int ccat, int off,
+template <int C>
+__global__ void k_pool_bwd(int H, int W, const uint16_t *dpool, const uint16_t *dcat, int ccat, int off,
                            const uint16_t *act, uint16_t *dact)
 {
-    const int h = H / 2, w = W / 2;
-    const long long total = (long long)n * H * W * C;
-    for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < total;
-         e += (long long)gridDim.x * blockDim.x) {
-        const int c = (int)(e % C);
-        const long long p = e / C;
-        const int x = (int)(p % W), yq = (int)((p / W) % H), im = (int)(p / ((long long)W * H));
-        const long long q = ((long long)(im * h + yq / 2) * w + x / 2) * C + c;
-        float v = 0.25f * u_bf2f(dpool[q]);
-        if (dcat) v += u_bf2f(dcat[p * ccat + off + c]);
-        if (!(u_bf2f(act[e]) > 0.0f)) v = 0.0f;
-        dact[e] = u_f2bf(v);
-    }
+    constexpr int C8 = C / 8;
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= W * C8) return;
+    const int x = e / C8, c = 8 * (e - x * C8);
+    const long long row = blockIdx.y, p = row * W + x;    // row: image * H + y
+    const long long img = row / H, yl = (row - img * H) / 2;
+    float dp[8], dc[8], ac[8];
+    unpack8(dpool + ((img * (H / 2) + yl) * (W / 2) + x / 2) * C + c, dp);
+    unpack8(dcat + p * ccat + off + c, dc);
+    unpack8(act + p * C + c, ac);
+    u8v o;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) o[k] = ac[k] > 0.0f ? u_f2bf(0.25f * dp[k] + dc[k]) : (uint16_t)0;
+    *(u8v *)(dact + p * C + c) = o;
 }
 
-// cat[p][0..Cu) = up[p/2][c]; cat[p][Cu..Cu+Cs) = skip[p][c]
-__global__ void k_upcat(int n, int H, int W, int Cu, int Cs, const uint16_t *up, const uint16_t *skip, uint16_t *cat)
+// dlow[q][c] = (act_low > 0) * sum over the 2x2 children of dcat[child][c], c < CU
+template <int CU>
+__global__ void k_up_bwd(int H, int W, int Ccat, const uint16_t *dcat, const uint16_t *act_low, uint16_t *dlow)
 {
-    const int Cc = Cu + Cs, h = H / 2, w = W / 2;
-    const long long total = (long long)n * H * W * Cc;
-    for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < total;
-         e += (long long)gridDim.x * blockDim.x) {
-        const int c = (int)(e % Cc);
-        const long long p = e / Cc;
-        if (c < Cu) {
-            const int x = (int)(p % W), yq = (int)((p / W) % H), im = (int)(p / ((long long)W * H));
-            cat[e] = up[((long long)(im * h + yq / 2) * w + x / 2) * Cu + c];
-        } else {
-            cat[e] = skip[p * Cs + (c - Cu)];
-        }
-    }
-}
-
-// dlow[q][c] = (act_low > 0) * sum over the 2x2 children of dcat[child][c], c < Cu
-__global__ void k_up_bwd(int n, int H, int W, int Cu, int Ccat, const uint16_t *dcat, const uint16_t *act_low,
-                         uint16_t *dlow)
-{
-    const int h = H / 2, w = W / 2;
-    const long long total = (long long)n * h * w * Cu;
-    for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < total;
-         e += (long long)gridDim.x * blockDim.x) {
-        const int c = (int)(e % Cu);
-        const long long q = e / Cu;
-        const int xo = (int)(q % w), yo = (int)((q / w) % h), im = (int)(q / ((long long)w * h));
-        const long long b = ((long long)(im * H + 2 * yo) * W + 2 * xo);
-        float s = (u_bf2f(dcat[b * Ccat + c]) + u_bf2f(dcat[(b + 1) * Ccat + c])) +
-                  (u_bf2f(dcat[(b + W) * Ccat + c]) + u_bf2f(dcat[(b + W + 1) * Ccat + c]));
-        if (!(u_bf2f(act_low[e]) > 0.0f)) s = 0.0f;
-        dlow[e] = u_f2bf(s);
-    }
+    constexpr int C8 = CU / 8;
+    const int w = W / 2, e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= w * C8) return;
+    const int xo = e / C8, c = 8 * (e - xo * C8);
+    const long long row = blockIdx.y;                     // image * H/2 + y
+    const uint16_t *b = dcat + ((2 * row * W + 2 * xo) * Ccat + c);
+    const long long q = (row * w + xo) * CU + c;
+    float p0[8], p1[8], p2[8], p3[8], ac[8];
+    unpack8(b, p0);
+    unpack8(b + Ccat, p1);
+    unpack8(b + (long long)W * Ccat, p2);
+    unpack8(b + (long long)W * Ccat + Ccat, p3);
+    unpack8(act_low + q, ac);
+    u8v o;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) o[k] = ac[k] > 0.0f ? u_f2bf((p0[k] + p1[k]) + (p2[k] + p3[k])) : (uint16_t)0;
+    *(u8v *)(dlow + q) = o;
 }
 
 static dim3 grid_for(long long total)
@@ -412,62 +593,79 @@ static dim3 grid_for(long long total)
     return dim3((unsigned)std::max<long long>(1, std::min<long long>(8192, (total + 255) / 256)));
 }
 
+static dim3 row_grid(int items, long long rows) { return dim3((unsigned)((items + 255) / 256), (unsigned)rows); }
+
 hipError_t launch_pool(int n, int H, int W, int C, const uint16_t *x, uint16_t *y, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_pool, grid_for((long long)n * (H / 2) * (W / 2) * C), dim3(256), 0, st, n, H, W, C, x, y);
+    const dim3 g = row_grid(W / 2 * (C / 8), (long long)n * (H / 2));
+    switch (C) {
+    case 16: hipLaunchKernelGGL(k_pool<16>, g, dim3(256), 0, st, H, W, x, y); break;
+    case 32: hipLaunchKernelGGL(k_pool<32>, g, dim3(256), 0, st, H, W, x, y); break;
+    case 48: hipLaunchKernelGGL(k_pool<48>, g, dim3(256), 0, st, H, W, x, y); break;
+    default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 hipError_t launch_pool_bwd(int n, int H, int W, int C, const uint16_t *dpool, const uint16_t *dcat, int ccat, int off,
                            const uint16_t *act, uint16_t *dact, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_pool_bwd, grid_for((long long)n * H * W * C), dim3(256), 0, st, n, H, W, C, dpool, dcat, ccat,
-                       off, act, dact);
-    return hipGetLastError();
-}
-hipError_t launch_upcat(int n, int H, int W, int Cu, int Cs, const uint16_t *up, const uint16_t *skip, uint16_t *cat,
-                        hipStream_t st)
-{
-    hipLaunchKernelGGL(k_upcat, grid_for((long long)n * H * W * (Cu + Cs)), dim3(256), 0, st, n, H, W, Cu, Cs, up, skip,
-                       cat);
+    const dim3 g = row_grid(W * (C / 8), (long long)n * H);
+    switch (C) {
+    case 16: hipLaunchKernelGGL(k_pool_bwd<16>, g, dim3(256), 0, st, H, W, dpool, dcat, ccat, off, act, dact); break;
+    case 32: hipLaunchKernelGGL(k_pool_bwd<32>, g, dim3(256), 0, st, H, W, dpool, dcat, ccat, off, act, dact); break;
+    case 48: hipLaunchKernelGGL(k_pool_bwd<48>, g, dim3(256), 0, st, H, W, dpool, dcat, ccat, off, act, dact); break;
+    default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 hipError_t launch_up_bwd(int n, int H, int W, int Cu, int Ccat, const uint16_t *dcat, const uint16_t *act_low,
                          uint16_t *dlow, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_up_bwd, grid_for((long long)n * (H / 2) * (W / 2) * Cu), dim3(256), 0, st, n, H, W, Cu, Ccat,
-                       dcat, act_low, dlow);
+    const dim3 g = row_grid(W / 2 * (Cu / 8), (long long)n * (H / 2));
+    switch (Cu) {
+    case 32: hipLaunchKernelGGL(k_up_bwd<32>, g, dim3(256), 0, st, H, W, Ccat, dcat, act_low, dlow); break;
+    case 48: hipLaunchKernelGGL(k_up_bwd<48>, g, dim3(256), 0, st, H, W, Ccat, dcat, act_low, dlow); break;
+    case 64: hipLaunchKernelGGL(k_up_bwd<64>, g, dim3(256), 0, st, H, W, Ccat, dcat, act_low, dlow); break;
+    default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
 // Input packing, output extraction, loss, parameter casts and Adam
 // ---------------------------------------------------------------------------
-// x [n][3][H][W] fp32 (planar) -> [n][H][W][16] bf16 with channels 3..15 zero
-__global__ void k_pack_input(int n, int H, int W, const float *x, uint16_t *xp)
+// x [n][3][H][W] fp32 (planar) -> [n][H][W][16] bf16 with channels 3..15
+// zero: one pixel per thread
+__global__ void k_pack_input(long long hw, const float *x, uint16_t *xp)
 {
-    const long long total = (long long)n * H * W * 16;
-    for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < total;
-         e += (long long)gridDim.x * blockDim.x) {
-        const int c = (int)(e % 16);
-        const long long p = e / 16;
-        const long long hw = (long long)H * W;
-        const long long im = p / hw, r = p - im * hw;
-        xp[e] = (c < 3) ? u_f2bf(x[(im * 3 + c) * hw + r]) : (uint16_t)0;
-    }
+    const long long r = blockIdx.x * (long long)blockDim.x + threadIdx.x, im = blockIdx.y;
+    if (r >= hw) return;
+    const float *b = x + im * 3 * hw + r;
+    const u8v z = u8v{0, 0, 0, 0, 0, 0, 0, 0};
+    u8v v = z;
+    v[0] = u_f2bf(b[0]);
+    v[1] = u_f2bf(b[hw]);
+    v[2] = u_f2bf(b[2 * hw]);
+    u8v *o = (u8v *)(xp + (im * hw + r) * 16);
+    o[0] = v;
+    o[1] = z;
 }
 
-// loss = mean (y[p][0] - t[p])^2 ; dy[p][c] = c == 0 ? 2 (y - t) / P : 0
+// loss = mean (y[p] - t[p])^2 ; dy[p][c] = c == 0 ? 2 (y - t) / P : 0
 __global__ void k_mse(long long P, const float *y, const float *t, uint16_t *dy, double *part)
 {
     __shared__ double sh[256];
     double acc = 0.0;
     for (long long p = blockIdx.x * (long long)blockDim.x + threadIdx.x; p < P; p += (long long)gridDim.x * blockDim.x) {
-        const float d = y[p * 16] - t[p];
+        const float d = y[p] - t[p];
         acc += (double)d * (double)d;
         if (dy) {
-            dy[p * 16] = u_f2bf(2.0f * d / (float)P);
-#pragma unroll
-            for (int c = 1; c < 16; ++c) dy[p * 16 + c] = 0;
+            const u8v z = u8v{0, 0, 0, 0, 0, 0, 0, 0};
+            u8v v = z;
+            v[0] = u_f2bf(2.0f * d / (float)P);
+            u8v *o = (u8v *)(dy + p * 16);
+            o[0] = v;
+            o[1] = z;
         }
     }
     sh[threadIdx.x] = acc;
@@ -477,12 +675,6 @@ __global__ void k_mse(long long P, const float *y, const float *t, uint16_t *dy,
         __syncthreads();
     }
     if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
-}
-
-__global__ void k_extract(long long P, const float *y, float *out)
-{
-    for (long long p = blockIdx.x * (long long)blockDim.x + threadIdx.x; p < P; p += (long long)gridDim.x * blockDim.x)
-        out[p] = y[p * 16];
 }
 
 // fp32 master W [9][Co][Ci] -> bf16 W and bf16 W^T for the data gradient:
@@ -516,18 +708,14 @@ __global__ void k_adam(long long n, float *w, const float *g, float *m, float *v
 
 hipError_t launch_pack_input(int n, int H, int W, const float *x, uint16_t *xp, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_pack_input, grid_for((long long)n * H * W * 16), dim3(256), 0, st, n, H, W, x, xp);
+    const long long hw = (long long)H * W;
+    hipLaunchKernelGGL(k_pack_input, dim3((unsigned)((hw + 255) / 256), (unsigned)n), dim3(256), 0, st, hw, x, xp);
     return hipGetLastError();
 }
 hipError_t launch_mse(long long P, const float *y, const float *t, uint16_t *dy, double *part, int nblocks,
                       hipStream_t st)
 {
     hipLaunchKernelGGL(k_mse, dim3(nblocks), dim3(256), 0, st, P, y, t, dy, part);
-    return hipGetLastError();
-}
-hipError_t launch_extract(long long P, const float *y, float *out, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_extract, grid_for(P), dim3(256), 0, st, P, y, out);
     return hipGetLastError();
 }
 hipError_t launch_cast_weights(int Co, int Ci, const float *w32, uint16_t *w16, uint16_t *wt16, hipStream_t st)

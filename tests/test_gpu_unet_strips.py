@@ -1,0 +1,36 @@
+"""Shapes at the edges of the convolution's row strips and column tiles and
+of the weight gradient's segments, against the bf16 CPU oracle (the bounds of
+test_gpu_unet.py: bfloat16 accuracy of activations and gradients)."""
+import sys
+
+import numpy as np
+import pytest
+
+from common import product, rel_l2
+from unet_oracle import LAYERS, UNetOracle, offsets
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,h,w", [(1, 8, 8), (3, 8, 136), (1, 104, 72), (1, 152, 24), (2, 56, 64)])
+def test_unet_strips(n, h, w):
+    print("unet", n, h, w)
+    sys.stdout.flush()
+    net = product().UNet(seed=21)
+    p = net.get_params()
+    wo, bo, _ = offsets()
+    rng = np.random.default_rng(22)
+    for l, (ci, co, _) in enumerate(LAYERS):
+        p[bo[l]:bo[l] + co] = (rng.standard_normal(co) * 0.05).astype(np.float32)
+    net.set_params(p)
+    x = rng.standard_normal((n, 3, h, w)).astype(np.float32)
+    t = (0.5 * x[:, 0] - 0.3 * x[:, 1]).astype(np.float32)
+    ref = UNetOracle(p, bf16=True)
+    assert rel_l2(net.forward(x), ref.forward(x)) < 1e-2
+    loss, g = net.loss_grad(x, t)
+    lr, gr = ref.loss_grad(x, t)
+    assert abs(loss - lr) <= 1e-2 * abs(lr)
+    for l, (ci, co, _) in enumerate(LAYERS):
+        sl = slice(wo[l], bo[l] + co)
+        if np.max(np.abs(gr[sl])) > 0:
+            assert rel_l2(g[sl], gr[sl]) < 5e-2, l
