@@ -116,7 +116,8 @@ static int ensure_buffers(dn_unet *u, int n, int H, int W)
     UCHK(dal(&u->yout, P0));
     size_t plen = 0, blen = 0;
     for (int l = 0; l < kNL; ++l) {
-        const size_t nch = (size_t)wgrad_chunks(n, H >> level_of(l));
+        const int lv = level_of(l);
+        const size_t nch = (size_t)wgrad_chunks(n, H >> lv, W >> lv, kLayers[l].ci, kLayers[l].co);
         plen = std::max(plen, nch * 9 * kLayers[l].co * kLayers[l].ci);
         blen = std::max(blen, nch * kLayers[l].co);
     }
@@ -189,7 +190,6 @@ static int wgrad(dn_unet *u, int l, int n, int H, int W, const uint16_t *x, cons
     w.x = x;
     w.up = up;
     w.dy = dy;
-    w.chunk_rows = wgrad_chunk_rows(n, H);
     w.part = u->part;
     w.bpart = u->bpart;
     UCHK(launch_wgrad(w, u->g + u->woff[l], u->g + u->boff[l], u->stream));

@@ -27,14 +27,13 @@ struct WgradArgs {
     const uint16_t *x;         // layer input [n][H][W][Ci] (with up: the skip tensor, as in ConvArgs)
     const uint16_t *up;
     const uint16_t *dy;        // output gradient [n][H][W][Co]
-    int chunk_rows;            // image rows per partial: wgrad_chunk_rows(n, H)
-    float *part;               // [nchunks][9][Co][Ci]
-    float *bpart;              // [nchunks][Co]
+    float *part;               // [partials][9][Co][Ci]
+    float *bpart;              // [partials][Co]
+    int nseg, hchunks, chunk_rows;   // column segments, row chunks per image, rows per chunk (set by the launcher)
 };
-int wgrad_chunk_rows(int n, int H);
-int wgrad_chunks(int n, int H);   // partials of a layer of n images of H rows
-// dw [9][Co][Ci] and (if db) db [Co], fp32, summed in a fixed order
-hipError_t launch_wgrad(const WgradArgs &a, float *dw, float *db, hipStream_t st);
+int wgrad_chunks(int n, int H, int W, int Ci, int Co);   // partials of a layer
+// dw [9][Co][Ci] and db [Co], fp32, summed in a fixed order
+hipError_t launch_wgrad(WgradArgs a, float *dw, float *db, hipStream_t st);
 
 hipError_t launch_pool(int n, int H, int W, int C, const uint16_t *x, uint16_t *y, hipStream_t st);
 hipError_t launch_pool_bwd(int n, int H, int W, int C, const uint16_t *dpool, const uint16_t *dcat, int ccat, int off,

@@ -286,229 +286,278 @@ hipError_t launch_conv3x3(const ConvArgs &a, hipStream_t st)
 // ---------------------------------------------------------------------------
 // Weight gradient dW[tap][co][ci] = sum_p dY[p][co] * X[p + shift(tap)][ci]
 // as a GEMM over pixels (K) on MFMA 16x16x32, with the bias gradient
-// db[co] = sum_p dY[p][co].  Workgroup (4 waves): one chunk of image rows
-// (blockIdx.x) and one kernel row ky (blockIdx.y), walked in segments of 64
-// pixels of a row.  Per segment the output gradient dY[64 px][CO] and, for
-// each kx, the shifted input row X[y + ky - 1][x + kx - 1][CI] are staged in
-// LDS transposed ([channel][pixel], zero outside the image; one 16-byte load
-// of 8 channels per thread and item, issued while the segment before is
-// multiplied), so that a lane reads 8 consecutive
-// pixels of one channel as one 16-byte operand: A = dY^T (co = lane % 16),
-// B = X_shift (ci = lane % 16).  The 3 x (CO/16) x (CI/16) tiles of the
-// kernel row are dealt round-robin to the waves (at most 16 each) and
-// accumulated over the chunk; each chunk writes a partial, added over the
-// chunks in chunk order (deterministic).
+// db[co] = sum_p dY[p][co] (an operand of ones).  A workgroup (4 waves) walks
+// down rows y0..y1-1 of one image in a column segment of 128 pixels.  The
+// rows are staged in LDS as they lie in memory (channels last, 16-byte
+// accesses, loaded a row ahead) and read back transposed, four pixels of one
+// channel per lane, by ds_read_b64_tr_b16: A = dY^T (co = lane % 16) and
+// B = X (ci = lane % 16), 8 pixels per lane quarter, the taps as pixel and row
+// offsets.  Wave w multiplies pixels 32 w..32 w + 31 into all the workgroup's
+// tiles; their sum over the waves, in wave order, is the workgroup's partial,
+// and the partials are added in order (deterministic).
+//
+// Bytes bound it where one workgroup takes all nine taps (KYS 1: the X rows
+// rotate through three LDS slots and are loaded once); where the accumulators
+// allow three taps only (KYS 3) blockIdx.y selects ky, and blockIdx.z a group
+// of NTB input-channel tiles.  Transposing by 2-byte LDS stores, each X row
+// stored for three kx and loaded for three ky, took 140 us (16 -> 16 channels,
+// 4 x 304 x 1200) and 312 us (48 -> 16); now 25 and 49.
 // ---------------------------------------------------------------------------
-constexpr int kSegPx = 64;     // pixels per segment
-constexpr int kSegPad = 72;    // LDS pixels per channel row (16-byte aligned rows, staggered banks)
+constexpr int kSegPx = 128;    // pixels per segment
 
-template <int CI, int CO>
-__global__ __launch_bounds__(256) void k_wgrad(WgradArgs a)
+typedef short s4v __attribute__((ext_vector_type(4)));
+
+// 8 pixels (rows of `pitch` elements) of 16 channels, transposed: p points at
+// the lane's 4 channels of its pixel, see tr_lane
+__device__ __forceinline__ u8v tr_read(const uint16_t *p, int pitch)
 {
-    constexpr int NMT = CO / 16, NNT = CI / 16, NTILES = 3 * NMT * NNT;
-    static_assert(NTILES <= 64, "at most 16 tiles per wave");
-    __shared__ __attribute__((aligned(16))) uint16_t sdy[CO * kSegPad];
-    __shared__ __attribute__((aligned(16))) uint16_t sx[3 * CI * kSegPad];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    typedef __attribute__((address_space(3))) s4v *lds_t;
+    const s4v a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_t)p);
+    const s4v b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_t)(p + 4 * pitch));
+    return u8v{(unsigned short)a.x, (unsigned short)a.y, (unsigned short)a.z, (unsigned short)a.w,
+               (unsigned short)b.x, (unsigned short)b.y, (unsigned short)b.z, (unsigned short)b.w};
+}
+
+constexpr bool wgrad_cat(int CI, int CO) { return CI >= 80 || (CI == 48 && CO == 16); }
+
+template <int CI, int CO, int KYS, int NTB>
+__global__ __launch_bounds__(256, 2) void k_wgrad(WgradArgs a)
+{
+    constexpr bool CAT = wgrad_cat(CI, CO);              // the input is [up-sampled | skip]
+    constexpr int NMT = CO / 16, NNT = CI / 16, TAPS = 9 / KYS, NR = KYS == 1 ? 3 : 1;
+    constexpr int CW = 16 * NTB, BW = CW / 8;            // input channels of the workgroup
+    constexpr int XP = kSegPx + 2;                       // X pixels per row (x0 - 1 .. x0 + 128)
+    constexpr int ND = (kSegPx * (CO / 8) + 255) / 256, NX = (XP * BW + 255) / 256;
+    constexpr int NTILE = TAPS * NMT * NTB;
+    constexpr int RED = 4;                               // tiles summed over the waves per turn
+    constexpr int SXN = NR * XP * CW, SDN = kSegPx * CO;
+    __shared__ __attribute__((aligned(16))) uint16_t lds[SXN + SDN > RED * 4 * 512 ? SXN + SDN : RED * 4 * 512];
+    uint16_t *sx = lds, *sdy = lds + SXN;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int nl = lane & 15, kq = lane >> 4;
-    const int ky = blockIdx.y;
-    const int rows_total = a.n * a.H;
-    const int r0 = blockIdx.x * a.chunk_rows, r1 = min(rows_total, r0 + a.chunk_rows);
-    f4v acc[16];
+    const int ky0 = KYS == 1 ? 0 : blockIdx.y, c8g = blockIdx.z * BW;
+    const int seg = blockIdx.x % a.nseg, chunk = blockIdx.x / a.nseg;
+    const int img = chunk / a.hchunks, y0 = (chunk - img * a.hchunks) * a.chunk_rows;
+    const int y1 = min(y0 + a.chunk_rows, a.H), x0 = seg * kSegPx;
+    f4v acc[TAPS][NMT][NTB], accb[NMT];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) acc[q] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
-    float bsum = 0.0f;
-    // items (pixel, 8 channels) of a segment per thread
-    constexpr int ND = (kSegPx * (CO / 8) + 255) / 256, NX = ((kSegPx + 2) * (CI / 8) + 255) / 256;
+    for (int m = 0; m < NMT; ++m) {
+        accb[m] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int p = 0; p < TAPS; ++p)
+#pragma unroll
+            for (int t = 0; t < NTB; ++t) acc[p][m][t] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+    }
     u8v rd[ND], rx[NX];
-    const int nseg = (a.W + kSegPx - 1) / kSegPx;
-    // the segment's loads: zero outside the row (buffer range) and, by an
-    // empty range, for a row outside the image
-    auto fetch = [&](int r, int x0) {
-        const int img = r / a.H, y = r - img * a.H, yy = y + ky - 1;
-        const bool yin = yy >= 0 && yy < a.H;
-        const rsrc_t sd = row_rsrc(a.dy + (long long)r * a.W * CO, a.W * CO * 2);
-#pragma unroll
-        for (int k = 0; k < ND; ++k) {
-            const int e = (int)threadIdx.x + 256 * k, j = e / (CO / 8), c8 = e - j * (CO / 8);
-            rd[k] = __builtin_bit_cast(u8v, __builtin_amdgcn_raw_buffer_load_b128(sd, ((x0 + j) * CO + 8 * c8) * 2, 0, 0));
-        }
-        const long long xr = yin ? (long long)(img * a.H + yy) : 0;
-        if (!a.up) {
-            const rsrc_t sx_ = row_rsrc(a.x + xr * a.W * CI, yin ? a.W * CI * 2 : 0);
+    // zero outside the row (buffer range) and, by an empty range, for a row
+    // outside the image
+    auto fetch_x = [&](int yy) {
+        const bool in = yy >= 0 && yy < a.H;
+        const long long xr = in ? (long long)(img * a.H + yy) : 0;
+        constexpr int CU = CAT ? cat_up(CI) : 0, CS = CI - CU;
+        const rsrc_t s0 = row_rsrc(a.x + xr * a.W * CS, in ? a.W * CS * 2 : 0);
+        if (!CAT) {
 #pragma unroll
             for (int k = 0; k < NX; ++k) {
-                const int e = (int)threadIdx.x + 256 * k, jj = e / (CI / 8), c8 = e - jj * (CI / 8);
-                rx[k] = __builtin_bit_cast(
-                    u8v, __builtin_amdgcn_raw_buffer_load_b128(sx_, ((x0 + jj - 1) * CI + 8 * c8) * 2, 0, 0));
+                const int e = (int)threadIdx.x + 256 * k, jj = e / BW, c8 = c8g + e - jj * BW;
+                const int off = c8 < CI / 8 ? ((x0 + jj - 1) * CI + 8 * c8) * 2 : -16;
+                rx[k] = __builtin_bit_cast(u8v, __builtin_amdgcn_raw_buffer_load_b128(s0, off, 0, 0));
             }
         } else {   // up-sampled and skip channels, as in k_conv3x3: one of the two reads zero
-            constexpr int CU = cat_up(CI), CS = CI - CU > 0 ? CI - CU : 8;
-            const long long ur = yin ? (long long)(img * (a.H >> 1) + (yy >> 1)) : 0;
+            const long long ur = in ? (long long)(img * (a.H >> 1) + (yy >> 1)) : 0;
             const int wu = a.W >> 1;
-            const rsrc_t su = row_rsrc(a.up + ur * wu * CU, yin ? wu * CU * 2 : 0);
-            const rsrc_t ss = row_rsrc(a.x + xr * a.W * CS, yin ? a.W * CS * 2 : 0);
+            const rsrc_t su = row_rsrc(a.up + ur * wu * CU, in ? wu * CU * 2 : 0);
 #pragma unroll
             for (int k = 0; k < NX; ++k) {
-                const int e = (int)threadIdx.x + 256 * k, jj = e / (CI / 8), c8 = e - jj * (CI / 8);
-                const int px = x0 + jj - 1;
-                const bool up = c8 < CU / 8;
+                const int e = (int)threadIdx.x + 256 * k, jj = e / BW, c8 = c8g + e - jj * BW, px = x0 + jj - 1;
+                const bool up = c8 < CU / 8, skip = !up && c8 < CI / 8;
                 const u8v vu = __builtin_bit_cast(
                     u8v, __builtin_amdgcn_raw_buffer_load_b128(su, up ? ((px >> 1) * CU + 8 * c8) * 2 : -16, 0, 0));
                 const u8v vs = __builtin_bit_cast(
-                    u8v, __builtin_amdgcn_raw_buffer_load_b128(ss, up ? -16 : (px * CS + 8 * c8 - CU) * 2, 0, 0));
+                    u8v, __builtin_amdgcn_raw_buffer_load_b128(s0, skip ? (px * CS + 8 * c8 - CU) * 2 : -16, 0, 0));
                 rx[k] = vu | vs;
             }
         }
     };
-    fetch(r0, 0);
-    for (int r = r0; r < r1; ++r) {
-        for (int sg = 0; sg < nseg; ++sg) {
-            __syncthreads();   // the previous segment is consumed
-            // dY[y][x0 + j][8c .. 8c+7] -> sdy[8c + k][j]
+    auto fetch_d = [&](int y) {
+        const rsrc_t sd = row_rsrc(a.dy + (long long)(img * a.H + y) * a.W * CO, a.W * CO * 2);
 #pragma unroll
-            for (int n = 0; n < ND; ++n) {
-                const int e = (int)threadIdx.x + 256 * n, j = e / (CO / 8), c8 = e - j * (CO / 8);
-                if (e < kSegPx * (CO / 8))
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) sdy[(8 * c8 + k) * kSegPad + j] = rd[n][k];
-            }
-            // X[yy][x0 + jj - 1][8c .. 8c+7] -> sx[kx][8c + k][jj - kx]
-#pragma unroll
-            for (int n = 0; n < NX; ++n) {
-                const int e = (int)threadIdx.x + 256 * n, jj = e / (CI / 8), c8 = e - jj * (CI / 8);
-                if (e < (kSegPx + 2) * (CI / 8))
-#pragma unroll
-                    for (int kx = 0; kx < 3; ++kx) {
-                        const int j = jj - kx;
-                        if (j >= 0 && j < kSegPx)
-#pragma unroll
-                            for (int k = 0; k < 8; ++k) sx[(kx * CI + 8 * c8 + k) * kSegPad + j] = rx[n][k];
-                    }
-            }
-            __syncthreads();
-            // the next segment's loads go out before this one is multiplied
-            {
-                const bool wrap = sg + 1 == nseg;
-                const int rn = wrap ? min(r + 1, r1 - 1) : r;
-                fetch(rn, wrap ? 0 : (sg + 1) * kSegPx);
-            }
-            if (ky == 0 && (int)threadIdx.x < CO)
-#pragma unroll 8
-                for (int j = 0; j < kSegPx; ++j) bsum += u_bf2f(sdy[threadIdx.x * kSegPad + j]);
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int tile = wave + 4 * q;
-                if (tile < NTILES) {
-                    const int kx = tile / (NMT * NNT), rem = tile - kx * (NMT * NNT);
-                    const int mt = rem / NNT, nt = rem - mt * NNT;
-                    const uint16_t *pa = sdy + (mt * 16 + nl) * kSegPad + 8 * kq;
-                    const uint16_t *pb = sx + (kx * CI + nt * 16 + nl) * kSegPad + 8 * kq;
-#pragma unroll
-                    for (int s = 0; s < kSegPx; s += 32)
-                        acc[q] = mfma32(*(const u8v *)(pa + s), *(const u8v *)(pb + s), acc[q]);
-                }
-            }
+        for (int k = 0; k < ND; ++k) {
+            const int e = (int)threadIdx.x + 256 * k, j = e / (CO / 8), c8 = e - j * (CO / 8);
+            const int off = j < kSegPx ? ((x0 + j) * CO + 8 * c8) * 2 : -16;
+            rd[k] = __builtin_bit_cast(u8v, __builtin_amdgcn_raw_buffer_load_b128(sd, off, 0, 0));
         }
-    }
+    };
+    auto store_x = [&](int slot) {
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        const int tile = wave + 4 * q;
-        if (tile < NTILES) {
-            const int kx = tile / (NMT * NNT), rem = tile - kx * (NMT * NNT);
-            const int mt = rem / NNT, nt = rem - mt * NNT;
-            const int tap = 3 * ky + kx;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int co = mt * 16 + 4 * kq + j, ci = nt * 16 + nl;
-                a.part[(((long long)blockIdx.x * 9 + tap) * CO + co) * CI + ci] = acc[q][j];
-            }
+        for (int k = 0; k < NX; ++k) {
+            const int e = (int)threadIdx.x + 256 * k;
+            if (e < XP * BW) *(u8v *)(sx + slot * (XP * CW) + 8 * e) = rx[k];
         }
-    }
-    if (ky == 0 && (int)threadIdx.x < CO) a.bpart[(long long)blockIdx.x * CO + threadIdx.x] = bsum;
-}
-
-// out[e] = sum over c of part[c][e], c in increasing order: each thread
-// walks the chunks of one element (adjacent threads, adjacent elements)
-__global__ void k_reduce_chunks(int nchunks, long long len, const float *part, float *out)
-{
-    for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < len;
-         e += (long long)gridDim.x * blockDim.x) {
-        float s = 0.0f;
-        int c = 0;
-        // 32 partials are read before the first is added
-        for (; c + 32 <= nchunks; c += 32) {
-            float p[32];
+    };
+    auto store_d = [&]() {
 #pragma unroll
-            for (int k = 0; k < 32; ++k) p[k] = part[(long long)(c + k) * len + e];
-#pragma unroll
-            for (int k = 0; k < 32; ++k) s += p[k];
+        for (int k = 0; k < ND; ++k) {
+            const int e = (int)threadIdx.x + 256 * k;
+            if (e < kSegPx * (CO / 8)) *(u8v *)(sdy + 8 * e) = rd[k];
         }
-        for (; c < nchunks; ++c) s += part[(long long)c * len + e];
-        out[e] = s;
+    };
+    // the transposed read's lane: lanes 4 r + q of a quarter supply channels
+    // 4 q.. of pixel r, lane n receives channel n of pixels 0..3
+    const int tp = 32 * wave + 8 * kq + (nl >> 2), tc = 4 * (nl & 3);
+    if (KYS == 1) {
+        // rows y0 - 1 and y0; row yy lives in slot (yy + 3) % 3
+        fetch_x(y0 - 1);
+        store_x((y0 + 2) % 3);
+        fetch_x(y0);
+        store_x(y0 % 3);
     }
-}
-
-// The same sum for a short vector (the bias gradient): one workgroup per
-// element; thread t adds chunks t, t + 256, ... in order, then a fixed
-// pairwise tree over the threads
-__global__ __launch_bounds__(256) void k_reduce_chunks_short(int nchunks, int len, const float *part, float *out)
-{
-    __shared__ float sh[256];
-    const int e = blockIdx.x;
-    float s = 0.0f;
-    for (int c = threadIdx.x; c < nchunks; c += 256) s += part[(long long)c * len + e];
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int h = 128; h > 0; h >>= 1) {
-        if ((int)threadIdx.x < h) sh[threadIdx.x] += sh[threadIdx.x + h];
+    fetch_x(KYS == 1 ? y0 + 1 : y0 + ky0 - 1);
+    fetch_d(y0);
+    const u8v ones = u8v{0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80};
+    for (int y = y0; y < y1; ++y) {
+        __syncthreads();   // the row before is consumed
+        store_x(KYS == 1 ? (y + 1) % 3 : 0);
+        store_d();
         __syncthreads();
+        // the next row's loads go out before this one is multiplied
+        const int yn = min(y + 1, y1 - 1);
+        fetch_x(KYS == 1 ? yn + 1 : yn + ky0 - 1);
+        fetch_d(yn);
+        u8v av[NMT];
+#pragma unroll
+        for (int m = 0; m < NMT; ++m) {
+            av[m] = tr_read(sdy + tp * CO + 16 * m + tc, CO);
+            if (ky0 == 0 && blockIdx.z == 0) accb[m] = mfma32(av[m], ones, accb[m]);
+        }
+#pragma unroll
+        for (int p = 0; p < TAPS; ++p) {
+            const int kx = p % 3, slot = KYS == 1 ? (y + p / 3 + 2) % 3 : 0;   // row y + ky - 1
+            const uint16_t *bx = sx + slot * (XP * CW) + (tp + kx) * CW + tc;
+#pragma unroll
+            for (int t = 0; t < NTB; ++t) {
+                const u8v bv = tr_read(bx + 16 * t, CW);
+#pragma unroll
+                for (int m = 0; m < NMT; ++m) acc[p][m][t] = mfma32(av[m], bv, acc[p][m][t]);
+            }
+        }
     }
-    if (threadIdx.x == 0) out[e] = sh[0];
+    // sums over the waves, RED tiles per turn; element (lane, j) of a tile is
+    // co = 16 m + 4 (lane / 16) + j, ci = lane % 16
+    float *red = (float *)lds;
+    auto turn = [&](int tile0, int nt, auto get, auto put) {
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < RED; ++q)
+            if (q < nt) *(f4v *)(red + ((q * 4 + wave) * 64 + lane) * 4) = get(tile0 + q);
+        __syncthreads();
+        const int e = threadIdx.x;
+#pragma unroll
+        for (int q = 0; q < RED; ++q)
+            if (q < nt) {
+                const float *r = red + q * 1024 + e;
+                put(tile0 + q, ((r[0] + r[256]) + r[512]) + r[768]);
+            }
+    };
+    const int el = threadIdx.x >> 2, ej = threadIdx.x & 3;
+    float *part = a.part + (long long)blockIdx.x * 9 * CO * CI;
+#pragma unroll
+    for (int t0 = 0; t0 < NTILE; t0 += RED)
+        turn(t0, NTILE - t0 < RED ? NTILE - t0 : RED,
+             [&](int q) { return acc[q / (NMT * NTB)][q / NTB % NMT][q % NTB]; },
+             [&](int q, float v) {
+                 const int p = q / (NMT * NTB), m = q / NTB % NMT, t = q % NTB;
+                 const int tap = KYS == 1 ? p : 3 * ky0 + p;
+                 const int co = 16 * m + 4 * (el >> 4) + ej, ci = 8 * c8g + 16 * t + (el & 15);
+                 if (NNT % NTB == 0 || ci < CI) part[((long long)tap * CO + co) * CI + ci] = v;
+             });
+    if (ky0 == 0 && blockIdx.z == 0)
+        turn(0, NMT, [&](int q) { return accb[q < NMT ? q : 0]; },
+             [&](int q, float v) {
+                 if ((el & 15) == 0) a.bpart[(long long)blockIdx.x * CO + 16 * q + 4 * (el >> 4) + ej] = v;
+             });
 }
 
-int wgrad_chunk_rows(int n, int H)
+// dw[e] = sum over c of part[c][e] and, behind them, db[e] from bpart: four
+// waves take a quarter of the partials each, in order, for 64 elements, and
+// the quarters are added in order (one wave over all of 512 partials and a
+// launch of its own for db: 10.4 + 4.7 us per layer, now 9.3)
+__global__ __launch_bounds__(256) void k_reduce_chunks(int nchunks, int len, const float *part, float *dw, int blen,
+                                                       const float *bpart, float *db)
 {
-    return std::max(1, (n * H + 255) / 256);
+    __shared__ float sh[4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int nb = (len + 63) / 64;
+    const bool bias = (int)blockIdx.x >= nb;
+    const int n = bias ? blen : len, e = ((int)blockIdx.x - (bias ? nb : 0)) * 64 + lane;
+    const float *src = (bias ? bpart : part) + min(e, n - 1);
+    const int c0 = (int)((long long)nchunks * wave / 4), c1 = (int)((long long)nchunks * (wave + 1) / 4);
+    float s = 0.0f;
+    int c = c0;
+    for (; c + 32 <= c1; c += 32) {   // 32 are read before the first is added
+        float p[32];
+#pragma unroll
+        for (int k = 0; k < 32; ++k) p[k] = src[(long long)(c + k) * n];
+#pragma unroll
+        for (int k = 0; k < 32; ++k) s += p[k];
+    }
+    for (; c < c1; ++c) s += src[(long long)c * n];
+    sh[wave][lane] = s;
+    __syncthreads();
+    if (wave == 0 && e < n) (bias ? db : dw)[e] = ((sh[0][lane] + sh[1][lane]) + sh[2][lane]) + sh[3][lane];
 }
 
-int wgrad_chunks(int n, int H)
+// the layers' (input, output) channel pairs: taps per workgroup and input
+// channel tiles per workgroup, as the accumulators allow
+static bool wgrad_all_taps(int Ci, int Co) { return Ci * Co <= 1024; }
+
+// column segments and row chunks: about 512 workgroups of partials (256 where
+// blockIdx.y triples them), a chunk within one image
+static void wgrad_split(int n, int H, int W, int Ci, int Co, int &nseg, int &hchunks, int &rows)
 {
-    const int cr = wgrad_chunk_rows(n, H);
-    return (n * H + cr - 1) / cr;
+    nseg = (W + kSegPx - 1) / kSegPx;
+    const int want = std::max(1, (wgrad_all_taps(Ci, Co) ? 512 : 256) / (nseg * n));
+    rows = std::max(1, (H + want - 1) / want);
+    hchunks = (H + rows - 1) / rows;
 }
 
-template <int CI, int CO> static void wgrad_launch(const WgradArgs &a, int nch, hipStream_t st)
+int wgrad_chunks(int n, int H, int W, int Ci, int Co)
 {
-    hipLaunchKernelGGL((k_wgrad<CI, CO>), dim3(nch, 3), dim3(256), 0, st, a);
+    int nseg, hchunks, rows;
+    wgrad_split(n, H, W, Ci, Co, nseg, hchunks, rows);
+    return n * nseg * hchunks;
 }
 
-hipError_t launch_wgrad(const WgradArgs &a, float *dw, float *db, hipStream_t st)
+template <int CI, int CO, int KYS, int NTB> static void wgrad_launch(const WgradArgs &a, int nch, hipStream_t st)
 {
-    if (a.chunk_rows != wgrad_chunk_rows(a.n, a.H) || a.n < 1 || a.H < 1 || a.W < 1) return hipErrorInvalidValue;
-    const int nch = wgrad_chunks(a.n, a.H);
-    const int key = a.Ci * 1000 + a.Co;
-    switch (key) {   // the (input, output) channel pairs of the network's layers
-    case 16016: wgrad_launch<16, 16>(a, nch, st); break;
-    case 16032: wgrad_launch<16, 32>(a, nch, st); break;
-    case 32032: wgrad_launch<32, 32>(a, nch, st); break;
-    case 32048: wgrad_launch<32, 48>(a, nch, st); break;
-    case 48048: wgrad_launch<48, 48>(a, nch, st); break;
-    case 48064: wgrad_launch<48, 64>(a, nch, st); break;
-    case 64064: wgrad_launch<64, 64>(a, nch, st); break;
-    case 112048: wgrad_launch<112, 48>(a, nch, st); break;
-    case 80032: wgrad_launch<80, 32>(a, nch, st); break;
-    case 48016: wgrad_launch<48, 16>(a, nch, st); break;
+    constexpr int Z = (CI / 16 + NTB - 1) / NTB;
+    static_assert((KYS == 1) == (CI * CO <= 1024), "as wgrad_all_taps");
+    hipLaunchKernelGGL((k_wgrad<CI, CO, KYS, NTB>), dim3(nch, KYS, Z), dim3(256), 0, st, a);
+}
+
+hipError_t launch_wgrad(WgradArgs a, float *dw, float *db, hipStream_t st)
+{
+    if (a.n < 1 || a.H < 1 || a.W < 1 || (a.up && ((a.H | a.W) & 1))) return hipErrorInvalidValue;
+    wgrad_split(a.n, a.H, a.W, a.Ci, a.Co, a.nseg, a.hchunks, a.chunk_rows);
+    const int nch = wgrad_chunks(a.n, a.H, a.W, a.Ci, a.Co);
+    switch ((a.up ? 1000000 : 0) + a.Ci * 1000 + a.Co) {   // the network's layers
+    case 16016: wgrad_launch<16, 16, 1, 1>(a, nch, st); break;
+    case 16032: wgrad_launch<16, 32, 1, 1>(a, nch, st); break;
+    case 32032: wgrad_launch<32, 32, 1, 2>(a, nch, st); break;
+    case 32048: wgrad_launch<32, 48, 3, 2>(a, nch, st); break;
+    case 48048: wgrad_launch<48, 48, 3, 3>(a, nch, st); break;
+    case 48064: wgrad_launch<48, 64, 3, 3>(a, nch, st); break;
+    case 64064: wgrad_launch<64, 64, 3, 2>(a, nch, st); break;
+    case 1112048: wgrad_launch<112, 48, 3, 4>(a, nch, st); break;
+    case 1080032: wgrad_launch<80, 32, 3, 5>(a, nch, st); break;
+    case 1048016: wgrad_launch<48, 16, 1, 3>(a, nch, st); break;
     default: return hipErrorInvalidValue;
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const long long len = 9LL * a.Co * a.Ci;
-    hipLaunchKernelGGL(k_reduce_chunks, dim3((unsigned)std::min<long long>(1024, (len + 255) / 256)), dim3(256), 0, st,
-                       nch, len, a.part, dw);
-    e = hipGetLastError();
-    if (e != hipSuccess || !db) return e;
-    hipLaunchKernelGGL(k_reduce_chunks_short, dim3(a.Co), dim3(256), 0, st, nch, a.Co, a.bpart, db);
+    const int len = 9 * a.Co * a.Ci;
+    hipLaunchKernelGGL(k_reduce_chunks, dim3((unsigned)((len + 63) / 64 + (a.Co + 63) / 64)), dim3(256), 0, st, nch, len,
+                       a.part, dw, a.Co, a.bpart, db);
     return hipGetLastError();
 }
 
