@@ -15,9 +15,14 @@
 // fixed order; the reference accumulates Ebar in float.
 //
 // FFT: radix-2 decimation in time, a bit-reversal gather then log2(Npad)
-// butterfly passes over all traces at once, complex double in HBM.
+// butterfly stages over all traces at once, complex double.  The stages run
+// in LDS, eight in the pass that gathers the traces and up to seven in each
+// pass after it: two passes over HBM instead of one per stage for 2^15
+// points, with the same butterflies.  240 traces of 5000 samples (Npad 2^15):
+// 32 launches of 20-38 us for the two transforms before, now four of about 75.
 #include "dn_core.h"
 
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -31,43 +36,94 @@ struct cd {
 
 __device__ inline cd cmul(cd a, cd b) { return cd{a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re}; }
 
-// x [ntr][ns] float (row stride ld) -> X [ntr][N] complex, bit-reversed
-// order, zero padding beyond ns; mute[i] != 0 gives a zero trace; samples
-// 2..ns are divided by scale[i] (mul = 0) or multiplied by it (mul = 1),
-// sample 1 is kept (util.c:502-520, 545-571)
-__global__ void k_fft_load(int ntr, int ns, int ld, int N, int logN, const float *__restrict__ x,
-                           const unsigned char *__restrict__ mute, const float *__restrict__ scale, int mul,
-                           cd *__restrict__ X)
+// w[k] = exp(i pi k / (N / 2)), k < N / 2: the twiddles of every stage
+__global__ void k_twiddles(int N, cd *__restrict__ w)
 {
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long long)ntr * N) return;
-    const int i = (int)(t / N), j = (int)(t % N);
-    const unsigned r = __builtin_bitreverse32((unsigned)j) >> (32 - logN);
-    double v = 0.0;
-    if (j < ns && !(mute && mute[i])) {
-        float f = x[(long long)i * ld + j];
-        if (scale && j >= 1) f = mul ? f * scale[i] : f / scale[i];
-        v = (double)f;
-    }
-    X[(long long)i * N + r] = cd{v, 0.0};
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= N / 2) return;
+    double sn, cs;
+    sincospi((double)k / (double)(N / 2), &sn, &cs);
+    w[k] = cd{cs, sn};
 }
 
-// one butterfly pass of half-length h for every trace; sign +1 or -1
-__global__ void k_fft_pass(int ntr, int N, int h, int sign, cd *__restrict__ X)
+constexpr int kFirstBits = 8, kNextBits = 7;
+constexpr int kFirstPts = 512, kNextPts = 1024;   // points of a workgroup of 256 threads
+
+__device__ inline void butterfly(cd &a, cd &b, cd w, int sign)
 {
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int nb = N / 2;
-    if (t >= (long long)ntr * nb) return;
-    const int i = (int)(t / nb), b = (int)(t % nb);
-    const int grp = b / h, pos = b % h;
-    const int i0 = grp * 2 * h + pos, i1 = i0 + h;
-    double sn, cs;
-    sincospi((double)pos / (double)h, &sn, &cs);   // angle pi pos / h = 2 pi pos / (2h)
-    const cd w{cs, sign * sn};
-    cd *row = X + (long long)i * N;
-    const cd a = row[i0], b1 = cmul(row[i1], w);
-    row[i0] = cd{a.re + b1.re, a.im + b1.im};
-    row[i1] = cd{a.re - b1.re, a.im - b1.im};
+    const cd b1 = cmul(b, cd{w.re, sign * w.im}), a0 = a;
+    a = cd{a0.re + b1.re, a0.im + b1.im};
+    b = cd{a0.re - b1.re, a0.im - b1.im};
+}
+
+// x [ntr][ns] float (row stride ld) -> X [ntr][N] complex after the first
+// `bits` stages (sign +1): gathered in bit-reversed order, zero padding beyond
+// ns; mute[i] != 0 gives a zero trace; samples 2..ns are divided by scale[i]
+// (mul = 0) or multiplied by it (mul = 1), sample 1 is kept (util.c:502-520,
+// 545-571).  With src the points come from there, already in that order
+// (then sign applies).  A workgroup takes kFirstPts consecutive points.
+__global__ __launch_bounds__(256) void k_fft_first(int ntr, int ns, int ld, int logN, int bits,
+                                                   const float *__restrict__ x, const unsigned char *__restrict__ mute,
+                                                   const float *__restrict__ scale, int mul, const cd *src, int sign,
+                                                   const cd *__restrict__ tw, cd *X)
+{
+    __shared__ cd p[kFirstPts];
+    const long long total = (long long)ntr << logN, g0 = (long long)blockIdx.x * kFirstPts;
+#pragma unroll
+    for (int k = 0; k < kFirstPts / 256; ++k) {
+        const long long g = g0 + threadIdx.x + 256 * k;
+        cd v{0.0, 0.0};
+        if (g < total) {
+            if (src) {
+                v = src[g];
+            } else {
+                const int i = (int)(g >> logN);
+                const unsigned r = (unsigned)(g & ((1LL << logN) - 1));
+                const int j = (int)(__builtin_bitreverse32(r) >> (32 - logN));
+                if (j < ns && !(mute && mute[i])) {
+                    float f = x[(long long)i * ld + j];
+                    if (scale && j >= 1) f = mul ? f * scale[i] : f / scale[i];
+                    v.re = (double)f;
+                }
+            }
+        }
+        p[threadIdx.x + 256 * k] = v;
+    }
+    for (int q = 0; q < bits; ++q) {
+        __syncthreads();
+        const int b = threadIdx.x, pos = b & ((1 << q) - 1), i0 = ((b >> q) << (q + 1)) + pos;
+        butterfly(p[i0], p[i0 + (1 << q)], tw[(size_t)pos << (logN - 1 - q)], sign);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kFirstPts / 256; ++k) {
+        const long long g = g0 + threadIdx.x + 256 * k;
+        if (g < total) X[g] = p[threadIdx.x + 256 * k];
+    }
+}
+
+// stages s0 .. s0 + bits - 1 in place: a workgroup takes, of one span of
+// 2^(s0 + bits) points, the 2^bits points 2^s0 apart of C consecutive columns
+__global__ __launch_bounds__(256) void k_fft_next(int logN, int s0, int bits, int logC, int sign,
+                                                  const cd *__restrict__ tw, cd *__restrict__ X)
+{
+    __shared__ cd p[kNextPts];
+    const int C = 1 << logC, pts = 1 << (bits + logC);
+    const long long wg = blockIdx.x;
+    const int lo0 = (int)(wg & ((1LL << (s0 - logC)) - 1)) << logC;
+    cd *base = X + ((wg >> (s0 - logC)) << (s0 + bits)) + lo0;
+    for (int e = threadIdx.x; e < pts; e += 256) p[e] = base[((size_t)(e >> logC) << s0) + (e & (C - 1))];
+    for (int q = 0; q < bits; ++q) {
+        __syncthreads();
+        for (int b = threadIdx.x; b < pts / 2; b += 256) {
+            const int c = b & (C - 1), kb = b >> logC;               // butterfly kb of column c
+            const int pos = kb & ((1 << q) - 1), k0 = ((kb >> q) << (q + 1)) + pos;
+            const size_t ang = ((size_t)pos << s0) + lo0 + c;        // of 2^(s0 + q)
+            butterfly(p[(k0 << logC) + c], p[((k0 + (1 << q)) << logC) + c], tw[ang << (logN - 1 - s0 - q)], sign);
+        }
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < pts; e += 256) base[((size_t)(e >> logC) << s0) + (e & (C - 1))] = p[e];
 }
 
 // per-trace scales of NORMALIZE 1 / 2 (max |x| over samples 2..ns, 0 -> 1)
@@ -115,15 +171,26 @@ __global__ void k_wiener_sums(int ntr, int N, const cd *__restrict__ D, const cd
     const double n = (double)ntr;
     cd a{0.0, 0.0};
     double d = 0.0, e = 0.0;
-    for (int i = 0; i < ntr; ++i) {
-        const cd dd = D[(long long)i * N + k], mm = M[(long long)i * N + k];
+    auto add = [&](const cd &dd, const cd &mm) {
         const cd nd{n * dd.re, n * dd.im}, nm{n * mm.re, n * mm.im};
         const cd p = cmul(nd, cd{mm.re, -mm.im});
         a.re += p.re;
         a.im += p.im;
         d += nm.re * mm.re + nm.im * mm.im;
         e += d;
+    };
+    int i = 0;
+    for (; i + 8 <= ntr; i += 8) {   // eight traces are read before the first is added
+        cd dd[8], mm[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            dd[q] = D[(long long)(i + q) * N + k];
+            mm[q] = M[(long long)(i + q) * N + k];
+        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) add(dd[q], mm[q]);
     }
+    for (; i < ntr; ++i) add(D[(long long)i * N + k], M[(long long)i * N + k]);
     sn[k] = a;
     sd[k] = d;
     erow[k] = e;
@@ -134,7 +201,15 @@ __global__ void k_sum_fixed(int N, const double *__restrict__ v, double *__restr
 {
     __shared__ double sm[256];
     double a = 0.0;
-    for (int k = threadIdx.x; k < N; k += blockDim.x) a += v[k];
+    int k = threadIdx.x;
+    for (; k + 15 * 256 < N; k += 16 * 256) {
+        double x[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) x[q] = v[k + 256 * q];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) a += x[q];
+    }
+    for (; k < N; k += 256) a += v[k];
     sm[threadIdx.x] = a;
     __syncthreads();
     for (int o = blockDim.x / 2; o > 0; o >>= 1) {
@@ -171,17 +246,43 @@ __global__ void k_stf_out(int ns, int N, const cd *__restrict__ x, float *__rest
 
 unsigned blocks(long long n, int b = 256) { return (unsigned)((n + b - 1) / b); }
 
+// device buffers of one call, cut from one allocation
 struct StfDev {
     hipStream_t st = nullptr;
+    char *mem = nullptr;
+    size_t used = 0;
     float *obs = nullptr, *syn = nullptr, *sig = nullptr, *stf = nullptr, *mx = nullptr;
     unsigned char *mute = nullptr;
-    cd *D = nullptr, *M = nullptr, *S = nullptr, *sn = nullptr, *Y = nullptr;
+    cd *D = nullptr, *M = nullptr, *S = nullptr, *sn = nullptr, *Y = nullptr, *tw = nullptr;
     double *sd = nullptr, *erow = nullptr, *esum = nullptr;
+    // sizes first (mem null: only `used` grows), then pointers
+    template <typename T> void take(T *&p, size_t n)
+    {
+        if (mem) p = (T *)(mem + used);
+        used += (n * sizeof(T) + 255) / 256 * 256;
+    }
+    void layout(size_t ntr, size_t ns, size_t N)
+    {
+        used = 0;
+        take(obs, ntr * ns);
+        take(syn, ntr * ns);
+        take(sig, ns);
+        take(stf, ns);
+        take(mx, 4 * ntr);
+        take(mute, ntr);
+        take(D, ntr * N);
+        take(M, ntr * N);
+        take(S, N);
+        take(sn, N);
+        take(Y, N);
+        take(tw, N / 2);
+        take(sd, N);
+        take(erow, N);
+        take(esum, 2);
+    }
     void release()
     {
-        void *ps[] = {obs, syn, sig, stf, mx, mute, D, M, S, sn, Y, sd, erow, esum};
-        for (void *p : ps)
-            if (p) (void)hipFree(p);
+        if (mem) (void)hipFree(mem);
         if (st) (void)hipStreamDestroy(st);
         *this = StfDev{};
     }
@@ -196,10 +297,25 @@ struct StfDev {
         }                                                                                        \
     } while (0)
 
-void fft(cd *X, int ntr, int N, int logN, int sign, hipStream_t st)
+// the stages after the first pass, of ntr transforms
+void fft_rest(cd *X, int ntr, int logN, int sign, const cd *tw, hipStream_t st)
 {
-    for (int h = 1; h < N; h *= 2)
-        hipLaunchKernelGGL(k_fft_pass, dim3(blocks((long long)ntr * (N / 2))), dim3(256), 0, st, ntr, N, h, sign, X);
+    for (int s0 = kFirstBits; s0 < logN;) {
+        const int bits = std::min(kNextBits, logN - s0);
+        const int logC = std::min(s0, 10 - bits);   // kNextPts points
+        const long long wgs = (long long)ntr << (logN - bits - logC);
+        hipLaunchKernelGGL(k_fft_next, dim3((unsigned)wgs), dim3(256), 0, st, logN, s0, bits, logC, sign, tw, X);
+        s0 += bits;
+    }
+}
+
+// transforms of ntr float traces (sign +1)
+void fft_traces(int ntr, int ns, int logN, const float *x, const unsigned char *mute, const float *scale, int mul,
+                const cd *tw, cd *X, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_fft_first, dim3(blocks((long long)ntr << logN, kFirstPts)), dim3(256), 0, st, ntr, ns, ns, logN,
+                       std::min(kFirstBits, logN), x, mute, scale, mul, (const cd *)nullptr, 1, tw, X);
+    fft_rest(X, ntr, logN, 1, tw, st);
 }
 
 }  // namespace
@@ -216,20 +332,9 @@ extern "C" int dn_stf(int ntr, int ns, const float *obs, const float *syn, const
     StfDev R;
     SCHK(hipStreamCreateWithFlags(&R.st, hipStreamNonBlocking));
     const size_t nd = (size_t)ntr * ns;
-    SCHK(hipMalloc((void **)&R.obs, nd * sizeof(float)));
-    SCHK(hipMalloc((void **)&R.syn, nd * sizeof(float)));
-    SCHK(hipMalloc((void **)&R.sig, (size_t)ns * sizeof(float)));
-    SCHK(hipMalloc((void **)&R.stf, (size_t)ns * sizeof(float)));
-    SCHK(hipMalloc((void **)&R.mx, (size_t)4 * ntr * sizeof(float)));
-    SCHK(hipMalloc((void **)&R.mute, (size_t)ntr));
-    SCHK(hipMalloc((void **)&R.D, (size_t)ntr * N * sizeof(cd)));
-    SCHK(hipMalloc((void **)&R.M, (size_t)ntr * N * sizeof(cd)));
-    SCHK(hipMalloc((void **)&R.S, (size_t)N * sizeof(cd)));
-    SCHK(hipMalloc((void **)&R.sn, (size_t)N * sizeof(cd)));
-    SCHK(hipMalloc((void **)&R.Y, (size_t)N * sizeof(cd)));
-    SCHK(hipMalloc((void **)&R.sd, (size_t)N * sizeof(double)));
-    SCHK(hipMalloc((void **)&R.erow, (size_t)N * sizeof(double)));
-    SCHK(hipMalloc((void **)&R.esum, 2 * sizeof(double)));
+    R.layout(ntr, ns, N);
+    SCHK(hipMalloc((void **)&R.mem, R.used));
+    R.layout(ntr, ns, N);
     hipStream_t st = R.st;
     SCHK(hipMemcpyAsync(R.obs, obs, nd * sizeof(float), hipMemcpyHostToDevice, st));
     SCHK(hipMemcpyAsync(R.syn, syn, nd * sizeof(float), hipMemcpyHostToDevice, st));
@@ -254,20 +359,18 @@ extern "C" int dn_stf(int ntr, int ns, const float *obs, const float *syn, const
             mul_obs = 1;
         }
     }
-    hipLaunchKernelGGL(k_fft_load, dim3(blocks((long long)ntr * N)), dim3(256), 0, st, ntr, ns, ns, N, logN, R.obs,
-                       R.mute, sc_obs, mul_obs, R.D);
-    hipLaunchKernelGGL(k_fft_load, dim3(blocks((long long)ntr * N)), dim3(256), 0, st, ntr, ns, ns, N, logN, R.syn,
-                       R.mute, sc_syn, 0, R.M);
-    hipLaunchKernelGGL(k_fft_load, dim3(blocks(N)), dim3(256), 0, st, 1, ns, ns, N, logN, R.sig,
-                       (const unsigned char *)nullptr, (const float *)nullptr, 0, R.S);
-    fft(R.D, ntr, N, logN, +1, st);
-    fft(R.M, ntr, N, logN, +1, st);
-    fft(R.S, 1, N, logN, +1, st);
+    hipLaunchKernelGGL(k_twiddles, dim3(blocks(N / 2)), dim3(256), 0, st, N, R.tw);
+    fft_traces(ntr, ns, logN, R.obs, R.mute, sc_obs, mul_obs, R.tw, R.D, st);
+    fft_traces(ntr, ns, logN, R.syn, R.mute, sc_syn, 0, R.tw, R.M, st);
+    fft_traces(1, ns, logN, R.sig, nullptr, nullptr, 0, R.tw, R.S, st);
     hipLaunchKernelGGL(k_wiener_sums, dim3(blocks(N)), dim3(256), 0, st, ntr, N, R.D, R.M, R.sn, R.sd, R.erow);
     hipLaunchKernelGGL(k_sum_fixed, dim3(1), dim3(256), 0, st, N, R.erow, R.esum);
     hipLaunchKernelGGL(k_eps, dim3(1), dim3(1), 0, st, R.esum, N, ntr, o->eps_stf, R.esum + 1);
     hipLaunchKernelGGL(k_wiener_div, dim3(blocks(N)), dim3(256), 0, st, N, logN, R.S, R.sn, R.sd, R.esum + 1, R.Y);
-    fft(R.Y, 1, N, logN, -1, st);
+    hipLaunchKernelGGL(k_fft_first, dim3(blocks(N, kFirstPts)), dim3(256), 0, st, 1, ns, ns, logN,
+                       std::min(kFirstBits, logN), (const float *)nullptr, (const unsigned char *)nullptr,
+                       (const float *)nullptr, 0, R.Y, -1, R.tw, R.Y);
+    fft_rest(R.Y, 1, logN, -1, R.tw, st);
     hipLaunchKernelGGL(k_stf_out, dim3(blocks(ns)), dim3(256), 0, st, ns, N, R.Y, R.stf);
     SCHK(hipGetLastError());
     SCHK(hipMemcpyAsync(stf, R.stf, (size_t)ns * sizeof(float), hipMemcpyDeviceToHost, st));

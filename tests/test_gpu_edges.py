@@ -66,3 +66,20 @@ def test_gauss_out_of_range_is_refused():
     vel[7, 33] = 1e6
     with pytest.raises(dn.DeniseError):
         dn.gauss_filt_var(np.ones((20, 70), np.float32), vel, 0.25, 0.3, 0.3, 25.0)
+
+
+@pytest.mark.parametrize("ntr,ns", [(1, 2), (3, 3), (5, 64), (9, 65), (16, 130), (17, 300), (2, 5000), (7, 9000), (1, 40000)])
+def test_stf_passes(ntr, ns):
+    """Transform lengths 2^3 to 2^18: one, two and three passes, the last of
+    one to seven stages; trace counts around the eight read ahead.  The bound
+    is the float rounding of the regulariser and the output, as for the
+    record lengths of the other STF tests."""
+    import stf_oracle
+    say("stf", ntr, ns)
+    rng = np.random.default_rng(ns)
+    syn = rng.standard_normal((ntr, ns)).astype(np.float32)
+    obs = (0.7 * syn + 0.3 * rng.standard_normal((ntr, ns))).astype(np.float32)
+    sig = rng.standard_normal(ns).astype(np.float32)
+    got = product().stf(obs, syn, sig, eps_stf=0.05)
+    want = stf_oracle.stf(obs, syn, sig, eps_stf=0.05)
+    assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
