@@ -30,6 +30,7 @@ DEVICE = ["--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-pa
 # half-order, so that the objects build in parallel
 SOURCES = [("dn_tile.hip", ["-DDN_TILE_K=%d" % k], "dn_tile_k%d" % k) for k in (4, 6, 5, 3, 2, 1)] + [
     ("dn_kernels.hip", []),
+    ("dn_multi.hip", []),
     ("dn_core.cpp", []),
     ("dn_setup.cpp", []),
     ("dn_dropin.cpp", []),

@@ -13,6 +13,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <numeric>
 #include <string>
 #include <thread>
 #include <vector>
@@ -207,7 +208,7 @@ static void free_batch(dn_ctx *c)
         dfree_t(c->d_psx[k]);
         dfree_t(c->d_psy[k]);
     }
-    dfree_t(c->d_rq); dfree_t(c->d_pvx); dfree_t(c->d_pvy);
+    dfree_t(c->d_rq); dfree_t(c->d_pvx); dfree_t(c->d_pvy); dfree_t(c->d_pvx2); dfree_t(c->d_pvy2);
     dfree_t(c->d_seis); dfree_t(c->d_resid); dfree_t(c->d_snap); dfree_t(c->d_snap16); dfree_t(c->d_snap_scale);
     dfree_t(c->d_stage); dfree_t(c->d_stage_max);
     dfree_t(c->d_Ws); dfree_t(c->d_Wr); dfree_t(c->d_gu_shot); dfree_t(c->d_grho_shot); dfree_t(c->d_part);
@@ -704,6 +705,9 @@ extern "C" int dn_autotune(dn_ctx *c, int nshots, int nsteps, int *rows_out, int
     return 0;
 }
 
+// grids that dn_multi.hip can step
+static bool multi_capable(const dn_ctx *c) { return c->p.L == 0 && c->K <= 2; }
+
 int dn_nsnap(const dn_ctx *c) { return (c->nt_max + c->p.dtinv - 1) / c->p.dtinv; }
 
 // bytes of per-shot device state for a gradient batch
@@ -712,7 +716,7 @@ static size_t per_shot_bytes(const dn_ctx *c, bool gradient)
     const Geo &g = c->g;
     const size_t P = (size_t)g.plane, nxny = (size_t)g.nx * g.ny;
     size_t b = 6 * P * 4 + 2 * (size_t)g.L * P * 4;                 // vy,sxy,syz x2, r, q
-    b += (size_t)(2 * 2 + 2) * (size_t)(2 * g.fw) * (g.nx + g.ny) * 4;  // psi
+    b += (size_t)(2 * 2 + 2) * (size_t)(2 * g.fw) * (g.nx + g.ny) * 4;  // psi, at least as many as there are
     b += 2 * (size_t)c->ntr * c->nt_max * 4;                        // seis + resid
     b += 4 * nxny * 4 + (size_t)c->ntr * 16;                        // Ws, Wr, gu, grho, partials
     if (gradient) {
@@ -758,6 +762,10 @@ int dn_ensure_batch(dn_ctx *c, int want, bool gradient)
     HIPCHK(c, dalloc(&c->d_rq, S * P * 2 * std::max(1, g.L)));
     HIPCHK(c, dalloc(&c->d_pvx, S * fw2 * g.ny));
     HIPCHK(c, dalloc(&c->d_pvy, S * fw2 * g.nx));
+    if (multi_capable(c)) {
+        HIPCHK(c, dalloc(&c->d_pvx2, S * fw2 * g.ny));
+        HIPCHK(c, dalloc(&c->d_pvy2, S * fw2 * g.nx));
+    }
     HIPCHK(c, dalloc(&c->d_seis, S * c->ntr * c->nt_max));
     HIPCHK(c, dalloc(&c->d_resid, S * c->ntr * c->nt_max));
     HIPCHK(c, dalloc(&c->d_Ws, S * nxny));
@@ -849,6 +857,23 @@ static int choose_tile(const dn_ctx *c, int nshots)
     return tiles16 <= 256 ? 1 : 2;
 }
 
+// Several steps per launch (dn_multi.hip)?  Where nothing needs another launch
+// between two steps (FP16 snapshots are packed after each stored step, BF16
+// ones scaled by the snapshot before) and the recomputed cells do not cost
+// more than the launches.  Microseconds per step, tiles / several steps, by
+// workgroups of 24 x 8 cells, forward and gradient: FDORDER 4: 255 (400x120)
+// 5.5 / 2.5, 6.6 / 3.2; 510 5.7 / 3.3, 6.9 / 5.0; 750 (700x200) 5.8 / 4.5,
+// 7.3 / 6.7; 850 6.1 / 5.1, 7.7 / 8.1; 1020 6.5 / 5.2, 8.1 / 8.3.  FDORDER 2:
+// 1292 (800x300) 6.3 / 3.4, 7.9 / 5.4; 2100 8.0 / 5.0, 9.9 / 8.1; 2584
+// 8.2 / 6.0, 10.0 / 9.2.
+static bool choose_multi(const dn_ctx *c, int nshots, bool adjoint, bool store, bool hess)
+{
+    if (!multi_capable(c) || choose_tile(c, nshots) == 0) return false;
+    if ((adjoint || store) && c->p.snap_precision != 0) return false;
+    const int limit = c->K == 1 ? 2048 : (adjoint || store || hess ? 768 : 1024);
+    return (long long)nshots * multi_tiles(c->g.nx, c->g.ny) <= limit;
+}
+
 void dn_fill_step_common(dn_ctx *c, StepArgs &a, int n)
 {
     const Geo &g = c->g;
@@ -930,6 +955,10 @@ int dn_zero_state(dn_ctx *c, int n)
     }
     HIPCHK(c, launch_fill(c->d_pvx, S * fw2 * g.ny, 0.0f, c->stream));
     HIPCHK(c, launch_fill(c->d_pvy, S * fw2 * g.nx, 0.0f, c->stream));
+    if (c->d_pvx2) {
+        HIPCHK(c, launch_fill(c->d_pvx2, S * fw2 * g.ny, 0.0f, c->stream));
+        HIPCHK(c, launch_fill(c->d_pvy2, S * fw2 * g.nx, 0.0f, c->stream));
+    }
     return 0;
 }
 
@@ -940,7 +969,15 @@ static int enqueue_steps(dn_ctx *c, StepArgs &a, int n, bool adjoint, bool pack_
                          const int *nt_base, int &cur, const std::vector<char> &corr_res, bool fwd_extra)
 {
     const int kind = c->p.snap_precision;
-    for (int k = 0; k < count; ++k) {
+    // does some shot of the launch store, sum or correlate at step nt
+    // (adjoint: shot s correlates at step nt when nt = NT_s (mod dtinv));
+    // inside a chunk the counter is a multiple of dtinv
+    const int dt = c->p.dtinv;
+    auto extra_at = [&](int nt) -> bool {
+        return adjoint ? corr_res[((nt % dt) + dt) % dt] != 0 : (fwd_extra && ((nt - 1) % dt) == 0);
+    };
+    const int per = a.ms_steps > 0 ? multi_steps(c->K) : 1;   // steps per launch
+    for (int k = 0; k < count; k += per) {
         const int nt = nt0 + k;
         a.nt = nt;
         a.nt_base = nt_base ? nt_base : c->d_ntbase + 1;   // the second word stays zero
@@ -954,15 +991,23 @@ static int enqueue_steps(dn_ctx *c, StepArgs &a, int n, bool adjoint, bool pack_
         a.psx_out = c->d_psx[cur ^ 1];
         a.psy_in = c->d_psy[cur];
         a.psy_out = c->d_psy[cur ^ 1];
+        if (a.ms_steps > 0) {
+            a.pvx_in = cur ? c->d_pvx2 : c->d_pvx;
+            a.pvy_in = cur ? c->d_pvy2 : c->d_pvy;
+            a.pvx = cur ? c->d_pvx : c->d_pvx2;
+            a.pvy = cur ? c->d_pvy : c->d_pvy2;
+            a.ms_steps = std::min(per, count - k);
+            bool extra = false;
+            for (int q = 0; q < a.ms_steps; ++q) extra = extra || extra_at(nt + q);
+            HIPCHK(c, launch_multi(a, c->K, adjoint, extra, c->stream));
+            cur ^= 1;
+            continue;
+        }
         // inside a chunk the counter is a multiple of dtinv, so the store
         // pattern depends on the offset only
         const bool pack = pack_mode && ((nt - 1) % c->p.dtinv) == 0;
         if (pack) HIPCHK(c, launch_fill_u32(c->d_stage_max, (size_t)n * 3, 0u, c->stream));
-        // adjoint: shot s correlates at step nt when nt = NT_s (mod dtinv);
-        // inside a chunk the counter is a multiple of dtinv
-        const int dt = c->p.dtinv;
-        const bool extra = adjoint ? corr_res[((nt % dt) + dt) % dt] != 0 : (fwd_extra && ((nt - 1) % dt) == 0);
-        HIPCHK(c, launch_step(a, c->K, c->p.L > 0, adjoint, extra, c->stream));
+        HIPCHK(c, launch_step(a, c->K, c->p.L > 0, adjoint, extra_at(nt), c->stream));
         if (pack)
             HIPCHK(c, launch_snap_pack(n, c->g.nx, c->g.ny, c->d_stage, c->d_stage_max, c->d_snap16, c->d_snap_scale,
                                        a.snap_shot_stride, nsnap, nt_base, nt, c->p.dtinv, kind, c->stream));
@@ -971,12 +1016,13 @@ static int enqueue_steps(dn_ctx *c, StepArgs &a, int n, bool adjoint, bool pack_
     return 0;
 }
 
-static int chunk_steps(const dn_ctx *c)
+// per: steps per launch.  The ping-pong parity (two launches) and the store
+// pattern (dtinv steps) repeat from chunk to chunk.
+static int chunk_steps(const dn_ctx *c, int per)
 {
     if (c->graph_steps == 0) return 0;
     const int target = c->graph_steps > 0 ? c->graph_steps : 64;
-    const int dt = c->p.dtinv;
-    const int l = (dt % 2 == 0) ? dt : 2 * dt;   // lcm(2, dtinv): ping-pong parity and store pattern repeat
+    const int l = std::lcm(2 * per, c->p.dtinv);
     return l * std::max(1, (target + l - 1) / l);
 }
 
@@ -987,9 +1033,10 @@ static int get_graph(dn_ctx *c, StepArgs a, int n, bool adjoint, bool store, boo
 {
     const int kind = c->p.snap_precision;
     const bool hess = a.hess != 0;
+    const int multi = a.ms_steps > 0;
     for (auto &gr : c->graphs)
-        if (gr.n == n && gr.R == a.R && gr.steps == steps && gr.kind == kind && gr.adjoint == adjoint &&
-            gr.store == store && gr.record == record && gr.hess == hess && gr.corr_res == corr_res) {
+        if (gr.n == n && gr.R == a.R && gr.steps == steps && gr.kind == kind && gr.multi == multi &&
+            gr.adjoint == adjoint && gr.store == store && gr.record == record && gr.hess == hess && gr.corr_res == corr_res) {
             *out = gr.exec;
             return 0;
         }
@@ -1009,7 +1056,7 @@ static int get_graph(dn_ctx *c, StepArgs a, int n, bool adjoint, bool store, boo
     const hipError_t ei = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
     if (ei != hipSuccess) return dn_fail(c, "graph instantiate failed: %s", hipGetErrorString(ei));
-    c->graphs.push_back({n, a.R, steps, kind, adjoint, store, record, hess, corr_res, exec});
+    c->graphs.push_back({n, a.R, steps, kind, multi, adjoint, store, record, hess, corr_res, exec});
     *out = exec;
     return 0;
 }
@@ -1079,7 +1126,14 @@ int dn_run_pass(dn_ctx *c, const std::vector<int> &shots, bool adjoint, bool sto
     std::vector<char> corr_res(c->p.dtinv, 0);
     for (int sh : shots) corr_res[c->shot_nt[sh] % c->p.dtinv] = 1;
     const bool fwd_extra = store || c->hess_mode;
-    const int CH = chunk_steps(c);
+    if (choose_multi(c, n, adjoint, store, c->hess_mode != 0)) {
+        a.ms_steps = multi_steps(c->K);
+        a.tl_ny = multi_tiles_y(c->g.ny);
+        a.tl_nblk = n * multi_tiles(c->g.nx, c->g.ny);
+        a.tl_nblk8 = (a.tl_nblk + 7) / 8;
+    }
+    const int per = a.ms_steps > 0 ? multi_steps(c->K) : 1;
+    const int CH = chunk_steps(c, per);
     const int nchunks = (CH > 0 && ntmax >= 2 * CH) ? ntmax / CH : 0;
     hipGraphExec_t exec = nullptr;
     if (nchunks > 0) {
@@ -1093,10 +1147,11 @@ int dn_run_pass(dn_ctx *c, const std::vector<int> &shots, bool adjoint, bool sto
         for (int k = 0; k < nchunks; ++k) HIPCHK(c, hipGraphLaunch(exec, c->stream));
         c->graph_replays += nchunks;
     }
-    const int done = nchunks * CH;   // even: the fields are back in half 0
+    const int done = nchunks * CH;   // an even number of launches: the fields are back in half 0
     if (enqueue_steps(c, a, n, adjoint, pack_mode, nsnap, done + 1, ntmax - done, nullptr, cur, corr_res, fwd_extra))
         return -1;
-    c->launches += ntmax;
+    const int nlaunch = done / per + (ntmax - done + per - 1) / per;
+    c->launches += nlaunch;
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     HIPCHK(c, hipEventSynchronize(c->ev1));
     float ms = 0.0f;
@@ -1106,7 +1161,7 @@ int dn_run_pass(dn_ctx *c, const std::vector<int> &shots, bool adjoint, bool sto
     for (int s = 0; s < n; ++s) cells += (long long)c->g.nx * c->g.ny * std::min(c->shot_nt[shots[s]], ntmax);
     c->cell_updates += cells;
     c->ms_pass[adjoint ? 1 : 0] += ms;
-    c->launches_pass[adjoint ? 1 : 0] += ntmax;
+    c->launches_pass[adjoint ? 1 : 0] += nlaunch;
     c->cells_pass[adjoint ? 1 : 0] += cells;
     c->cur_final = cur;
     // the kernel's latch: NaN at the probe cell after some step

@@ -61,6 +61,7 @@ struct dn_ctx {
     float *d_vy[2] = {nullptr, nullptr}, *d_sxy[2] = {nullptr, nullptr}, *d_syz[2] = {nullptr, nullptr};
     float *d_psx[2] = {nullptr, nullptr}, *d_psy[2] = {nullptr, nullptr};
     float *d_rq = nullptr, *d_pvx = nullptr, *d_pvy = nullptr;
+    float *d_pvx2 = nullptr, *d_pvy2 = nullptr;   // second halves for several steps per launch
     float *d_seis = nullptr, *d_resid = nullptr, *d_snap = nullptr;
     uint16_t *d_snap16 = nullptr;
     float *d_snap_scale = nullptr, *d_stage = nullptr;
@@ -80,7 +81,7 @@ struct dn_ctx {
     long long launches_pass[2] = {0, 0}, cells_pass[2] = {0, 0};
     // time-loop replay: captured chunks of `steps` time steps per batch shape
     struct Graph {
-        int n, R, steps, kind;
+        int n, R, steps, kind, multi;
         bool adjoint, store, record, hess;
         std::vector<char> corr_res;   // record-length residues that select the correlating launches
         hipGraphExec_t exec;

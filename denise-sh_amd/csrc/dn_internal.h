@@ -82,6 +82,7 @@ struct StepArgs {
     int nshots;                    // shots in this launch
     int nshots_all;                // shots of the context (bound of shot_map entries)
     int tl_rw;                     // tile step: rows per wave; 0: the strip step
+    int ms_steps;                  // steps of a launch of launch_multi
     int tl_w, tl_h;                // columns and rows of a tile
     int tl_ny;                     // tiles in a column of tiles
     int tl_nblk, tl_nblk8;         // tiles of all shots, and per XCD slice
@@ -108,6 +109,7 @@ struct StepArgs {
     const float *psy_in;                    // psi_syy_y [s][2fw][nx] (ping-pong)
     float *psx_out, *psy_out;
     float *pvx, *pvy;                       // psi_vyx [s][ny][2fw], psi_vyy [s][2fw][nx]
+    const float *pvx_in, *pvy_in;           // several steps per launch: their old values (ping-pong)
     float *vy_out, *sxy_out, *syz_out;
     float DT, DH, dhi, dthalbe;
     float hc[7];
@@ -163,6 +165,15 @@ hipError_t launch_step(const StepArgs &a, int K, bool visco, bool adjoint, bool 
 // the same step on two-dimensional tiles (dn_tile.hip, one object per K);
 // a.tl_* must be set
 template <int K> hipError_t launch_tile_k(const StepArgs &a, int L, bool adjoint, bool extra, hipStream_t st);
+
+// up to multi_steps(K) elastic steps (L 0, K 1 or 2) in one launch (dn_multi.hip);
+// a.ms_steps and a.tl_ny, tl_nblk, tl_nblk8 must be set for multi_tiles, and
+// every *_in / *_out pair with pvx_in, pvx and pvy_in, pvy be two buffers.
+// extra as in launch_step, for any of the steps; FP32 snapshots only.
+int multi_steps(int K);
+int multi_tiles(int nx, int ny);
+int multi_tiles_y(int ny);
+hipError_t launch_multi(const StepArgs &a, int K, bool adjoint, bool extra, hipStream_t st);
 
 struct ModelPrepArgs {
     Geo g;

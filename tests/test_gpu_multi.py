@@ -1,0 +1,55 @@
+"""Several time steps per launch against the strip step (chosen by a
+rows-per-segment request) at the edges of its tiles of 24 x 8 cells: forward
+seismograms, gradients, misfits, energy maps, pseudo-Hessian and fields must
+be the same bits, and the gradient the oracle's.  Records end at every place
+inside a launch, and the longest replay captured launches."""
+import numpy as np
+import pytest
+
+from common import oracle, product
+from test_gpu_tile import _inputs, _run, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nx,ny,fdorder,free_surf,boundary,shots,snap,dtinv,two,nt", [
+    (48, 24, 4, 0, 0, 1, 0, 1, False, 150),
+    (47, 25, 4, 1, 0, 3, 0, 2, True, 149),
+    (49, 23, 2, 0, 0, 2, 0, 3, False, 151),
+    (97, 40, 4, 0, 0, 3, 0, 5, False, 162),
+    (64, 41, 2, 1, 0, 4, 0, 4, True, 150),
+    (128, 33, 4, 1, 1, 2, 0, 2, False, 150),   # periodic: the narrowest grid on tiles
+    (130, 40, 2, 0, 1, 3, 0, 1, True, 149),
+    (65, 39, 4, 0, 0, 2, 1, 2, False, 150),    # 16-bit snapshots: recording passes only
+    (70, 24, 4, 1, 0, 1, 2, 2, False, 3),      # shorter than a launch
+    (24, 24, 4, 0, 0, 1, 0, 1, False, 5),
+    (576, 64, 4, 0, 0, 4, 0, 3, False, 40),    # 768 workgroups: the most for a gradient
+    (577, 64, 4, 0, 0, 4, 0, 3, False, 40),    # 800: forward several steps, gradient tiles
+    (1104, 88, 2, 0, 0, 4, 0, 2, False, 40),   # 2024 of FDORDER 2
+])
+def test_several_steps_equal_strips(nx, ny, fdorder, free_surf, boundary, shots, snap, dtinv, two, nt):
+    say("several steps", nx, ny, "FDORDER", fdorder, "shots", shots, "steps", nt)
+    par = dict(nx=nx, ny=ny, fdorder=fdorder, L=0, free_surf=free_surf, boundary=boundary, snap=snap, dtinv=dtinv, fw=8)
+    inp = list(_inputs(nx, ny, shots, nt, seed=nx + ny))
+    inp[8] = np.maximum(1, nt - np.arange(shots)).astype(np.int32)
+    dn = product()
+    a = _run(dn, par, inp, 0, two)
+    b = _run(dn, par, inp, 13, two)
+    assert np.isfinite(a[2]).all() and (nt < 40 or np.abs(a[2]).max() > 0)
+    for k, (x, y) in enumerate(zip(a, b)):
+        assert np.array_equal(x, y), "output %d differs" % k
+
+
+@pytest.mark.parametrize("nx,ny,fdorder", [(65, 33, 4), (40, 30, 2)])
+def test_several_steps_equal_oracle(nx, ny, fdorder):
+    from pyoracle import make_cfg
+    say("several steps against the oracle", nx, ny)
+    par = dict(nx=nx, ny=ny, fdorder=fdorder, L=0, free_surf=0, boundary=0, snap=0, dtinv=2, fw=8)
+    inp = list(_inputs(nx, ny, 2, 62, seed=3))
+    inp[8] = np.full(2, 62, np.int32)
+    vs, rho, _, sig, si, sj, ri, rj, _, obs = inp
+    got = _run(product(), par, inp, 0, False)
+    cfg = make_cfg(nx, ny, fdorder=fdorder, fw=8, free_surf=0, L=0, nt=62, dtinv=2, dt=1e-4, dh=0.25, damping=300.0,
+                   fpml=40.0, fl=[])
+    ref = oracle("f32").gradient(cfg, vs, rho, None, si, sj, sig, ri, rj, obs)
+    assert np.array_equal(got[2], ref["grad_vs"]) and np.array_equal(got[3], ref["grad_rho"])
