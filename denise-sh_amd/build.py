@@ -26,11 +26,11 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Wall", "-Wno-unus
 DEVICE = ["--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
           "-fno-gpu-rdc"]
 
-# (source, flags[, object name]); the tile step is compiled once per stencil
-# half-order, so that the objects build in parallel
+# (source, flags[, object name]); the tile step and the several-step kernel are
+# compiled once per stencil half-order, so that the objects build in parallel
 SOURCES = [("dn_tile.hip", ["-DDN_TILE_K=%d" % k], "dn_tile_k%d" % k) for k in (4, 6, 5, 3, 2, 1)] + [
+    ("dn_multi.hip", ["-DDN_MULTI_K=%d" % k], "dn_multi_k%d" % k) for k in (4, 3, 2, 1)] + [
     ("dn_kernels.hip", []),
-    ("dn_multi.hip", []),
     ("dn_core.cpp", []),
     ("dn_setup.cpp", []),
     ("dn_dropin.cpp", []),

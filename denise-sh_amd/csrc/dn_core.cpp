@@ -208,7 +208,7 @@ static void free_batch(dn_ctx *c)
         dfree_t(c->d_psx[k]);
         dfree_t(c->d_psy[k]);
     }
-    dfree_t(c->d_rq); dfree_t(c->d_pvx); dfree_t(c->d_pvy); dfree_t(c->d_pvx2); dfree_t(c->d_pvy2);
+    dfree_t(c->d_rq); dfree_t(c->d_pvx); dfree_t(c->d_pvy); dfree_t(c->d_rq2); dfree_t(c->d_pvx2); dfree_t(c->d_pvy2);
     dfree_t(c->d_seis); dfree_t(c->d_resid); dfree_t(c->d_snap); dfree_t(c->d_snap16); dfree_t(c->d_snap_scale);
     dfree_t(c->d_stage); dfree_t(c->d_stage_max);
     dfree_t(c->d_Ws); dfree_t(c->d_Wr); dfree_t(c->d_gu_shot); dfree_t(c->d_grho_shot); dfree_t(c->d_part);
@@ -705,8 +705,35 @@ extern "C" int dn_autotune(dn_ctx *c, int nshots, int nsteps, int *rows_out, int
     return 0;
 }
 
-// grids that dn_multi.hip can step
-static bool multi_capable(const dn_ctx *c) { return c->p.L == 0 && c->K <= 2; }
+// The most workgroups of the several-step kernel (dn_multi.hip; 24 x 8 cells
+// each) with which it is faster than the tile step.  extra: passes that store
+// snapshots or sum or correlate (more registers: one workgroup per CU).
+// Microseconds per step, tiles / several steps, forward and gradient, by
+// workgroups (1: 400x120, 255; 2: two such shots, 510):
+// FDORDER 2       1 5.4 / 1.5, 6.3 / 2.1   800x480 (2040) 7.7 / 4.9, 10.7 / 8.5
+//   with L 3                               800x480 9.4 / 6.0, 12.4 / 9.5
+// FDORDER 4       1 5.5 / 2.5, 6.6 / 3.2   2 5.7 / 3.3, 6.9 / 5.0
+//   750 (700x200) 5.8 / 4.5, 7.3 / 6.7     1020 6.5 / 5.2, 8.1 / 8.3
+//   with L 2      1 5.7 / 2.7, 6.5 / 3.5   2 5.8 / 4.7, 6.9 / 5.9
+//   with L 2, 625 (600x200) 5.7 / 6.2, 6.9 / 8.0
+// FDORDER 6       1 5.6 / 3.3, 6.5 / 4.0   420 (500x160) 5.6 / 4.3, 6.6 / 6.8
+//   with L 2      1 5.9 / 3.6, 6.8 / 4.4   420, two steps 5.9 / 6.2, 7.0 / 7.8
+// FDORDER 8       1 5.8 / 4.0, 6.6 / 5.0   2 5.9 / 5.4, 6.9 / 8.6
+//   with L 2      1 6.0 / 4.4, 6.9 / 5.4   420 6.0 / 7.5, 7.1 / 9.1
+// Beyond FDORDER 8 a second step reaches too many cells.
+static int multi_limit(const dn_ctx *c, bool extra)
+{
+    if (c->K > kMultiMaxK || c->p.L > kMultiMaxL) return 0;
+    if (c->K == 1) return 2048;
+    if (c->K == 2) return c->p.L > 0 ? 512 : (extra ? 768 : 1024);
+    return c->p.L > 0 || extra ? 256 : 512;
+}
+static int multi_tiles(const dn_ctx *c)
+{
+    return ((c->g.nx + kMultiX - 1) / kMultiX) * ((c->g.ny + kMultiY - 1) / kMultiY);
+}
+// some pass over one shot can use it: the batch holds the second halves
+static bool multi_capable(const dn_ctx *c) { return multi_tiles(c) <= multi_limit(c, false); }
 
 int dn_nsnap(const dn_ctx *c) { return (c->nt_max + c->p.dtinv - 1) / c->p.dtinv; }
 
@@ -715,7 +742,7 @@ static size_t per_shot_bytes(const dn_ctx *c, bool gradient)
 {
     const Geo &g = c->g;
     const size_t P = (size_t)g.plane, nxny = (size_t)g.nx * g.ny;
-    size_t b = 6 * P * 4 + 2 * (size_t)g.L * P * 4;                 // vy,sxy,syz x2, r, q
+    size_t b = 6 * P * 4 + (multi_capable(c) ? 4 : 2) * (size_t)g.L * P * 4;   // vy,sxy,syz x2, r, q
     b += (size_t)(2 * 2 + 2) * (size_t)(2 * g.fw) * (g.nx + g.ny) * 4;  // psi, at least as many as there are
     b += 2 * (size_t)c->ntr * c->nt_max * 4;                        // seis + resid
     b += 4 * nxny * 4 + (size_t)c->ntr * 16;                        // Ws, Wr, gu, grho, partials
@@ -763,6 +790,7 @@ int dn_ensure_batch(dn_ctx *c, int want, bool gradient)
     HIPCHK(c, dalloc(&c->d_pvx, S * fw2 * g.ny));
     HIPCHK(c, dalloc(&c->d_pvy, S * fw2 * g.nx));
     if (multi_capable(c)) {
+        if (g.L > 0) HIPCHK(c, dalloc(&c->d_rq2, S * P * 2 * g.L));
         HIPCHK(c, dalloc(&c->d_pvx2, S * fw2 * g.ny));
         HIPCHK(c, dalloc(&c->d_pvy2, S * fw2 * g.nx));
     }
@@ -859,19 +887,12 @@ static int choose_tile(const dn_ctx *c, int nshots)
 
 // Several steps per launch (dn_multi.hip)?  Where nothing needs another launch
 // between two steps (FP16 snapshots are packed after each stored step, BF16
-// ones scaled by the snapshot before) and the recomputed cells do not cost
-// more than the launches.  Microseconds per step, tiles / several steps, by
-// workgroups of 24 x 8 cells, forward and gradient: FDORDER 4: 255 (400x120)
-// 5.5 / 2.5, 6.6 / 3.2; 510 5.7 / 3.3, 6.9 / 5.0; 750 (700x200) 5.8 / 4.5,
-// 7.3 / 6.7; 850 6.1 / 5.1, 7.7 / 8.1; 1020 6.5 / 5.2, 8.1 / 8.3.  FDORDER 2:
-// 1292 (800x300) 6.3 / 3.4, 7.9 / 5.4; 2100 8.0 / 5.0, 9.9 / 8.1; 2584
-// 8.2 / 6.0, 10.0 / 9.2.
+// ones scaled by the snapshot before), within multi_limit.
 static bool choose_multi(const dn_ctx *c, int nshots, bool adjoint, bool store, bool hess)
 {
     if (!multi_capable(c) || choose_tile(c, nshots) == 0) return false;
     if ((adjoint || store) && c->p.snap_precision != 0) return false;
-    const int limit = c->K == 1 ? 2048 : (adjoint || store || hess ? 768 : 1024);
-    return (long long)nshots * multi_tiles(c->g.nx, c->g.ny) <= limit;
+    return (long long)nshots * multi_tiles(c) <= multi_limit(c, adjoint || store || hess);
 }
 
 void dn_fill_step_common(dn_ctx *c, StepArgs &a, int n)
@@ -956,6 +977,7 @@ int dn_zero_state(dn_ctx *c, int n)
     HIPCHK(c, launch_fill(c->d_pvx, S * fw2 * g.ny, 0.0f, c->stream));
     HIPCHK(c, launch_fill(c->d_pvy, S * fw2 * g.nx, 0.0f, c->stream));
     if (c->d_pvx2) {
+        if (c->d_rq2) HIPCHK(c, launch_fill(c->d_rq2, S * P * 2 * g.L, 0.0f, c->stream));
         HIPCHK(c, launch_fill(c->d_pvx2, S * fw2 * g.ny, 0.0f, c->stream));
         HIPCHK(c, launch_fill(c->d_pvy2, S * fw2 * g.nx, 0.0f, c->stream));
     }
@@ -996,10 +1018,12 @@ static int enqueue_steps(dn_ctx *c, StepArgs &a, int n, bool adjoint, bool pack_
             a.pvy_in = cur ? c->d_pvy2 : c->d_pvy;
             a.pvx = cur ? c->d_pvx : c->d_pvx2;
             a.pvy = cur ? c->d_pvy : c->d_pvy2;
+            a.rq_in = cur ? c->d_rq2 : c->d_rq;
+            a.rq = cur ? c->d_rq : c->d_rq2;
             a.ms_steps = std::min(per, count - k);
             bool extra = false;
             for (int q = 0; q < a.ms_steps; ++q) extra = extra || extra_at(nt + q);
-            HIPCHK(c, launch_multi(a, c->K, adjoint, extra, c->stream));
+            HIPCHK(c, launch_step(a, c->K, c->p.L > 0, adjoint, extra, c->stream));
             cur ^= 1;
             continue;
         }
@@ -1128,8 +1152,8 @@ int dn_run_pass(dn_ctx *c, const std::vector<int> &shots, bool adjoint, bool sto
     const bool fwd_extra = store || c->hess_mode;
     if (choose_multi(c, n, adjoint, store, c->hess_mode != 0)) {
         a.ms_steps = multi_steps(c->K);
-        a.tl_ny = multi_tiles_y(c->g.ny);
-        a.tl_nblk = n * multi_tiles(c->g.nx, c->g.ny);
+        a.tl_ny = (c->g.ny + kMultiY - 1) / kMultiY;
+        a.tl_nblk = n * multi_tiles(c);
         a.tl_nblk8 = (a.tl_nblk + 7) / 8;
     }
     const int per = a.ms_steps > 0 ? multi_steps(c->K) : 1;

@@ -109,7 +109,7 @@ struct StepArgs {
     const float *psy_in;                    // psi_syy_y [s][2fw][nx] (ping-pong)
     float *psx_out, *psy_out;
     float *pvx, *pvy;                       // psi_vyx [s][ny][2fw], psi_vyy [s][2fw][nx]
-    const float *pvx_in, *pvy_in;           // several steps per launch: their old values (ping-pong)
+    const float *pvx_in, *pvy_in, *rq_in;   // several steps per launch: the old values (ping-pong)
     float *vy_out, *sxy_out, *syz_out;
     float DT, DH, dhi, dthalbe;
     float hc[7];
@@ -166,14 +166,14 @@ hipError_t launch_step(const StepArgs &a, int K, bool visco, bool adjoint, bool 
 // a.tl_* must be set
 template <int K> hipError_t launch_tile_k(const StepArgs &a, int L, bool adjoint, bool extra, hipStream_t st);
 
-// up to multi_steps(K) elastic steps (L 0, K 1 or 2) in one launch (dn_multi.hip);
-// a.ms_steps and a.tl_ny, tl_nblk, tl_nblk8 must be set for multi_tiles, and
-// every *_in / *_out pair with pvx_in, pvx and pvy_in, pvy be two buffers.
-// extra as in launch_step, for any of the steps; FP32 snapshots only.
-int multi_steps(int K);
-int multi_tiles(int nx, int ny);
-int multi_tiles_y(int ny);
-hipError_t launch_multi(const StepArgs &a, int K, bool adjoint, bool extra, hipStream_t st);
+// Up to multi_steps(K) steps of a grid in one launch (dn_multi.hip; K <= 4,
+// L <= 3).  a.ms_steps and a.tl_ny, tl_nblk, tl_nblk8 must be set for tiles of
+// kMultiX x kMultiY cells, and every *_in / *_out pair with pvx_in, pvx;
+// pvy_in, pvy; rq_in, rq be two buffers.  extra as in launch_step, for any of
+// the steps; FP32 snapshots only.
+constexpr int kMultiX = 24, kMultiY = 8, kMultiMaxK = 4, kMultiMaxL = 3;
+__host__ __device__ constexpr int multi_steps(int K) { return K == 1 ? 6 : (K == 2 ? 4 : (K == 3 ? 3 : 2)); }
+template <int K> hipError_t launch_multi_k(const StepArgs &a, bool adjoint, bool extra, hipStream_t st);
 
 struct ModelPrepArgs {
     Geo g;

@@ -781,11 +781,22 @@ template <> hipError_t launch_tile_k<3>(const StepArgs &a, int L, bool adjoint, 
 template <> hipError_t launch_tile_k<4>(const StepArgs &a, int L, bool adjoint, bool extra, hipStream_t st);
 template <> hipError_t launch_tile_k<5>(const StepArgs &a, int L, bool adjoint, bool extra, hipStream_t st);
 template <> hipError_t launch_tile_k<6>(const StepArgs &a, int L, bool adjoint, bool extra, hipStream_t st);
+template <> hipError_t launch_multi_k<1>(const StepArgs &a, bool adjoint, bool extra, hipStream_t st);
+template <> hipError_t launch_multi_k<2>(const StepArgs &a, bool adjoint, bool extra, hipStream_t st);
+template <> hipError_t launch_multi_k<3>(const StepArgs &a, bool adjoint, bool extra, hipStream_t st);
+template <> hipError_t launch_multi_k<4>(const StepArgs &a, bool adjoint, bool extra, hipStream_t st);
 
 hipError_t launch_step(const StepArgs &a, int K, bool visco, bool adjoint, bool extra, hipStream_t st)
 {
     const int L = visco ? a.g.L : 0;
     if (visco != (a.g.L > 0)) return hipErrorInvalidValue;
+    if (a.ms_steps > 0) switch (K) {
+        case 1: return launch_multi_k<1>(a, adjoint, extra, st);
+        case 2: return launch_multi_k<2>(a, adjoint, extra, st);
+        case 3: return launch_multi_k<3>(a, adjoint, extra, st);
+        case 4: return launch_multi_k<4>(a, adjoint, extra, st);
+        default: return hipErrorInvalidValue;
+        }
     if (a.tl_rw > 0) switch (K) {
         case 1: return launch_tile_k<1>(a, L, adjoint, extra, st);
         case 2: return launch_tile_k<2>(a, L, adjoint, extra, st);

@@ -1,4 +1,4 @@
-// Several elastic time steps per launch for grids that leave most of the chip
+// Several time steps per launch for grids that leave most of the chip
 // idle (gfx950).  Same arithmetic, in the same order and rounding, as the
 // tile step (dn_tile.hip); compiled with -ffp-contract=off.
 //
@@ -13,41 +13,44 @@
 // barriers and stores) and the next follows 1.4 us later; a step in here is
 // two updates from LDS, so T of them share one load, one store and one
 // launch.  The price is work: 1536 cells for 192 owned ones in the first step
-// of FDORDER 4, so the rule (dn_core.cpp) stops where that fills the chip.
-// 400 x 120, one shot, microseconds per step, tiles -> several steps:
-// FDORDER 4 forward 5.5 -> 2.5, gradient 6.6 -> 3.2; FDORDER 2 5.4 -> 1.5,
-// 6.3 -> 2.1.
+// of FDORDER 4, so the rule (multi_limit in dn_core.cpp, with both sides'
+// times) stops where that fills the chip.  400 x 120, one shot, microseconds
+// per step, tiles -> several steps: FDORDER 4 forward 5.5 -> 2.5, gradient
+// 6.6 -> 3.2; FDORDER 8 with L 2 6.0 -> 4.4, 6.9 -> 5.4.
 // Shape (the same forward / gradient of FDORDER 4, whole calls of 2000 / 1500
 // steps, ms): 24 x 8 cells and 4 steps 4.73 / 8.73; 32 x 8 and 3, 4, 5, 6
 // steps 5.40 / 9.90, 4.95 / 9.32, 5.21 / 11.8, 4.99 / 9.26; 20 x 10 4.83 /
-// 8.93; 16 x 16 5.02 / 9.46.  FDORDER 2 with 4, 6, 8 steps: 1.64, 1.46, 1.57
-// us per step.  The CPML profiles lie in LDS, not in registers, and all but
-// the correlating kernel are held to 80 registers: two workgroups share a CU
-// (500 x 160: 4.09 -> 3.22 us per step, gradient 5.31 -> 4.86; the correlating
-// kernel spilled at that limit, +12 % at 400 x 120).
+// 8.93; 16 x 16 5.02 / 9.46.  Steps of other orders: FDORDER 2 with 4, 6, 8
+// 1.64, 1.46, 1.57 us per step; FDORDER 6 with 2, 3 3.44, 3.29.  The CPML
+// profiles lie in LDS, not in registers, and the elastic kernels of FDORDER 2
+// and 4 are held to 80 registers: two workgroups share a CU (500 x 160: 4.09
+// -> 3.22 us per step, gradient 5.31 -> 4.86); not the correlating one, which
+// spilled at that limit (+12 % at 400 x 120).
 //
 // Everything the cells around the tile read is double-buffered (here also the
-// stress CPML memory, which the single steps update in place).
+// stress CPML memory and the relaxation variables, which the single steps
+// update in place).
 #include "dn_internal.h"
 
 #pragma clang fp contract(off)
+
+#ifndef DN_MULTI_K
+#error "compile with -DDN_MULTI_K=<FDORDER / 2>"
+#endif
 
 namespace dn {
 
 namespace {
 
-constexpr int kMX = 24, kMY = 8, kMThreads = 768;
-
-// steps per launch: as many as leave at most two cells for a thread (FDORDER 4:
-// 48 x 32 cells, 3 steps) or one (FDORDER 2: 36 x 20)
-constexpr int steps_of(int K) { return K == 1 ? 6 : 4; }
+constexpr int kMThreads = 768;
 
 // EX: launches that store FP32 snapshots or sum the pseudo-Hessian (forward),
 // or correlate with FP32 snapshots (adjoint), in some of their steps
-template <int K, bool ADJ, bool EX>
-__global__ __launch_bounds__(kMThreads, ADJ && EX ? 3 : 6) void k_multi(const StepArgs a)
+template <int K, int L, bool ADJ, bool EX>
+__global__ __launch_bounds__(kMThreads, L == 0 && K <= 2 && !(ADJ && EX) ? 6 : 3) void k_multi(const StepArgs a)
 {
-    constexpr int T = steps_of(K), H = 2 * K - 1, M = T * H;
+    constexpr int T = multi_steps(K), H = 2 * K - 1, M = T * H, kMX = kMultiX, kMY = kMultiY;
+    constexpr int LD = L > 0 ? L : 1;
     constexpr int W = kMX + 2 * M, HT = kMY + 2 * M, N = W * HT, NC = (N + kMThreads - 1) / kMThreads;
     __shared__ float lv[N], lx[N], lz[N];
     __shared__ float lkx[6 * W], lky[6 * HT];   // CPML K, a, b of the velocity, then of the stress
@@ -71,6 +74,7 @@ __global__ __launch_bounds__(kMThreads, ADJ && EX ? 3 : 6) void k_multi(const St
     const float *__restrict__ vyi = a.vy_in + s0 * g.plane;
     const float *__restrict__ sxi = a.sxy_in + s0 * g.plane;
     const float *__restrict__ szi = a.syz_in + s0 * g.plane;
+    const float *__restrict__ rqi = L > 0 ? a.rq_in + s0 * 2 * L * g.plane : nullptr;
     const float *__restrict__ pmlb = a.pml.Kx;
     const float *__restrict__ pxi = a.psx_in + s0 * g.ny * fw2, *__restrict__ pyi = a.psy_in + s0 * fw2 * g.nx;
     const float *__restrict__ wxi = a.pvx_in + s0 * g.ny * fw2, *__restrict__ wyi = a.pvy_in + s0 * fw2 * g.nx;
@@ -79,6 +83,7 @@ __global__ __launch_bounds__(kMThreads, ADJ && EX ? 3 : 6) void k_multi(const St
     int cr[NC], cq[NC], cj[NC], cw[NC];   // row and column in the workgroup's region, grid row, wrapped column
     bool in[NC], own[NC];
     float v[NC], sx[NC], sz[NC], b[NC], u1[NC], u2[NC];
+    float rr[NC][LD], qq[NC][LD], dp[NC][LD], dd[NC][LD];   // relaxation variables and their coefficients
     unsigned off[NC];
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
@@ -97,9 +102,36 @@ __global__ __launch_bounds__(kMThreads, ADJ && EX ? 3 : 6) void k_multi(const St
         sx[i] = sxi[off[i]];
         sz[i] = szi[off[i]];
         b[i] = a.bfield[off[i]];
-        const float2 u = *(const float2 *)(a.spk + 2 * (size_t)off[i]);
-        u1[i] = u.x;
-        u2[i] = u.y;
+        if (L == 0) {
+            const float2 u = *(const float2 *)(a.spk + 2 * (size_t)off[i]);
+            u1[i] = u.x;
+            u2[i] = u.y;
+        } else {
+            const float4 u = *(const float4 *)(a.spk + 4 * (size_t)off[i]);
+            u1[i] = u.x;
+            u2[i] = u.y;
+            dp[i][0] = u.z;
+            dd[i][0] = u.w;
+#pragma unroll
+            for (int l = 1; l < L; ++l) {
+                const float2 w = *(const float2 *)(a.spk + (2 + 2 * l) * g.plane + 2 * (size_t)off[i]);
+                dp[i][l] = w.x;
+                dd[i][l] = w.y;
+            }
+#pragma unroll
+            for (int l = 0; l + 1 < L; l += 2) {
+                const float4 w = *(const float4 *)(rqi + 2 * l * g.plane + 4 * (size_t)off[i]);
+                rr[i][l] = w.x;
+                qq[i][l] = w.y;
+                rr[i][l + 1] = w.z;
+                qq[i][l + 1] = w.w;
+            }
+            if (L & 1) {
+                const float2 w = *(const float2 *)(rqi + 2 * (L - 1) * g.plane + 2 * (size_t)off[i]);
+                rr[i][L - 1] = w.x;
+                qq[i][L - 1] = w.y;
+            }
+        }
     }
     // CPML variables and profiles, in workgroups that reach into an absorbing
     // region (uniform)
@@ -133,7 +165,9 @@ __global__ __launch_bounds__(kMThreads, ADJ && EX ? 3 : 6) void k_multi(const St
     if (tpy) {
         for (int e = threadIdx.x; e < 6 * HT; e += kMThreads) {
             const int f = e / HT, j = j0 - M + (e - f * HT);
-            lky[e] = pmlb[(6 + f) * pn + min(max(j <= fw ? j : j - g.ny + fw2, 0), fw2)];
+            // Q2: the viscoelastic stress uses the full-grid y profile on top
+            const int fp = (L > 0 && f >= 3 && !g.free_surf && j <= fw) ? f + 3 : f + 6;
+            lky[e] = pmlb[fp * pn + min(max(j <= fw ? j : j - g.ny + fw2, 0), fw2)];
         }
     }
     // the gradient sums of the owned cells stay in registers over the steps
@@ -294,8 +328,30 @@ __global__ __launch_bounds__(kMThreads, ADJ && EX ? 3 : 6) void k_multi(const St
             vyy = vyy * a.dhi;
             if (xk[i] > 0) cpml(lkx[3 * W + cq[i]], lkx[4 * W + cq[i]], lkx[5 * W + cq[i]], wx[i], vyx);
             if (yk[i] > 0) cpml(lky[3 * HT + cr[i]], lky[4 * HT + cr[i]], lky[5 * HT + cr[i]], wy[i], vyy);
-            sx[i] = sx[i] + u1[i] * vyx;
-            sz[i] = sz[i] + u2[i] * vyy;
+            if (L == 0) {
+                sx[i] = sx[i] + u1[i] * vyx;
+                sz[i] = sz[i] + u2[i] * vyy;
+            } else {
+                float sumr = 0.0f, sumq = 0.0f;
+#pragma unroll
+                for (int l = 0; l < L; ++l) {
+                    sumr += rr[i][l];
+                    sumq += qq[i][l];
+                }
+                sx[i] = sx[i] + ((u1[i] * vyx) + (a.dthalbe * sumr));
+                sz[i] = sz[i] + ((u2[i] * vyy) + (a.dthalbe * sumq));
+                sumr = 0.0f;
+                sumq = 0.0f;
+#pragma unroll
+                for (int l = 0; l < L; ++l) {
+                    rr[i][l] = a.bip[l] * (rr[i][l] * a.cip[l] - (dp[i][l] * vyx));
+                    qq[i][l] = a.bjm[l] * (qq[i][l] * a.cjm[l] - (dd[i][l] * vyy));
+                    sumr += rr[i][l];
+                    sumq += qq[i][l];
+                }
+                sx[i] = sx[i] + (a.dthalbe * sumr);
+                sz[i] = sz[i] + (a.dthalbe * sumq);
+            }
             lx[e] = sx[i];
             lz[e] = sz[i];
             if (EX && own[i]) {
@@ -324,12 +380,18 @@ __global__ __launch_bounds__(kMThreads, ADJ && EX ? 3 : 6) void k_multi(const St
     float *__restrict__ vyo = a.vy_out + s0 * g.plane;
     float *__restrict__ sxo = a.sxy_out + s0 * g.plane;
     float *__restrict__ szo = a.syz_out + s0 * g.plane;
+    float *__restrict__ rqo = L > 0 ? a.rq + s0 * 2 * L * g.plane : nullptr;
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
         if (!own[i]) continue;
         vyo[off[i]] = v[i];
         sxo[off[i]] = sx[i];
         szo[off[i]] = sz[i];
+#pragma unroll
+        for (int l = 0; l + 1 < L; l += 2)
+            *(float4 *)(rqo + 2 * l * g.plane + 4 * (size_t)off[i]) =
+                make_float4(rr[i][l], qq[i][l], rr[i][l + 1], qq[i][l + 1]);
+        if (L & 1) *(float2 *)(rqo + 2 * (L - 1) * g.plane + 2 * (size_t)off[i]) = make_float2(rr[i][L - 1], qq[i][L - 1]);
         if (xk[i] > 0) {
             const long long o = s0 * g.ny * fw2 + (cj[i] - 1) * fw2 + (xk[i] - 1);
             a.psx_out[o] = px[i];
@@ -348,35 +410,34 @@ __global__ __launch_bounds__(kMThreads, ADJ && EX ? 3 : 6) void k_multi(const St
     }
 }
 
-template <int K> hipError_t launch_k(const StepArgs &a, bool adjoint, bool extra, hipStream_t st)
+template <int L> hipError_t launch_l(const StepArgs &a, bool adjoint, bool extra, hipStream_t st)
 {
+    constexpr int K = DN_MULTI_K;
     const dim3 grid((unsigned)(a.tl_nblk8 * 8)), block(kMThreads);
     if (adjoint) {
         if (extra)
-            hipLaunchKernelGGL((k_multi<K, true, true>), grid, block, 0, st, a);
+            hipLaunchKernelGGL((k_multi<K, L, true, true>), grid, block, 0, st, a);
         else
-            hipLaunchKernelGGL((k_multi<K, true, false>), grid, block, 0, st, a);
+            hipLaunchKernelGGL((k_multi<K, L, true, false>), grid, block, 0, st, a);
     } else {
         if (extra)
-            hipLaunchKernelGGL((k_multi<K, false, true>), grid, block, 0, st, a);
+            hipLaunchKernelGGL((k_multi<K, L, false, true>), grid, block, 0, st, a);
         else
-            hipLaunchKernelGGL((k_multi<K, false, false>), grid, block, 0, st, a);
+            hipLaunchKernelGGL((k_multi<K, L, false, false>), grid, block, 0, st, a);
     }
     return hipGetLastError();
 }
 
 }  // namespace
 
-int multi_tiles(int nx, int ny) { return ((nx + kMX - 1) / kMX) * ((ny + kMY - 1) / kMY); }
-int multi_steps(int K) { return steps_of(K); }
-int multi_tiles_y(int ny) { return (ny + kMY - 1) / kMY; }
-
-hipError_t launch_multi(const StepArgs &a, int K, bool adjoint, bool extra, hipStream_t st)
+template <> hipError_t launch_multi_k<DN_MULTI_K>(const StepArgs &a, bool adjoint, bool extra, hipStream_t st)
 {
-    if (a.g.L != 0 || a.ms_steps < 1 || a.ms_steps > multi_steps(K)) return hipErrorInvalidValue;
-    switch (K) {
-    case 1: return launch_k<1>(a, adjoint, extra, st);
-    case 2: return launch_k<2>(a, adjoint, extra, st);
+    if (a.ms_steps < 1 || a.ms_steps > multi_steps(DN_MULTI_K)) return hipErrorInvalidValue;
+    switch (a.g.L) {
+    case 0: return launch_l<0>(a, adjoint, extra, st);
+    case 1: return launch_l<1>(a, adjoint, extra, st);
+    case 2: return launch_l<2>(a, adjoint, extra, st);
+    case 3: return launch_l<3>(a, adjoint, extra, st);
     default: return hipErrorInvalidValue;
     }
 }

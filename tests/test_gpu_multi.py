@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from common import oracle, product
-from test_gpu_tile import _inputs, _run, say
+from test_gpu_tile import FL, _inputs, _run, say
 
 pytestmark = pytest.mark.gpu
 
@@ -52,4 +52,44 @@ def test_several_steps_equal_oracle(nx, ny, fdorder):
     cfg = make_cfg(nx, ny, fdorder=fdorder, fw=8, free_surf=0, L=0, nt=62, dtinv=2, dt=1e-4, dh=0.25, damping=300.0,
                    fpml=40.0, fl=[])
     ref = oracle("f32").gradient(cfg, vs, rho, None, si, sj, sig, ri, rj, obs)
+    assert np.array_equal(got[2], ref["grad_vs"]) and np.array_equal(got[3], ref["grad_rho"])
+
+
+@pytest.mark.parametrize("nx,ny,fdorder,L,free_surf,boundary,shots,dtinv,two", [
+    (48, 24, 4, 2, 0, 0, 1, 1, False),
+    (49, 25, 2, 3, 1, 0, 3, 2, True),
+    (97, 40, 6, 0, 0, 0, 3, 5, False),
+    (63, 33, 6, 3, 0, 0, 2, 3, True),
+    (71, 41, 8, 2, 0, 0, 2, 4, False),
+    (72, 40, 8, 1, 1, 0, 1, 3, False),
+    (130, 39, 8, 0, 0, 1, 2, 2, True),
+    (128, 47, 4, 1, 1, 1, 4, 2, False),
+    (24, 24, 8, 3, 0, 0, 1, 1, False),
+])
+def test_several_higher_order_and_viscoelastic_steps_equal_strips(nx, ny, fdorder, L, free_surf, boundary, shots, dtinv,
+                                                                  two):
+    say("several steps", nx, ny, "FDORDER", fdorder, "L", L, "shots", shots)
+    par = dict(nx=nx, ny=ny, fdorder=fdorder, L=L, free_surf=free_surf, boundary=boundary, snap=0, dtinv=dtinv, fw=8)
+    inp = list(_inputs(nx, ny, shots, 150, seed=nx + ny))
+    inp[8] = (150 - np.arange(shots)).astype(np.int32)
+    dn = product()
+    a = _run(dn, par, inp, 0, two)
+    b = _run(dn, par, inp, 13, two)
+    assert np.isfinite(a[2]).all() and np.abs(a[2]).max() > 0
+    for k, (x, y) in enumerate(zip(a, b)):
+        assert np.array_equal(x, y), "output %d differs" % k
+
+
+@pytest.mark.parametrize("nx,ny,fdorder,L", [(65, 33, 8, 2), (70, 41, 6, 1), (50, 30, 4, 3)])
+def test_several_viscoelastic_steps_equal_oracle(nx, ny, fdorder, L):
+    from pyoracle import make_cfg
+    say("several steps against the oracle", nx, ny, "FDORDER", fdorder, "L", L)
+    par = dict(nx=nx, ny=ny, fdorder=fdorder, L=L, free_surf=0, boundary=0, snap=0, dtinv=2, fw=8)
+    inp = list(_inputs(nx, ny, 2, 62, seed=3))
+    inp[8] = np.full(2, 62, np.int32)
+    vs, rho, qs, sig, si, sj, ri, rj, _, obs = inp
+    got = _run(product(), par, inp, 0, False)
+    cfg = make_cfg(nx, ny, fdorder=fdorder, fw=8, free_surf=0, L=L, nt=62, dtinv=2, dt=1e-4, dh=0.25, damping=300.0,
+                   fpml=40.0, fl=FL[:L])
+    ref = oracle("f32").gradient(cfg, vs, rho, qs, si, sj, sig, ri, rj, obs)
     assert np.array_equal(got[2], ref["grad_vs"]) and np.array_equal(got[3], ref["grad_rho"])
