@@ -48,13 +48,31 @@ __device__ __forceinline__ f4v mfma32(u8v a, u8v b, f4v c)
 // taps' weights are staged in LDS once, so the walk has no barrier.  One row
 // per workgroup, each row's weights staged and waited for and each input row
 // loaded for three output rows, took 118 us for 16 -> 16 channels at 800 x
-// 4000 and 168 us for 80 -> 32 at half of it; now 47 us (4.4 TB/s) and 79.
+// 4000 and 168 us for 80 -> 32 at half of it; now 47 us (4.4 TB/s) and 81.
 //
 // CAT: the input is the concatenation of an up-sampled tensor (CU channels at
 // half resolution, nearest) and a skip tensor, read from both where they are:
 // the concatenated copy (243 us per layer at 800 x 4000) is never written.
+// The groups stay in the order of the concatenated channels, so the sums round
+// as those over a concatenated copy; with all groups of one part first, without
+// the second loads, 48 -> 16 took 95 us instead of 105, but every activation
+// behind it may round to another bfloat16.
 // ---------------------------------------------------------------------------
 constexpr int cat_up(int CI) { return CI == 112 ? 64 : (CI == 80 ? 48 : 32); }
+// groups 4i..4i+3 of cb groups per tap, the first b0 of them up-sampled: does
+// MFMA i read up-sampled (up) or skip channels; how many MFMAs below n read both
+constexpr bool cat_reads(int i, int cb, int b0, bool up)
+{
+    for (int g = 4 * i; g < 4 * i + 4 && g < 3 * cb; ++g)
+        if ((g % cb < b0) == up) return true;
+    return false;
+}
+constexpr int cat_both(int n, int cb, int b0)
+{
+    int k = 0;
+    for (int i = 0; i < n; ++i) k += cat_reads(i, cb, b0, true) && cat_reads(i, cb, b0, false);
+    return k;
+}
 
 // One row of a tensor as a buffer resource: an offset outside [0, bytes)
 // reads zero and stores nothing, which is the convolution's padding, without
@@ -72,9 +90,9 @@ __global__ __launch_bounds__(256, 2) void k_conv3x3(ConvArgs a)
 {
     // the input's parts: the up-sampled and the skip tensor, or one tensor
     constexpr int C0 = CAT ? cat_up(CI) : CI, C1 = CI - C0;
-    constexpr int B0 = C0 / 8, B1 = C1 / 8;                          // 8-channel groups per tap
-    constexpr int N0 = (3 * B0 + 3) / 4, N1 = (3 * B1 + 3) / 4;      // MFMAs per kernel row
-    constexpr int NKI = N0 + N1;
+    constexpr int CB = CI / 8, B0 = C0 / 8;      // 8-channel groups per tap, of the first part
+    constexpr int NKI = (3 * CB + 3) / 4;        // MFMAs per kernel row
+    constexpr int N2 = cat_both(NKI, CB, B0);    // of them with groups of both parts
     constexpr int SW = 16 * NM + 1;     // LDS entries per group (+ 1 against bank conflicts)
     __shared__ u8v sw[3 * NKI * 4 * SW];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -86,13 +104,11 @@ __global__ __launch_bounds__(256, 2) void k_conv3x3(ConvArgs a)
     const int nmt = min(NM, (a.Co - cg) >> 4);
     for (int e = threadIdx.x; e < 3 * NKI * 4 * 16 * NM; e += 256) {
         const int co = e % (16 * NM), kg = e / (16 * NM);      // kg = ky * 4 NKI + group
-        const int ky = kg / (4 * NKI), gg = kg - ky * (4 * NKI);
-        const bool second = gg >= 4 * N0;
-        const int g = second ? gg - 4 * N0 : gg, cbs = second ? (B1 > 0 ? B1 : 1) : B0;
+        const int ky = kg / (4 * NKI), g = kg - ky * (4 * NKI);
         u8v v = u8v{0, 0, 0, 0, 0, 0, 0, 0};
-        if (g < 3 * cbs && cg + co < a.Co) {
-            const int kx = g / cbs, cb = g - kx * cbs;
-            v = *(const u8v *)(a.w + ((long long)(3 * ky + kx) * a.Co + cg + co) * CI + (second ? C0 : 0) + 8 * cb);
+        if (g < 3 * CB && cg + co < a.Co) {
+            const int kx = g / CB, cb = g - kx * CB;
+            v = *(const u8v *)(a.w + ((long long)(3 * ky + kx) * a.Co + cg + co) * CI + 8 * cb);
         }
         sw[kg * SW + co] = v;
     }
@@ -107,34 +123,32 @@ __global__ __launch_bounds__(256, 2) void k_conv3x3(ConvArgs a)
     __syncthreads();
     if (y0 >= y1) return;
 
-    // input fragment i, t of row yi (a group past the last tap: zero)
-    auto load = [&](int yi, int i, int t) -> u8v {
-        if (i < N0) {
-            const int g = 4 * i + kq, kx = g / B0, cb = g - kx * B0;
-            int px = x0 + 16 * t + nl + kx - 1;
-            const uint16_t *row;
-            int w;
-            if (CAT) {
-                w = a.W >> 1;
-                px >>= 1;                                  // -1 stays -1, W becomes W / 2
-                row = a.up + (long long)(img * (a.H >> 1) + (yi >> 1)) * w * C0;
-            } else {
-                w = a.W;
-                row = a.x + (long long)(img * a.H + yi) * w * C0;
-            }
-            int off = (px * C0 + 8 * cb) * 2;
-            if (4 * N0 > 3 * B0 && g >= 3 * B0) off = -16;
-            return __builtin_bit_cast(u8v, __builtin_amdgcn_raw_buffer_load_b128(row_rsrc(row, w * C0 * 2), off, 0, 0));
-        }
-        constexpr int CC = C1 > 0 ? C1 : 8, BB = CC / 8;
-        const int g = 4 * (i - N0) + kq, kx = g / BB, cb = g - kx * BB;
-        const int px = x0 + 16 * t + nl + kx - 1;
-        const uint16_t *row = a.x + (long long)(img * a.H + yi) * a.W * CC;
-        int off = (px * CC + 8 * cb) * 2;
-        if (4 * N1 > 3 * B1 && g >= 3 * BB) off = -16;
-        return __builtin_bit_cast(u8v, __builtin_amdgcn_raw_buffer_load_b128(row_rsrc(row, a.W * CC * 2), off, 0, 0));
+    // input fragment i, t of row yi: the groups of the one part; those of the
+    // other part and past the last tap read zero
+    auto load = [&](int yi, int i, int t, bool up) -> u8v {
+        const int g = 4 * i + kq, kx = g / CB, cb = g - kx * CB, px = x0 + 16 * t + nl + kx - 1;
+        const bool half = CAT && up;               // the part at half resolution
+        const int w = half ? a.W >> 1 : a.W, c = up ? C0 : C1;
+        const uint16_t *row = half ? a.up + (long long)(img * (a.H >> 1) + (yi >> 1)) * w * c
+                                   : a.x + (long long)(img * a.H + yi) * w * c;
+        // px >> 1: -1 stays -1, W becomes W / 2
+        int off = ((half ? px >> 1 : px) * c + 8 * (up ? cb : cb - B0)) * 2;
+        if (CAT && (cb < B0) != up) off = -16;
+        if (4 * NKI > 3 * CB && g >= 3 * CB) off = -16;
+        return __builtin_bit_cast(u8v, __builtin_amdgcn_raw_buffer_load_b128(row_rsrc(row, w * c * 2), off, 0, 0));
     };
-    u8v b[NKI][NT];
+    // An MFMA whose groups are of both parts takes the union of two loads: the
+    // sum keeps the order of the concatenated channels.
+    u8v b[NKI][NT], b2[N2 > 0 ? N2 : 1][NT];
+    auto fetch = [&](int yi, int i) {
+        const bool up = cat_reads(i, CB, B0, true);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) b[i][t] = load(yi, i, t, up);
+        if (up && cat_reads(i, CB, B0, false)) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) b2[cat_both(i, CB, B0)][t] = load(yi, i, t, false);
+        }
+    };
     f4v acc[3][NM][NT];
 #pragma unroll
     for (int q = 0; q < 3; ++q)
@@ -144,9 +158,7 @@ __global__ __launch_bounds__(256, 2) void k_conv3x3(ConvArgs a)
             for (int t = 0; t < NT; ++t) acc[q][m][t] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
     const int ya = max(y0 - 1, 0), yb = min(y1, a.H - 1);      // input rows
 #pragma unroll
-    for (int i = 0; i < NKI; ++i)
-#pragma unroll
-        for (int t = 0; t < NT; ++t) b[i][t] = load(ya, i, t);
+    for (int i = 0; i < NKI; ++i) fetch(ya, i);
 
     const int orow = a.W * a.Co * 2;                           // bytes of an output (or mask) row
     auto ooff = [&](int t, int m) -> int { return ((x0 + 16 * t + nl) * a.Co + cg + m * 16 + 4 * kq) * 2; };
@@ -200,6 +212,10 @@ __global__ __launch_bounds__(256, 2) void k_conv3x3(ConvArgs a)
         if (a.mask) masks(yi - 1, mk);
 #pragma unroll
         for (int i = 0; i < NKI; ++i) {
+            if (cat_reads(i, CB, B0, true) && cat_reads(i, CB, B0, false)) {
+#pragma unroll
+                for (int t = 0; t < NT; ++t) b[i][t] |= b2[cat_both(i, CB, B0)][t];
+            }
             auto mult = [&](int ky, f4v (&ac)[NM][NT]) {
                 const u8v *w = sw + (ky * 4 * NKI + 4 * i + kq) * SW + nl;
 #pragma unroll
@@ -213,8 +229,7 @@ __global__ __launch_bounds__(256, 2) void k_conv3x3(ConvArgs a)
             if (d0) mult(0, a0);
             if (d1) mult(1, a1);
             if (d2) mult(2, a2);
-#pragma unroll
-            for (int t = 0; t < NT; ++t) b[i][t] = load(yn, i, t);
+            fetch(yn, i);
         }
         if (d2) finish(yi - 1, a2, mk);
     };
@@ -275,7 +290,7 @@ hipError_t launch_conv3x3(const ConvArgs &a, hipStream_t st)
     case 484: conv_launch<48, 4, 2, false>(a, st); break;
     case 643: conv_launch<64, 3, 2, false>(a, st); break;
     case 644: conv_launch<64, 4, 2, false>(a, st); break;
-    case 10481: conv_launch<48, 1, 4, true>(a, st); break;
+    case 10481: conv_launch<48, 1, 2, true>(a, st); break;
     case 10802: conv_launch<80, 2, 2, true>(a, st); break;
     case 11121: conv_launch<112, 1, 2, true>(a, st); break;
     default: return hipErrorInvalidValue;
