@@ -15,11 +15,12 @@
 // fixed order; the reference accumulates Ebar in float.
 //
 // FFT: radix-2 decimation in time, a bit-reversal gather then log2(Npad)
-// butterfly stages over all traces at once, complex double.  The stages run
+// butterfly stages over kBatchPts points at once, complex double.  The stages run
 // in LDS, eight in the pass that gathers the traces and up to seven in each
 // pass after it: two passes over HBM instead of one per stage for 2^15
-// points, with the same butterflies.  240 traces of 5000 samples (Npad 2^15):
-// 32 launches of 20-38 us for the two transforms before, now four of about 75.
+// points, with the same butterflies.  The call for 240 traces of 5000 samples
+// (Npad 2^15): 2.67 ms with a pass per stage over all traces, 1.29 with these
+// over all traces (four launches of about 75 us), 1.03 in batches.
 #include "dn_core.h"
 
 #include <algorithm>
@@ -48,6 +49,13 @@ __global__ void k_twiddles(int N, cd *__restrict__ w)
 
 constexpr int kFirstBits = 8, kNextBits = 7;
 constexpr int kFirstPts = 512, kNextPts = 1024;   // points of a workgroup of 256 threads
+// points of the traces transformed together (at least one trace): 16 MB per
+// array, so the passes and the sums find them in the memory-side cache and a
+// call does not allocate the spectra of all traces (250 MB for 240 traces of
+// 5000 samples; memory that was freed before is cleared at some 40 GB/s when
+// it is allocated again, 7.4 ms per call after a thousand calls).  The call
+// with 2^18, 2^19, 2^20, 2^21 points: 1.52, 1.23, 1.03, 1.23 ms
+constexpr int kBatchPts = 1 << 20;
 
 __device__ inline void butterfly(cd &a, cd &b, cd w, int sign)
 {
@@ -162,15 +170,22 @@ __global__ void k_norm_ratio(int ntr, const float *mx_syn, const float *mx_obs, 
     if (i < ntr) ratio[i] = mx_syn[i] / mx_obs[i];
 }
 
-// S_n, S_d and the per-frequency share of Ebar (sum over the running sums)
-__global__ void k_wiener_sums(int ntr, int N, const cd *__restrict__ D, const cd *__restrict__ M, cd *__restrict__ sn,
+// S_n, S_d and the per-frequency share of Ebar (sum over the running sums);
+// n_all traces in all, ntr of them in D and M, behind those summed before
+// (more: some were)
+__global__ void k_wiener_sums(int n_all, int ntr, bool more, int N, const cd *__restrict__ D, const cd *__restrict__ M, cd *__restrict__ sn,
                               double *__restrict__ sd, double *__restrict__ erow)
 {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= N) return;
-    const double n = (double)ntr;
+    const double n = (double)n_all;
     cd a{0.0, 0.0};
     double d = 0.0, e = 0.0;
+    if (more) {
+        a = sn[k];
+        d = sd[k];
+        e = erow[k];
+    }
     auto add = [&](const cd &dd, const cd &mm) {
         const cd nd{n * dd.re, n * dd.im}, nm{n * mm.re, n * mm.im};
         const cd p = cmul(nd, cd{mm.re, -mm.im});
@@ -261,7 +276,7 @@ struct StfDev {
         if (mem) p = (T *)(mem + used);
         used += (n * sizeof(T) + 255) / 256 * 256;
     }
-    void layout(size_t ntr, size_t ns, size_t N)
+    void layout(size_t ntr, size_t ns, size_t N, size_t batch)
     {
         used = 0;
         take(obs, ntr * ns);
@@ -270,8 +285,8 @@ struct StfDev {
         take(stf, ns);
         take(mx, 4 * ntr);
         take(mute, ntr);
-        take(D, ntr * N);
-        take(M, ntr * N);
+        take(D, batch * N);
+        take(M, batch * N);
         take(S, N);
         take(sn, N);
         take(Y, N);
@@ -329,12 +344,13 @@ extern "C" int dn_stf(int ntr, int ns, const float *obs, const float *syn, const
     const int logN = (int)std::ceil(std::log((double)ns) / std::log(2.0)) + 2;
     if (logN > 26) return dn_fail(nullptr, "dn_stf: record too long");
     const int N = 1 << logN;
+    const int batch = std::max(1, std::min(ntr, kBatchPts / N));
     StfDev R;
     SCHK(hipStreamCreateWithFlags(&R.st, hipStreamNonBlocking));
     const size_t nd = (size_t)ntr * ns;
-    R.layout(ntr, ns, N);
+    R.layout(ntr, ns, N, batch);
     SCHK(hipMalloc((void **)&R.mem, R.used));
-    R.layout(ntr, ns, N);
+    R.layout(ntr, ns, N, batch);
     hipStream_t st = R.st;
     SCHK(hipMemcpyAsync(R.obs, obs, nd * sizeof(float), hipMemcpyHostToDevice, st));
     SCHK(hipMemcpyAsync(R.syn, syn, nd * sizeof(float), hipMemcpyHostToDevice, st));
@@ -360,10 +376,14 @@ extern "C" int dn_stf(int ntr, int ns, const float *obs, const float *syn, const
         }
     }
     hipLaunchKernelGGL(k_twiddles, dim3(blocks(N / 2)), dim3(256), 0, st, N, R.tw);
-    fft_traces(ntr, ns, logN, R.obs, R.mute, sc_obs, mul_obs, R.tw, R.D, st);
-    fft_traces(ntr, ns, logN, R.syn, R.mute, sc_syn, 0, R.tw, R.M, st);
     fft_traces(1, ns, logN, R.sig, nullptr, nullptr, 0, R.tw, R.S, st);
-    hipLaunchKernelGGL(k_wiener_sums, dim3(blocks(N)), dim3(256), 0, st, ntr, N, R.D, R.M, R.sn, R.sd, R.erow);
+    for (int i = 0; i < ntr; i += batch) {
+        const int n = std::min(batch, ntr - i);
+        fft_traces(n, ns, logN, R.obs + (size_t)i * ns, R.mute + i, sc_obs ? sc_obs + i : nullptr, mul_obs, R.tw, R.D, st);
+        fft_traces(n, ns, logN, R.syn + (size_t)i * ns, R.mute + i, sc_syn ? sc_syn + i : nullptr, 0, R.tw, R.M, st);
+        hipLaunchKernelGGL(k_wiener_sums, dim3(blocks(N)), dim3(256), 0, st, ntr, n, i > 0, N, R.D, R.M, R.sn, R.sd,
+                           R.erow);
+    }
     hipLaunchKernelGGL(k_sum_fixed, dim3(1), dim3(256), 0, st, N, R.erow, R.esum);
     hipLaunchKernelGGL(k_eps, dim3(1), dim3(1), 0, st, R.esum, N, ntr, o->eps_stf, R.esum + 1);
     hipLaunchKernelGGL(k_wiener_div, dim3(blocks(N)), dim3(256), 0, st, N, logN, R.S, R.sn, R.sd, R.esum + 1, R.Y);

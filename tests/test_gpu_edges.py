@@ -83,3 +83,21 @@ def test_stf_passes(ntr, ns):
     got = product().stf(obs, syn, sig, eps_stf=0.05)
     want = stf_oracle.stf(obs, syn, sig, eps_stf=0.05)
     assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("ntr,ns,normalize", [(33, 5000, 0), (64, 5000, 1), (65, 4100, 2), (3, 140000, 2)])
+def test_stf_batches(ntr, ns, normalize):
+    """32 traces of 2^15 points to a batch, or one of 2^20: remainders of one
+    trace, none, and muted traces on both sides of a batch's edge.  The bound
+    is test_stf_passes'."""
+    import stf_oracle
+    say("stf batches", ntr, ns, normalize)
+    rng = np.random.default_rng(ns + ntr)
+    syn = rng.standard_normal((ntr, ns)).astype(np.float32)
+    obs = (0.7 * syn + 0.3 * rng.standard_normal((ntr, ns))).astype(np.float32)
+    sig = rng.standard_normal(ns).astype(np.float32)
+    mute = np.zeros(ntr, np.uint8)
+    mute[[1, min(31, ntr - 1)]] = 1
+    got = product().stf(obs, syn, sig, mute=mute, eps_stf=0.05, normalize=normalize)
+    want = stf_oracle.stf(obs, syn, sig, mute=mute, eps_stf=0.05, normalize=normalize)
+    assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
