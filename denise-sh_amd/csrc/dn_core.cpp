@@ -922,10 +922,27 @@ void dn_fill_step_common(dn_ctx *c, StepArgs &a, int n)
         a.tl_w = kWave;
         a.tl_h = 8 * a.tl_rw;
         a.tl_ny = (g.ny + a.tl_h - 1) / a.tl_h;
-        a.tl_nblk = n * ((g.nx + a.tl_w - 1) / a.tl_w) * a.tl_ny;
-        a.tl_nblk8 = (a.tl_nblk + 7) / 8;
-        a.tl_mshots = 0xffffffffu / (unsigned)n;
-        a.tl_mny = 0xffffffffu / (unsigned)a.tl_ny;
+        // Order of the tiles (k_tile): more shots share a tile's coefficients,
+        // fewer keep its neighbours in reach.  Groups of 2, 3, 4, all shots:
+        // 1200x300, 4 shots 22.9 22.4 22.1 22.1 ms; 24 shots (Gcell-updates/s)
+        // 57.2 57.3 56.8 54.3; 1973x397x6 uneven 81.8 76.2 84.2 80.4 ms;
+        // 2000x400x9 56.6 56.9 56.2 55.5; 4000x800x4 61.4 60.5 62.1 61.9
+        const int tnx = (g.nx + a.tl_w - 1) / a.tl_w;
+        a.tl_tiles = tnx * a.tl_ny;
+        a.tl_grp = n <= 4 ? n : 3;
+        a.tl_full = n / a.tl_grp;
+        a.tl_last = std::max(1, n % a.tl_grp);
+        a.tl_g8 = (a.tl_grp * a.tl_tiles + 7) / 8;
+        a.tl_l8 = (a.tl_last * a.tl_tiles + 7) / 8;
+        a.tl_nblk8 = a.tl_full * a.tl_g8 + (n % a.tl_grp ? a.tl_l8 : 0);
+        a.tl_mgrp = 0xffffffffu / (unsigned)a.tl_grp;
+        a.tl_mlast = 0xffffffffu / (unsigned)a.tl_last;
+        a.tl_mg8 = 0xffffffffu / (unsigned)a.tl_g8;
+        a.tl_bblk = 8 * a.tl_ny;
+        a.tl_bfull = tnx / 8;
+        a.tl_blast = std::max(1, tnx % 8);
+        a.tl_mbblk = 0xffffffffu / (unsigned)a.tl_bblk;
+        a.tl_mblast = 0xffffffffu / (unsigned)a.tl_blast;
     }
     a.DT = c->p.dt;
     a.DH = c->p.dh;

@@ -86,7 +86,10 @@ struct StepArgs {
     int tl_w, tl_h;                // columns and rows of a tile
     int tl_ny;                     // tiles in a column of tiles
     int tl_nblk, tl_nblk8;         // tiles of all shots, and per XCD slice
-    unsigned tl_mshots, tl_mny;    // (2^32 - 1) / nshots, (2^32 - 1) / tl_ny
+    int tl_grp, tl_full, tl_last;  // shots of a group, full groups, shots of the last group where it is not full
+    int tl_tiles, tl_g8, tl_l8;    // tiles of a shot; tiles of an XCD in a full and in the last group
+    int tl_bblk, tl_bfull, tl_blast;   // tiles of a band of eight columns of tiles, such bands, columns of the last
+    unsigned tl_mgrp, tl_mlast, tl_mg8, tl_mbblk, tl_mblast;   // (2^32 - 1) / tl_grp, tl_last, tl_g8, tl_bblk, tl_blast
     Geo g;
     // per-shot dynamic state; shot stride = plane (2*L*plane for rq)
     const float *vy_in, *sxy_in, *syz_in;

@@ -29,6 +29,21 @@
 // two rows 41.7 / 117, of four rows 45.3 / 118; eight of four rows 47 / 125;
 // 128 columns, 4 x 2 waves of two rows 50 / 126; sixteen waves 63 / 151.
 //
+// Order of the tiles.  A tile reads 2K-1 columns of its neighbours on each
+// side, a whole line per row for each, and where the fields exceed the
+// memory-side cache that is HBM traffic unless the neighbour ran just before.
+// With all shots of a tile in turn and the tiles down a column, the next
+// column was a column of tiles times all shots away; now groups of three
+// shots (all up to four), an eighth of each group's tiles to each XCD, bands
+// of eight columns of tiles, row by row.  Gcell-updates/s of the gradient
+// (strips, one box; then down a column, now, another): 1200 x 300 with 24
+// shots 55.8; 51.0, 57.3; with 16 50.9; 54.1, 57.6; 2000 x 400 with 9 55.8;
+// 54.2, 56.9; 4000 x 800 with 2 56.8; 57.8, 60.2, with 4 57.4; 58.7, 62.1.
+// Bands of 4, 8, 16 columns (pairs of shots): 1200 x 300 with 24 shots 56.9
+// 56.9 56.5, 2000 x 400 with 9 56.2 57.2 57.3, 4000 x 800 with 2 59.8 60.2
+// 60.2.  Whole groups to one XCD leave XCDs idle once a group's records end
+// (1973 x 397, six uneven shots, 89.8 ms against 81.8 for pairs).
+//
 // Old and new vy, sxy, syz and the velocity CPML memory are separate buffers
 // (ping-pong), so the reads of the cells around a tile never race with their
 // owners' writes; the stress CPML and the relaxation memory variables are
@@ -108,13 +123,18 @@ __global__ __launch_bounds__(kWave *WX *WY) void k_tile(const StepArgs a)
     __shared__ float lz[NZ * VP];         // (j0-(2K-1).., c0-(K-1)..)
     __shared__ float lv[NV * VP];         // (j0-(K-1).., c0-(K-1)..)
 
-    const int w_ = blockIdx.x;
-    const int lin = (w_ & 7) * a.tl_nblk8 + (w_ >> 3);
-    if (lin >= a.tl_nblk) return;
-    // the shots of a tile next to each other (they share its static fields
-    // in the XCD's L2), then the tiles down a column of tiles
-    const int tile = udiv(lin, a.nshots, a.tl_mshots), s = lin - tile * a.nshots;
-    const int bx = udiv(tile, a.tl_ny, a.tl_mny), by = tile - bx * a.tl_ny;
+    // order: groups of shots, an eighth of each group's tiles to each XCD, and
+    // in a group bands of eight columns of tiles, in a band row by row, each
+    // tile for all shots of the group
+    const int w_ = blockIdx.x, grp = udiv(w_ >> 3, a.tl_g8, a.tl_mg8);
+    const bool full = grp < a.tl_full;
+    const int gs = full ? a.tl_grp : a.tl_last;
+    const int gl = (w_ & 7) * (full ? a.tl_g8 : a.tl_l8) + (w_ >> 3) - grp * a.tl_g8;
+    if (gl >= gs * a.tl_tiles) return;
+    const int tile = udiv(gl, gs, full ? a.tl_mgrp : a.tl_mlast), s = grp * a.tl_grp + gl - tile * gs;
+    const int band = udiv(tile, a.tl_bblk, a.tl_mbblk), bl = tile - band * a.tl_bblk;
+    const bool wide = band < a.tl_bfull;
+    const int by = wide ? bl >> 3 : udiv(bl, a.tl_blast, a.tl_mblast), bx = 8 * band + bl - by * (wide ? 8 : a.tl_blast);
     const Geo &g = a.g;
     const ShotSlot sl = a.slots[s];
     const int nt = *a.nt_base + a.nt;

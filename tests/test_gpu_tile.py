@@ -107,3 +107,19 @@ def test_tiles_equal_oracle(nx, ny, fdorder, L, shots):
                    fpml=40.0, fl=FL[:L])
     ref = oracle("f32").gradient(cfg, vs, rho, qs if L else None, si, sj, sig, ri, rj, obs)
     assert np.array_equal(got[2], ref["grad_vs"]) and np.array_equal(got[3], ref["grad_rho"])
+
+
+@pytest.mark.parametrize("nx,ny,fdorder,L,shots,dtinv", [
+    (512, 33, 10, 0, 1, 2),     # one band of eight columns of tiles, one shot
+    (513, 40, 8, 2, 3, 3),      # a band and one column, a pair of shots and one
+    (600, 40, 8, 2, 4, 2),      # a band and two columns, two pairs
+    (960, 35, 10, 1, 5, 4),     # a band and seven columns
+    (1088, 60, 12, 2, 2, 3),    # two bands and one column
+])
+def test_order_of_tiles_equals_strips(nx, ny, fdorder, L, shots, dtinv):
+    say("order of the tiles", nx, ny, "FDORDER", fdorder, "shots", shots)
+    par = dict(nx=nx, ny=ny, fdorder=fdorder, L=L, free_surf=1, boundary=0, snap=0, dtinv=dtinv, fw=8)
+    inp = _inputs(nx, ny, shots, 70, seed=nx + ny)
+    dn = product()
+    for x, y in zip(_run(dn, par, inp, 0, False), _run(dn, par, inp, 13, False)):
+        assert np.array_equal(x, y)
