@@ -244,7 +244,7 @@ def cpu_baseline(W, seconds):
 
 
 def traffic_file(W):
-    return os.path.join(ROOT, "profiles", "k_step_visco_gradient_%dx%d_hbm_traffic.md" % (W["nx"], W["ny"]))
+    return os.path.join(ROOT, "profiles", "k_tile_visco_gradient_%dx%d_hbm_traffic.md" % (W["nx"], W["ny"]))
 
 
 def measured_traffic(W, batch, cells_per_launch):
@@ -595,8 +595,9 @@ def main():
     wall = time.perf_counter() - t0
     cells = float(ce[0] + ce[1])
     value = cells / wall / 1e9
-    # dominant kernel: the fused step kernel k_step (all but a fraction of a
-    # percent of the GPU time), over the launches of both passes: the
+    # dominant kernel: the fused step (all but a fraction of a percent of the
+    # GPU time; k_tile, or k_step where a launch shape of the strips is asked
+    # for), over the launches of both passes: the
     # forward pass moves 84 + 20/DTINV bytes per cell-update, the adjoint
     # 84 + 36/DTINV (14/DTINV and 30/DTINV with 16-bit snapshots)
     nla = max(la[0] + la[1], 1)
@@ -608,7 +609,9 @@ def main():
     bytes_per_cell = (ce[0] * b_fwd + ce[1] * b_adj) / max(ce[0] + ce[1], 1)
     achieved = units_per_launch * bytes_per_cell / (per_launch_ms * 1e-3) / 1e9
     full = W["nt"] == (12000 if args.config == "c4" else 10000)
-    traffic = measured_traffic(W, batch, units_per_launch) if (prec == 0 and full) else None
+    shape = ctx.launch_shape()
+    tiles = shape[0] == 0 and shape[2] == 1 and shape[3] == 1
+    traffic = measured_traffic(W, batch, units_per_launch) if (prec == 0 and full and tiles) else None
     out = {
         "metric": "Gcell-updates/s fwd+adj",
         "value": round(value, 3),
@@ -629,7 +632,8 @@ def main():
                    else "gradient over all %d shots" % nshots},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "kernel": "k_step<4,visco> (forward and adjoint launches of the gradient)",
+                     "kernel": "%s<4,visco> (forward and adjoint launches of the gradient)"
+                     % ("k_tile" if tiles else "k_step"),
                      "ms_per_launch": round(per_launch_ms, 4), "bytes_per_cell_update": round(bytes_per_cell, 3),
                      "cell_updates_per_launch": units_per_launch},
         "misfit_l2": l2,

@@ -8,8 +8,8 @@
 // smooth2.  Every x system (one per grid row) and every z system (one per
 // column) has the same matrix, so the host factors the two matrices once
 // with tripd's float operations (util.c:638-671) and the device runs only
-// the substitutions: one thread per row for x, then one per column for z,
-// in tripd's order.  The reference's index ranges are kept: its gradient
+// the substitutions, row by row for x, then column by column for z, in
+// tripd's order, from chunks staged in LDS (k_smooth2_x, k_smooth2_z).  The reference's index ranges are kept: its gradient
 // sits at v[1..NX][1..NY] of a zeroed v[0..NX][0..NY] and it smooths over
 // 0..n-1, so the zero row and column take part and the last row and
 // column keep their values.
@@ -17,10 +17,10 @@
 // Gaussian smoothing.  Each cell's half widths (hx, hz) follow its local
 // wavelength vs / FC_END; its kernel weights exp(-ii^2/sx - jj^2/sz) depend
 // only on (hx, hz).  The device turns the vs model into a per-cell index of
-// the distinct (hx, hz) pairs; the host builds one weight table per pair with
-// the same float operands, the double exp() rounded to float and the same
-// sequential float sum as the reference, so the weights and their sums are
-// bit-identical to it.  The device then sums gradient x weight per cell in
+// the distinct (hx, hz) pairs (k_gauss_plan); the host builds one weight table
+// per pair with the same float operands, the double exp() rounded to float and
+// the same sequential float sum as the reference, so the weights and their
+// sums are bit-identical to it.  The device then sums gradient x weight per cell in
 // the reference's order (x offset outer, y offset inner; unfused float
 // multiply and add) with clamped indices, which is the reference's edge
 // continuation of the gradient (gauss_filt_var.c:126-157), and divides by

@@ -14,8 +14,8 @@
  *
  *  2. A handle API (dn_*) for the fast path: the model, acquisition and
  *     per-shot data stay resident in HBM, many shots advance together in one
- *     launch per time step, and only scalars and requested results cross the
- *     boundary.
+ *     launch per time step (or per few steps on small grids), and only
+ *     scalars and requested results cross the boundary.
  *
  * Conventions: grid indices are 1-based like the reference (i = x, j = y,
  * y pointing down).  Host 2-D arrays in the handle API are row-major
@@ -351,7 +351,8 @@ int dn_last_timing(dn_ctx *ctx, double *ms_steps, long long *launches, long long
 
 /* Same, split by pass: adjoint = 0 forward passes, 1 adjoint passes.  ms is
  * measured with HIP events on the library's stream around each pass's
- * time-step launches; launches counts fused step launches. */
+ * time-step launches; launches counts fused step launches (one for
+ * several steps on small grids). */
 int dn_pass_timing(dn_ctx *ctx, int adjoint, double *ms, long long *launches, long long *cell_updates);
 
 /* ------------------------------------------------------------------------
