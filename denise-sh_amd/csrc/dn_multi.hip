@@ -165,9 +165,11 @@ __global__ __launch_bounds__(kMThreads, L == 0 && K <= 2 && !(ADJ && EX) ? 6 : 3
     if (tpy) {
         for (int e = threadIdx.x; e < 6 * HT; e += kMThreads) {
             const int f = e / HT, j = j0 - M + (e - f * HT);
+            // no top frame under a free surface: its rows may be the bottom frame's (NY < 2 FW)
+            const bool top = !g.free_surf && j <= fw;
             // Q2: the viscoelastic stress uses the full-grid y profile on top
-            const int fp = (L > 0 && f >= 3 && !g.free_surf && j <= fw) ? f + 3 : f + 6;
-            lky[e] = pmlb[fp * pn + min(max(j <= fw ? j : j - g.ny + fw2, 0), fw2)];
+            const int fp = (L > 0 && f >= 3 && top) ? f + 3 : f + 6;
+            lky[e] = pmlb[fp * pn + min(max(top ? j : j - g.ny + fw2, 0), fw2)];
         }
     }
     // the gradient sums of the owned cells stay in registers over the steps

@@ -93,3 +93,37 @@ def test_several_viscoelastic_steps_equal_oracle(nx, ny, fdorder, L):
                    fpml=40.0, fl=FL[:L])
     ref = oracle("f32").gradient(cfg, vs, rho, qs, si, sj, sig, ri, rj, obs)
     assert np.array_equal(got[2], ref["grad_vs"]) and np.array_equal(got[3], ref["grad_rho"])
+
+
+# ny below 2 FW under a free surface: the bottom frame reaches rows that would
+# belong to the top one if there were one
+SHALLOW = [(64, 12, 4, 0), (64, 15, 4, 2), (49, 8, 2, 0), (70, 15, 8, 2), (65, 12, 6, 1), (47, 16, 8, 3), (130, 9, 2, 3)]
+
+
+@pytest.mark.parametrize("nx,ny,fdorder,L", SHALLOW)
+def test_several_steps_of_shallow_free_surface_grids_equal_strips(nx, ny, fdorder, L):
+    say("several steps, shallow", nx, ny, "FDORDER", fdorder, "L", L)
+    par = dict(nx=nx, ny=ny, fdorder=fdorder, L=L, free_surf=1, boundary=0, snap=0, dtinv=2, fw=8)
+    inp = list(_inputs(nx, ny, 2, 90, seed=nx + ny))
+    inp[8] = np.array([90, 89], np.int32)
+    dn = product()
+    a = _run(dn, par, inp, 0, False)
+    b = _run(dn, par, inp, 13, False)
+    assert np.isfinite(a[2]).all() and np.abs(a[2]).max() > 0
+    for k, (x, y) in enumerate(zip(a, b)):
+        assert np.array_equal(x, y), "output %d differs" % k
+
+
+@pytest.mark.parametrize("nx,ny,fdorder,L", SHALLOW)
+def test_several_steps_of_shallow_free_surface_grids_equal_oracle(nx, ny, fdorder, L):
+    from pyoracle import make_cfg
+    say("several steps against the oracle, shallow", nx, ny, "FDORDER", fdorder, "L", L)
+    par = dict(nx=nx, ny=ny, fdorder=fdorder, L=L, free_surf=1, boundary=0, snap=0, dtinv=2, fw=8)
+    inp = list(_inputs(nx, ny, 2, 62, seed=3))
+    inp[8] = np.full(2, 62, np.int32)
+    vs, rho, qs, sig, si, sj, ri, rj, _, obs = inp
+    got = _run(product(), par, inp, 0, False)
+    cfg = make_cfg(nx, ny, fdorder=fdorder, fw=8, free_surf=1, L=L, nt=62, dtinv=2, dt=1e-4, dh=0.25, damping=300.0,
+                   fpml=40.0, fl=FL[:L])
+    ref = oracle("f32").gradient(cfg, vs, rho, qs if L else None, si, sj, sig, ri, rj, obs)
+    assert np.array_equal(got[2], ref["grad_vs"]) and np.array_equal(got[3], ref["grad_rho"])
