@@ -101,3 +101,17 @@ def test_stf_batches(ntr, ns, normalize):
     got = product().stf(obs, syn, sig, mute=mute, eps_stf=0.05, normalize=normalize)
     want = stf_oracle.stf(obs, syn, sig, mute=mute, eps_stf=0.05, normalize=normalize)
     assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("nx,ny", [
+    # unknowns of a row: 511, 512, 513, 528, 1024, 1099 (chunks of 512; last
+    # chunks of 511, 512, 1, 16, 512 and 75)
+    (512, 18), (513, 5), (514, 17), (529, 34), (1025, 3), (1100, 20),
+    # unknowns of a column: 127, 128, 129, 257 (chunks of 128)
+    (70, 128), (65, 129), (66, 130), (129, 258),
+])
+def test_smooth2_carries_between_chunks(nx, ny):
+    say("smooth2, several chunks", nx, ny)
+    g = np.random.default_rng(nx * ny).standard_normal((ny, nx)).astype(np.float32)
+    for wd in (1.5, 11.0):
+        assert np.array_equal(bits(product().smooth2(g, wd)), bits(O32.smooth2(g, wd)))
