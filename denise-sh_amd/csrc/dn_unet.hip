@@ -97,10 +97,10 @@ __global__ __launch_bounds__(256, 2) void k_conv3x3(ConvArgs a)
     __shared__ u8v sw[3 * NKI * 4 * SW];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int nl = lane & 15, kq = lane >> 4;
-    const int img = blockIdx.y / a.hblocks, hb = blockIdx.y - img * a.hblocks;
+    const int strip = blockIdx.x / a.cols, img = strip / a.hblocks, hb = strip - img * a.hblocks;
     const int y0 = (hb * 4 + wave) * a.rows, y1 = min(y0 + a.rows, a.H);   // output rows of the wave
-    const int x0 = blockIdx.x * (16 * NT);
-    const int cg = blockIdx.z * (16 * NM);
+    const int x0 = (blockIdx.x - strip * a.cols) * (16 * NT);
+    const int cg = blockIdx.y * (16 * NM);
     const int nmt = min(NM, (a.Co - cg) >> 4);
     for (int e = threadIdx.x; e < 3 * NKI * 4 * 16 * NM; e += 256) {
         const int co = e % (16 * NM), kg = e / (16 * NM);      // kg = ky * 4 NKI + group
@@ -267,7 +267,8 @@ template <int CI, int NM, int NT, bool CAT> static void conv_launch(ConvArgs a, 
     while (R > 2 && (long long)cols * z * a.n * ((a.H + 4 * R - 1) / (4 * R)) < 1024) R /= 2;
     a.rows = R;
     a.hblocks = (a.H + 4 * R - 1) / (4 * R);
-    hipLaunchKernelGGL((k_conv3x3<CI, NM, NT, CAT>), dim3((unsigned)cols, (unsigned)(a.n * a.hblocks), (unsigned)z),
+    a.cols = cols;
+    hipLaunchKernelGGL((k_conv3x3<CI, NM, NT, CAT>), dim3((unsigned)cols * (unsigned)(a.n * a.hblocks), (unsigned)z),
                        dim3(256), 0, st, a);
 }
 
@@ -579,8 +580,9 @@ hipError_t launch_wgrad(WgradArgs a, float *dw, float *db, hipStream_t st)
 // ---------------------------------------------------------------------------
 // 2x2 average pooling and the adjoints of pooling and nearest upsampling with
 // the ReLU mask of the activation they feed.  Bytes only: one thread per 8
-// channels of a pixel (16-byte accesses), one image row per blockIdx.y, so
-// the only division is by the channel count, a constant.
+// channels of a pixel (16-byte accesses), one image row per blockIdx.x, so
+// the only division is by the channel count, a constant (a batch may have more
+// rows than the 65536 workgroups that y and z of a grid take).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void unpack8(const uint16_t *p, float (&f)[8])
 {
@@ -592,10 +594,10 @@ __device__ __forceinline__ void unpack8(const uint16_t *p, float (&f)[8])
 template <int C> __global__ void k_pool(int H, int W, const uint16_t *x, uint16_t *y)
 {
     constexpr int C8 = C / 8;
-    const int w = W / 2, e = blockIdx.x * blockDim.x + threadIdx.x;
+    const int w = W / 2, e = blockIdx.y * blockDim.x + threadIdx.x;
     if (e >= w * C8) return;
     const int xo = e / C8, c = 8 * (e - xo * C8);
-    const long long row = blockIdx.y;                     // image * H/2 + y
+    const long long row = blockIdx.x;                     // image * H/2 + y
     const uint16_t *b = x + ((2 * row * W + 2 * xo) * C + c);
     float p[8], q[8], r[8], t[8];
     unpack8(b, p);
@@ -614,10 +616,10 @@ __global__ void k_pool_bwd(int H, int W, const uint16_t *dpool, const uint16_t *
                            const uint16_t *act, uint16_t *dact)
 {
     constexpr int C8 = C / 8;
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    const int e = blockIdx.y * blockDim.x + threadIdx.x;
     if (e >= W * C8) return;
     const int x = e / C8, c = 8 * (e - x * C8);
-    const long long row = blockIdx.y, p = row * W + x;    // row: image * H + y
+    const long long row = blockIdx.x, p = row * W + x;    // row: image * H + y
     const long long img = row / H, yl = (row - img * H) / 2;
     float dp[8], dc[8], ac[8];
     unpack8(dpool + ((img * (H / 2) + yl) * (W / 2) + x / 2) * C + c, dp);
@@ -634,10 +636,10 @@ template <int CU>
 __global__ void k_up_bwd(int H, int W, int Ccat, const uint16_t *dcat, const uint16_t *act_low, uint16_t *dlow)
 {
     constexpr int C8 = CU / 8;
-    const int w = W / 2, e = blockIdx.x * blockDim.x + threadIdx.x;
+    const int w = W / 2, e = blockIdx.y * blockDim.x + threadIdx.x;
     if (e >= w * C8) return;
     const int xo = e / C8, c = 8 * (e - xo * C8);
-    const long long row = blockIdx.y;                     // image * H/2 + y
+    const long long row = blockIdx.x;                     // image * H/2 + y
     const uint16_t *b = dcat + ((2 * row * W + 2 * xo) * Ccat + c);
     const long long q = (row * w + xo) * CU + c;
     float p0[8], p1[8], p2[8], p3[8], ac[8];
@@ -657,7 +659,7 @@ static dim3 grid_for(long long total)
     return dim3((unsigned)std::max<long long>(1, std::min<long long>(8192, (total + 255) / 256)));
 }
 
-static dim3 row_grid(int items, long long rows) { return dim3((unsigned)((items + 255) / 256), (unsigned)rows); }
+static dim3 row_grid(int items, long long rows) { return dim3((unsigned)rows, (unsigned)((items + 255) / 256)); }
 
 hipError_t launch_pool(int n, int H, int W, int C, const uint16_t *x, uint16_t *y, hipStream_t st)
 {
@@ -699,10 +701,11 @@ hipError_t launch_up_bwd(int n, int H, int W, int Cu, int Ccat, const uint16_t *
 // Input packing, output extraction, loss, parameter casts and Adam
 // ---------------------------------------------------------------------------
 // x [n][3][H][W] fp32 (planar) -> [n][H][W][16] bf16 with channels 3..15
-// zero: one pixel per thread
-__global__ void k_pack_input(long long hw, const float *x, uint16_t *xp)
+// zero: one pixel per thread, nb workgroups per image
+__global__ void k_pack_input(unsigned nb, long long hw, const float *x, uint16_t *xp)
 {
-    const long long r = blockIdx.x * (long long)blockDim.x + threadIdx.x, im = blockIdx.y;
+    const unsigned im = blockIdx.x / nb;
+    const long long r = (blockIdx.x - im * nb) * (long long)blockDim.x + threadIdx.x;
     if (r >= hw) return;
     const float *b = x + im * 3 * hw + r;
     const u8v z = u8v{0, 0, 0, 0, 0, 0, 0, 0};
@@ -773,7 +776,8 @@ __global__ void k_adam(long long n, float *w, const float *g, float *m, float *v
 hipError_t launch_pack_input(int n, int H, int W, const float *x, uint16_t *xp, hipStream_t st)
 {
     const long long hw = (long long)H * W;
-    hipLaunchKernelGGL(k_pack_input, dim3((unsigned)((hw + 255) / 256), (unsigned)n), dim3(256), 0, st, hw, x, xp);
+    const unsigned nb = (unsigned)((hw + 255) / 256);
+    hipLaunchKernelGGL(k_pack_input, dim3(nb * (unsigned)n), dim3(256), 0, st, nb, hw, x, xp);
     return hipGetLastError();
 }
 hipError_t launch_mse(long long P, const float *y, const float *t, uint16_t *dy, double *part, int nblocks,

@@ -70,3 +70,24 @@ def test_unet_strips_of_several_rows(n, h, w):
         sl = slice(wo[l], bo[l] + co)
         if np.max(np.abs(gr[sl])) > 0:
             assert rel_l2(g[sl], gr[sl]) < 5e-2, l
+
+
+@pytest.mark.parametrize("copies", [512, 1024])
+def test_unet_batches_of_many_rows(copies):
+    """More image rows than the 65536 workgroups of a grid's second dimension:
+    69632 and 139264, half of them after pooling.  A batch of copies of 17
+    images gives their outputs' bits and, the scale 2 / pixels being a power
+    of two smaller, their gradient up to the fp32 sums over the partials: at
+    most 17408 / 4 terms one after the other, 2.6e-4 of the terms' magnitude."""
+    print("unet, many rows", copies)
+    sys.stdout.flush()
+    net = product().UNet(seed=3)
+    rng = np.random.default_rng(25)
+    x = rng.standard_normal((17, 3, 8, 8)).astype(np.float32)
+    t = (0.5 * x[:, 0] - 0.3 * x[:, 1]).astype(np.float32)
+    y, (loss, g) = net.forward(x), net.loss_grad(x, t)
+    xs, ts = np.tile(x, (copies, 1, 1, 1)), np.tile(t, (copies, 1, 1))
+    assert np.array_equal(net.forward(xs), np.tile(y, (copies, 1, 1)))
+    ls, gs = net.loss_grad(xs, ts)
+    assert abs(ls - loss) <= 1e-6 * loss
+    assert rel_l2(gs, g) < 1e-3
