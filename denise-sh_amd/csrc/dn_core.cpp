@@ -214,7 +214,7 @@ static void free_batch(dn_ctx *c)
     dfree_t(c->d_Ws); dfree_t(c->d_Wr); dfree_t(c->d_gu_shot); dfree_t(c->d_grho_shot); dfree_t(c->d_part);
     dfree_t(c->d_shot_map); dfree_t(c->d_slots);
     c->cur_map.clear();   // the shot map must be uploaded again into the new workspace
-    c->batch_cap = 0;
+    c->batch_cap = c->multi_cap = 0;
     c->batch_nt_max = 0;
     // allocated after the workspace, from what it leaves
     dfree_t(c->d_terms);
@@ -732,8 +732,9 @@ static int multi_tiles(const dn_ctx *c)
 {
     return ((c->g.nx + kMultiX - 1) / kMultiX) * ((c->g.ny + kMultiY - 1) / kMultiY);
 }
-// some pass over one shot can use it: the batch holds the second halves
-static bool multi_capable(const dn_ctx *c) { return multi_tiles(c) <= multi_limit(c, false); }
+// the most shots of a pass that can use it: the batch holds second halves of
+// the relaxation variables and the stress CPML memory for so many
+static int multi_shots(const dn_ctx *c) { return multi_limit(c, false) / multi_tiles(c); }
 
 int dn_nsnap(const dn_ctx *c) { return (c->nt_max + c->p.dtinv - 1) / c->p.dtinv; }
 
@@ -742,8 +743,8 @@ static size_t per_shot_bytes(const dn_ctx *c, bool gradient)
 {
     const Geo &g = c->g;
     const size_t P = (size_t)g.plane, nxny = (size_t)g.nx * g.ny;
-    size_t b = 6 * P * 4 + (multi_capable(c) ? 4 : 2) * (size_t)g.L * P * 4;   // vy,sxy,syz x2, r, q
-    b += (size_t)(2 * 2 + 2) * (size_t)(2 * g.fw) * (g.nx + g.ny) * 4;  // psi, at least as many as there are
+    size_t b = 6 * P * 4 + 2 * (size_t)g.L * P * 4;                 // vy,sxy,syz x2, r, q
+    b += (size_t)(2 * 2 + 2) * (size_t)(2 * g.fw) * (g.nx + g.ny) * 4;  // psi, second halves included
     b += 2 * (size_t)c->ntr * c->nt_max * 4;                        // seis + resid
     b += 4 * nxny * 4 + (size_t)c->ntr * 16;                        // Ws, Wr, gu, grho, partials
     if (gradient) {
@@ -771,7 +772,13 @@ int dn_ensure_batch(dn_ctx *c, int want, bool gradient)
     size_t freeb = 0, total = 0;
     HIPCHK(c, hipMemGetInfo(&freeb, &total));
     const size_t budget = (size_t)((double)freeb * 0.85);
-    const int fit = (int)std::max<size_t>(1, budget / std::max<size_t>(per, 1));
+    // second halves of r and q for as many shots as can use them, none where
+    // they would not leave room for one shot
+    const size_t second = (size_t)c->g.plane * 2 * c->g.L * 4;
+    size_t nfit = budget / (per + second);
+    const int nsecond = nfit > 0 ? multi_shots(c) : 0;
+    if (nfit == 0 || nfit > (size_t)nsecond) nfit = (budget - nsecond * second) / per;
+    const int fit = (int)std::max<size_t>(1, nfit);
     cap = std::max(1, std::min(std::min(cap, fit), 4096));
     c->batch_fit = std::min(fit, 4096);
     if (per > budget) return dn_fail(c, "one shot needs %zu MB but only %zu MB of HBM are free", per >> 20, freeb >> 20);
@@ -789,10 +796,12 @@ int dn_ensure_batch(dn_ctx *c, int want, bool gradient)
     HIPCHK(c, dalloc(&c->d_rq, S * P * 2 * std::max(1, g.L)));
     HIPCHK(c, dalloc(&c->d_pvx, S * fw2 * g.ny));
     HIPCHK(c, dalloc(&c->d_pvy, S * fw2 * g.nx));
-    if (multi_capable(c)) {
-        if (g.L > 0) HIPCHK(c, dalloc(&c->d_rq2, S * P * 2 * g.L));
-        HIPCHK(c, dalloc(&c->d_pvx2, S * fw2 * g.ny));
-        HIPCHK(c, dalloc(&c->d_pvy2, S * fw2 * g.nx));
+    c->multi_cap = std::min(cap, nsecond);
+    if (c->multi_cap > 0) {
+        const size_t S2 = (size_t)c->multi_cap;
+        if (g.L > 0) HIPCHK(c, dalloc(&c->d_rq2, S2 * P * 2 * g.L));
+        HIPCHK(c, dalloc(&c->d_pvx2, S2 * fw2 * g.ny));
+        HIPCHK(c, dalloc(&c->d_pvy2, S2 * fw2 * g.nx));
     }
     HIPCHK(c, dalloc(&c->d_seis, S * c->ntr * c->nt_max));
     HIPCHK(c, dalloc(&c->d_resid, S * c->ntr * c->nt_max));
@@ -890,7 +899,7 @@ static int choose_tile(const dn_ctx *c, int nshots)
 // ones scaled by the snapshot before), within multi_limit.
 static bool choose_multi(const dn_ctx *c, int nshots, bool adjoint, bool store, bool hess)
 {
-    if (!multi_capable(c) || choose_tile(c, nshots) == 0) return false;
+    if (nshots > c->multi_cap || choose_tile(c, nshots) == 0) return false;
     if ((adjoint || store) && c->p.snap_precision != 0) return false;
     return (long long)nshots * multi_tiles(c) <= multi_limit(c, adjoint || store || hess);
 }
@@ -993,11 +1002,8 @@ int dn_zero_state(dn_ctx *c, int n)
     }
     HIPCHK(c, launch_fill(c->d_pvx, S * fw2 * g.ny, 0.0f, c->stream));
     HIPCHK(c, launch_fill(c->d_pvy, S * fw2 * g.nx, 0.0f, c->stream));
-    if (c->d_pvx2) {
-        if (c->d_rq2) HIPCHK(c, launch_fill(c->d_rq2, S * P * 2 * g.L, 0.0f, c->stream));
-        HIPCHK(c, launch_fill(c->d_pvx2, S * fw2 * g.ny, 0.0f, c->stream));
-        HIPCHK(c, launch_fill(c->d_pvy2, S * fw2 * g.nx, 0.0f, c->stream));
-    }
+    // the second halves (d_rq2, d_pvx2, d_pvy2) are written by a pass's first
+    // launch, cell by cell, before its second reads them
     return 0;
 }
 

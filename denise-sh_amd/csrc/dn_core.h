@@ -61,7 +61,8 @@ struct dn_ctx {
     float *d_vy[2] = {nullptr, nullptr}, *d_sxy[2] = {nullptr, nullptr}, *d_syz[2] = {nullptr, nullptr};
     float *d_psx[2] = {nullptr, nullptr}, *d_psy[2] = {nullptr, nullptr};
     float *d_rq = nullptr, *d_pvx = nullptr, *d_pvy = nullptr;
-    float *d_rq2 = nullptr, *d_pvx2 = nullptr, *d_pvy2 = nullptr;   // second halves for several steps per launch
+    float *d_rq2 = nullptr, *d_pvx2 = nullptr, *d_pvy2 = nullptr;   // second halves for several steps per launch,
+    int multi_cap = 0;                                              // of the batch's first multi_cap slots
     float *d_seis = nullptr, *d_resid = nullptr, *d_snap = nullptr;
     uint16_t *d_snap16 = nullptr;
     float *d_snap_scale = nullptr, *d_stage = nullptr;

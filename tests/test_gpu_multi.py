@@ -127,3 +127,21 @@ def test_several_steps_of_shallow_free_surface_grids_equal_oracle(nx, ny, fdorde
                    fpml=40.0, fl=FL[:L])
     ref = oracle("f32").gradient(cfg, vs, rho, qs if L else None, si, sj, sig, ri, rj, obs)
     assert np.array_equal(got[2], ref["grad_vs"]) and np.array_equal(got[3], ref["grad_rho"])
+
+
+@pytest.mark.parametrize("nx,ny,fdorder,L,shots", [
+    (70, 40, 4, 2, 34),     # 15 workgroups a shot, 510 of 512: second halves for every shot
+    (70, 40, 4, 2, 35),     # one shot more: tiles, and several steps for one shot alone
+    (60, 24, 8, 3, 29),     # 9 workgroups a shot, 261 of 256
+    (60, 24, 2, 0, 30),
+])
+def test_batches_around_the_second_halves_equal_strips(nx, ny, fdorder, L, shots):
+    say("several steps, batch of", shots, nx, ny, "FDORDER", fdorder, "L", L)
+    par = dict(nx=nx, ny=ny, fdorder=fdorder, L=L, free_surf=0, boundary=0, snap=0, dtinv=2, fw=8)
+    inp = _inputs(nx, ny, shots, 60, seed=shots)
+    dn = product()
+    a = _run(dn, par, inp, 0, False)
+    b = _run(dn, par, inp, 13, False)
+    assert np.isfinite(a[2]).all() and np.abs(a[2]).max() > 0
+    for k, (x, y) in enumerate(zip(a, b)):
+        assert np.array_equal(x, y), "output %d differs" % k
