@@ -18,7 +18,7 @@ struct ConvArgs {
     const uint16_t *mask;      // [n][H][W][Co] or null: output zeroed where mask <= 0
     uint16_t *y16;             // [n][H][W][Co] or null
     float *y1;                 // [n][H][W] fp32 or null: channel 0
-    int rows, hblocks, cols;   // rows per wave, workgroups down and across an image (set by the launcher)
+    int rows, hblocks, strip0; // rows per wave, workgroups per image column, the launch's first (set by the launcher)
 };
 hipError_t launch_conv3x3(const ConvArgs &a, hipStream_t st);
 

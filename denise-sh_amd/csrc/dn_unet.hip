@@ -97,10 +97,10 @@ __global__ __launch_bounds__(256, 2) void k_conv3x3(ConvArgs a)
     __shared__ u8v sw[3 * NKI * 4 * SW];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int nl = lane & 15, kq = lane >> 4;
-    const int strip = blockIdx.x / a.cols, img = strip / a.hblocks, hb = strip - img * a.hblocks;
+    const int strip = a.strip0 + (int)blockIdx.y, img = strip / a.hblocks, hb = strip - img * a.hblocks;
     const int y0 = (hb * 4 + wave) * a.rows, y1 = min(y0 + a.rows, a.H);   // output rows of the wave
-    const int x0 = (blockIdx.x - strip * a.cols) * (16 * NT);
-    const int cg = blockIdx.y * (16 * NM);
+    const int x0 = blockIdx.x * (16 * NT);
+    const int cg = blockIdx.z * (16 * NM);
     const int nmt = min(NM, (a.Co - cg) >> 4);
     for (int e = threadIdx.x; e < 3 * NKI * 4 * 16 * NM; e += 256) {
         const int co = e % (16 * NM), kg = e / (16 * NM);      // kg = ky * 4 NKI + group
@@ -258,7 +258,22 @@ __global__ __launch_bounds__(256, 2) void k_conv3x3(ConvArgs a)
     }
 }
 
-template <int CI, int NM, int NT, bool CAT> static void conv_launch(ConvArgs a, hipStream_t st)
+// The second dimension of a grid takes 65536 workgroups; the rows (strips,
+// images) of a large batch go in several launches: f(first, count).  With the
+// rows in the first dimension, where one launch takes them all, 16 -> 32
+// channels took 20.4 us instead of 17.7 and k_pool_bwd<16> 48 instead of 44
+// (4 x 304 x 1200).
+template <typename F> static hipError_t by_grid_y(long long rows, F f)
+{
+    constexpr long long kMost = 65535;
+    for (long long r0 = 0; r0 < rows; r0 += kMost) {
+        const hipError_t e = f(r0, (unsigned)std::min(kMost, rows - r0));
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+template <int CI, int NM, int NT, bool CAT> static hipError_t conv_launch(ConvArgs a, hipStream_t st)
 {
     // rows per wave: a strip of R rows loads R + 2; shorter where the image
     // would leave CUs without a workgroup
@@ -267,9 +282,11 @@ template <int CI, int NM, int NT, bool CAT> static void conv_launch(ConvArgs a, 
     while (R > 2 && (long long)cols * z * a.n * ((a.H + 4 * R - 1) / (4 * R)) < 1024) R /= 2;
     a.rows = R;
     a.hblocks = (a.H + 4 * R - 1) / (4 * R);
-    a.cols = cols;
-    hipLaunchKernelGGL((k_conv3x3<CI, NM, NT, CAT>), dim3((unsigned)cols * (unsigned)(a.n * a.hblocks), (unsigned)z),
-                       dim3(256), 0, st, a);
+    return by_grid_y((long long)a.n * a.hblocks, [&](long long s0, unsigned strips) {
+        a.strip0 = (int)s0;
+        hipLaunchKernelGGL((k_conv3x3<CI, NM, NT, CAT>), dim3((unsigned)cols, strips, (unsigned)z), dim3(256), 0, st, a);
+        return hipGetLastError();
+    });
 }
 
 hipError_t launch_conv3x3(const ConvArgs &a, hipStream_t st)
@@ -280,23 +297,22 @@ hipError_t launch_conv3x3(const ConvArgs &a, hipStream_t st)
     // (112 input channels: one, its weights would fill the LDS of a CU)
     const int tiles = a.Co / 16, nm = a.Ci == 112 ? 1 : (tiles <= 4 ? tiles : (tiles == 5 ? 3 : 4));
     switch ((a.up ? 10000 : 0) + a.Ci * 10 + nm) {   // the layers and their data gradients
-    case 161: conv_launch<16, 1, 4, false>(a, st); break;
-    case 162: conv_launch<16, 2, 2, false>(a, st); break;
-    case 163: conv_launch<16, 3, 2, false>(a, st); break;
-    case 321: conv_launch<32, 1, 4, false>(a, st); break;
-    case 322: conv_launch<32, 2, 2, false>(a, st); break;
-    case 323: conv_launch<32, 3, 2, false>(a, st); break;
-    case 482: conv_launch<48, 2, 2, false>(a, st); break;
-    case 483: conv_launch<48, 3, 2, false>(a, st); break;
-    case 484: conv_launch<48, 4, 2, false>(a, st); break;
-    case 643: conv_launch<64, 3, 2, false>(a, st); break;
-    case 644: conv_launch<64, 4, 2, false>(a, st); break;
-    case 10481: conv_launch<48, 1, 2, true>(a, st); break;
-    case 10802: conv_launch<80, 2, 2, true>(a, st); break;
-    case 11121: conv_launch<112, 1, 2, true>(a, st); break;
+    case 161: return conv_launch<16, 1, 4, false>(a, st);
+    case 162: return conv_launch<16, 2, 2, false>(a, st);
+    case 163: return conv_launch<16, 3, 2, false>(a, st);
+    case 321: return conv_launch<32, 1, 4, false>(a, st);
+    case 322: return conv_launch<32, 2, 2, false>(a, st);
+    case 323: return conv_launch<32, 3, 2, false>(a, st);
+    case 482: return conv_launch<48, 2, 2, false>(a, st);
+    case 483: return conv_launch<48, 3, 2, false>(a, st);
+    case 484: return conv_launch<48, 4, 2, false>(a, st);
+    case 643: return conv_launch<64, 3, 2, false>(a, st);
+    case 644: return conv_launch<64, 4, 2, false>(a, st);
+    case 10481: return conv_launch<48, 1, 2, true>(a, st);
+    case 10802: return conv_launch<80, 2, 2, true>(a, st);
+    case 11121: return conv_launch<112, 1, 2, true>(a, st);
     default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
@@ -317,7 +333,8 @@ hipError_t launch_conv3x3(const ConvArgs &a, hipStream_t st)
 // allow three taps only (KYS 3) blockIdx.y selects ky, and blockIdx.z a group
 // of NTB input-channel tiles.  Transposing by 2-byte LDS stores, each X row
 // stored for three kx and loaded for three ky, took 140 us (16 -> 16 channels,
-// 4 x 304 x 1200) and 312 us (48 -> 16); now 25 and 49.
+// 4 x 304 x 1200) and 312 us (48 -> 16); now 25 and 49.  Of the layers only
+// 112 -> 48 spills: 8 registers, 20 bytes per lane.
 // ---------------------------------------------------------------------------
 constexpr int kSegPx = 128;    // pixels per segment
 
@@ -580,9 +597,8 @@ hipError_t launch_wgrad(WgradArgs a, float *dw, float *db, hipStream_t st)
 // ---------------------------------------------------------------------------
 // 2x2 average pooling and the adjoints of pooling and nearest upsampling with
 // the ReLU mask of the activation they feed.  Bytes only: one thread per 8
-// channels of a pixel (16-byte accesses), one image row per blockIdx.x, so
-// the only division is by the channel count, a constant (a batch may have more
-// rows than the 65536 workgroups that y and z of a grid take).
+// channels of a pixel (16-byte accesses), one image row per blockIdx.y, so
+// the only division is by the channel count, a constant.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void unpack8(const uint16_t *p, float (&f)[8])
 {
@@ -591,13 +607,13 @@ __device__ __forceinline__ void unpack8(const uint16_t *p, float (&f)[8])
     for (int k = 0; k < 8; ++k) f[k] = u_bf2f(v[k]);
 }
 
-template <int C> __global__ void k_pool(int H, int W, const uint16_t *x, uint16_t *y)
+template <int C> __global__ void k_pool(long long row0, int H, int W, const uint16_t *x, uint16_t *y)
 {
     constexpr int C8 = C / 8;
-    const int w = W / 2, e = blockIdx.y * blockDim.x + threadIdx.x;
+    const int w = W / 2, e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= w * C8) return;
     const int xo = e / C8, c = 8 * (e - xo * C8);
-    const long long row = blockIdx.x;                     // image * H/2 + y
+    const long long row = row0 + blockIdx.y;              // image * H/2 + y
     const uint16_t *b = x + ((2 * row * W + 2 * xo) * C + c);
     float p[8], q[8], r[8], t[8];
     unpack8(b, p);
@@ -612,14 +628,14 @@ template <int C> __global__ void k_pool(int H, int W, const uint16_t *x, uint16_
 
 // dact[p][c] = (act > 0) * (0.25 * dpool[p/2][c] + dcat[p][off + c])
 template <int C>
-__global__ void k_pool_bwd(int H, int W, const uint16_t *dpool, const uint16_t *dcat, int ccat, int off,
-                           const uint16_t *act, uint16_t *dact)
+__global__ void k_pool_bwd(long long row0, int H, int W, const uint16_t *dpool, const uint16_t *dcat, int ccat,
+                           int off, const uint16_t *act, uint16_t *dact)
 {
     constexpr int C8 = C / 8;
-    const int e = blockIdx.y * blockDim.x + threadIdx.x;
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= W * C8) return;
     const int x = e / C8, c = 8 * (e - x * C8);
-    const long long row = blockIdx.x, p = row * W + x;    // row: image * H + y
+    const long long row = row0 + blockIdx.y, p = row * W + x;   // row: image * H + y
     const long long img = row / H, yl = (row - img * H) / 2;
     float dp[8], dc[8], ac[8];
     unpack8(dpool + ((img * (H / 2) + yl) * (W / 2) + x / 2) * C + c, dp);
@@ -633,13 +649,14 @@ __global__ void k_pool_bwd(int H, int W, const uint16_t *dpool, const uint16_t *
 
 // dlow[q][c] = (act_low > 0) * sum over the 2x2 children of dcat[child][c], c < CU
 template <int CU>
-__global__ void k_up_bwd(int H, int W, int Ccat, const uint16_t *dcat, const uint16_t *act_low, uint16_t *dlow)
+__global__ void k_up_bwd(long long row0, int H, int W, int Ccat, const uint16_t *dcat, const uint16_t *act_low,
+                         uint16_t *dlow)
 {
     constexpr int C8 = CU / 8;
-    const int w = W / 2, e = blockIdx.y * blockDim.x + threadIdx.x;
+    const int w = W / 2, e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= w * C8) return;
     const int xo = e / C8, c = 8 * (e - xo * C8);
-    const long long row = blockIdx.x;                     // image * H/2 + y
+    const long long row = row0 + blockIdx.y;              // image * H/2 + y
     const uint16_t *b = dcat + ((2 * row * W + 2 * xo) * Ccat + c);
     const long long q = (row * w + xo) * CU + c;
     float p0[8], p1[8], p2[8], p3[8], ac[8];
@@ -659,53 +676,59 @@ static dim3 grid_for(long long total)
     return dim3((unsigned)std::max<long long>(1, std::min<long long>(8192, (total + 255) / 256)));
 }
 
-static dim3 row_grid(int items, long long rows) { return dim3((unsigned)rows, (unsigned)((items + 255) / 256)); }
-
 hipError_t launch_pool(int n, int H, int W, int C, const uint16_t *x, uint16_t *y, hipStream_t st)
 {
-    const dim3 g = row_grid(W / 2 * (C / 8), (long long)n * (H / 2));
-    switch (C) {
-    case 16: hipLaunchKernelGGL(k_pool<16>, g, dim3(256), 0, st, H, W, x, y); break;
-    case 32: hipLaunchKernelGGL(k_pool<32>, g, dim3(256), 0, st, H, W, x, y); break;
-    case 48: hipLaunchKernelGGL(k_pool<48>, g, dim3(256), 0, st, H, W, x, y); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    const unsigned nb = (unsigned)((W / 2 * (C / 8) + 255) / 256);
+    return by_grid_y((long long)n * (H / 2), [&](long long r0, unsigned rows) {
+        const dim3 g(nb, rows);
+        switch (C) {
+        case 16: hipLaunchKernelGGL(k_pool<16>, g, dim3(256), 0, st, r0, H, W, x, y); break;
+        case 32: hipLaunchKernelGGL(k_pool<32>, g, dim3(256), 0, st, r0, H, W, x, y); break;
+        case 48: hipLaunchKernelGGL(k_pool<48>, g, dim3(256), 0, st, r0, H, W, x, y); break;
+        default: return hipErrorInvalidValue;
+        }
+        return hipGetLastError();
+    });
 }
 hipError_t launch_pool_bwd(int n, int H, int W, int C, const uint16_t *dpool, const uint16_t *dcat, int ccat, int off,
                            const uint16_t *act, uint16_t *dact, hipStream_t st)
 {
-    const dim3 g = row_grid(W * (C / 8), (long long)n * H);
-    switch (C) {
-    case 16: hipLaunchKernelGGL(k_pool_bwd<16>, g, dim3(256), 0, st, H, W, dpool, dcat, ccat, off, act, dact); break;
-    case 32: hipLaunchKernelGGL(k_pool_bwd<32>, g, dim3(256), 0, st, H, W, dpool, dcat, ccat, off, act, dact); break;
-    case 48: hipLaunchKernelGGL(k_pool_bwd<48>, g, dim3(256), 0, st, H, W, dpool, dcat, ccat, off, act, dact); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    const unsigned nb = (unsigned)((W * (C / 8) + 255) / 256);
+    return by_grid_y((long long)n * H, [&](long long r0, unsigned rows) {
+        const dim3 g(nb, rows);
+        switch (C) {
+        case 16: hipLaunchKernelGGL(k_pool_bwd<16>, g, dim3(256), 0, st, r0, H, W, dpool, dcat, ccat, off, act, dact); break;
+        case 32: hipLaunchKernelGGL(k_pool_bwd<32>, g, dim3(256), 0, st, r0, H, W, dpool, dcat, ccat, off, act, dact); break;
+        case 48: hipLaunchKernelGGL(k_pool_bwd<48>, g, dim3(256), 0, st, r0, H, W, dpool, dcat, ccat, off, act, dact); break;
+        default: return hipErrorInvalidValue;
+        }
+        return hipGetLastError();
+    });
 }
 hipError_t launch_up_bwd(int n, int H, int W, int Cu, int Ccat, const uint16_t *dcat, const uint16_t *act_low,
                          uint16_t *dlow, hipStream_t st)
 {
-    const dim3 g = row_grid(W / 2 * (Cu / 8), (long long)n * (H / 2));
-    switch (Cu) {
-    case 32: hipLaunchKernelGGL(k_up_bwd<32>, g, dim3(256), 0, st, H, W, Ccat, dcat, act_low, dlow); break;
-    case 48: hipLaunchKernelGGL(k_up_bwd<48>, g, dim3(256), 0, st, H, W, Ccat, dcat, act_low, dlow); break;
-    case 64: hipLaunchKernelGGL(k_up_bwd<64>, g, dim3(256), 0, st, H, W, Ccat, dcat, act_low, dlow); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    const unsigned nb = (unsigned)((W / 2 * (Cu / 8) + 255) / 256);
+    return by_grid_y((long long)n * (H / 2), [&](long long r0, unsigned rows) {
+        const dim3 g(nb, rows);
+        switch (Cu) {
+        case 32: hipLaunchKernelGGL(k_up_bwd<32>, g, dim3(256), 0, st, r0, H, W, Ccat, dcat, act_low, dlow); break;
+        case 48: hipLaunchKernelGGL(k_up_bwd<48>, g, dim3(256), 0, st, r0, H, W, Ccat, dcat, act_low, dlow); break;
+        case 64: hipLaunchKernelGGL(k_up_bwd<64>, g, dim3(256), 0, st, r0, H, W, Ccat, dcat, act_low, dlow); break;
+        default: return hipErrorInvalidValue;
+        }
+        return hipGetLastError();
+    });
 }
 
 // ---------------------------------------------------------------------------
 // Input packing, output extraction, loss, parameter casts and Adam
 // ---------------------------------------------------------------------------
 // x [n][3][H][W] fp32 (planar) -> [n][H][W][16] bf16 with channels 3..15
-// zero: one pixel per thread, nb workgroups per image
-__global__ void k_pack_input(unsigned nb, long long hw, const float *x, uint16_t *xp)
+// zero: one pixel per thread
+__global__ void k_pack_input(long long im0, long long hw, const float *x, uint16_t *xp)
 {
-    const unsigned im = blockIdx.x / nb;
-    const long long r = (blockIdx.x - im * nb) * (long long)blockDim.x + threadIdx.x;
+    const long long r = blockIdx.x * (long long)blockDim.x + threadIdx.x, im = im0 + blockIdx.y;
     if (r >= hw) return;
     const float *b = x + im * 3 * hw + r;
     const u8v z = u8v{0, 0, 0, 0, 0, 0, 0, 0};
@@ -776,9 +799,10 @@ __global__ void k_adam(long long n, float *w, const float *g, float *m, float *v
 hipError_t launch_pack_input(int n, int H, int W, const float *x, uint16_t *xp, hipStream_t st)
 {
     const long long hw = (long long)H * W;
-    const unsigned nb = (unsigned)((hw + 255) / 256);
-    hipLaunchKernelGGL(k_pack_input, dim3(nb * (unsigned)n), dim3(256), 0, st, nb, hw, x, xp);
-    return hipGetLastError();
+    return by_grid_y(n, [&](long long im0, unsigned images) {
+        hipLaunchKernelGGL(k_pack_input, dim3((unsigned)((hw + 255) / 256), images), dim3(256), 0, st, im0, hw, x, xp);
+        return hipGetLastError();
+    });
 }
 hipError_t launch_mse(long long P, const float *y, const float *t, uint16_t *dy, double *part, int nblocks,
                       hipStream_t st)

@@ -72,11 +72,11 @@ def test_unet_strips_of_several_rows(n, h, w):
             assert rel_l2(g[sl], gr[sl]) < 5e-2, l
 
 
-@pytest.mark.parametrize("copies", [512, 1024])
+@pytest.mark.parametrize("copies", [512, 1024, 4096])
 def test_unet_batches_of_many_rows(copies):
     """More image rows than the 65536 workgroups of a grid's second dimension:
-    69632 and 139264, half of them after pooling.  A batch of copies of 17
-    images gives their outputs' bits and, the scale 2 / pixels being a power
+    69632 and 139264, half of them after pooling; and so many images (forward
+    only).  A batch of copies of 17 images gives their outputs' bits and, the scale 2 / pixels being a power
     of two smaller, their gradient up to the fp32 sums over the partials: at
     most 17408 / 4 terms one after the other, 2.6e-4 of the terms' magnitude."""
     print("unet, many rows", copies)
@@ -88,6 +88,8 @@ def test_unet_batches_of_many_rows(copies):
     y, (loss, g) = net.forward(x), net.loss_grad(x, t)
     xs, ts = np.tile(x, (copies, 1, 1, 1)), np.tile(t, (copies, 1, 1))
     assert np.array_equal(net.forward(xs), np.tile(y, (copies, 1, 1)))
+    if copies > 1024:
+        return
     ls, gs = net.loss_grad(xs, ts)
     assert abs(ls - loss) <= 1e-6 * loss
     assert rel_l2(gs, g) < 1e-3
