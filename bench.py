@@ -596,8 +596,9 @@ def main():
     cells = float(ce[0] + ce[1])
     value = cells / wall / 1e9
     # dominant kernel: the fused step (all but a fraction of a percent of the
-    # GPU time; k_tile, or k_step where a launch shape of the strips is asked
-    # for), over the launches of both passes: the
+    # GPU time; k_step where a launch shape of the strips is asked for, k_multi
+    # where a launch updates a cell several times, otherwise k_tile), over the
+    # launches of both passes: the
     # forward pass moves 84 + 20/DTINV bytes per cell-update, the adjoint
     # 84 + 36/DTINV (14/DTINV and 30/DTINV with 16-bit snapshots)
     nla = max(la[0] + la[1], 1)
@@ -610,7 +611,10 @@ def main():
     achieved = units_per_launch * bytes_per_cell / (per_launch_ms * 1e-3) / 1e9
     full = W["nt"] == (12000 if args.config == "c4" else 10000)
     shape = ctx.launch_shape()
-    tiles = shape[0] == 0 and shape[2] == 1 and shape[3] == 1
+    strips = shape[0] > 0 or shape[2] > 1 or shape[3] > 1
+    kernels = sorted(set("k_step" if strips else
+                         "k_multi" if ce[p] > 1.01 * la[p] * batch * W["nx"] * W["ny"] else "k_tile" for p in (0, 1)))
+    tiles = kernels == ["k_tile"]
     traffic = measured_traffic(W, batch, units_per_launch) if (prec == 0 and full and tiles) else None
     out = {
         "metric": "Gcell-updates/s fwd+adj",
@@ -632,17 +636,15 @@ def main():
                    else "gradient over all %d shots" % nshots},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "kernel": "%s<4,visco> (forward and adjoint launches of the gradient)"
-                     % ("k_tile" if tiles else "k_step"),
+                     "kernel": "%s<4,visco> (forward and adjoint launches of the gradient)" % ", ".join(kernels),
                      "ms_per_launch": round(per_launch_ms, 4), "bytes_per_cell_update": round(bytes_per_cell, 3),
                      "cell_updates_per_launch": units_per_launch},
         "misfit_l2": l2,
     }
     if tuned is not None:
-        shape = ctx.launch_shape()
         out["config"]["rows_per_segment"], out["config"]["graph_steps"] = shape[0], shape[1]
         out["config"]["tuned"] = {"rows_per_segment": shape[0], "graph_steps": shape[1], "wave_shots": shape[2],
-                                  "group_shots": shape[3], "note": "rows 0: the cost model's choice per batch"}
+                                  "group_shots": shape[3], "note": "rows 0: %s" % ("the cost model's choice per batch" if strips else "tiles")}
     elif args.rows:
         out["config"]["rows_per_segment"] = args.rows
     if args.max_batch:
@@ -650,15 +652,15 @@ def main():
     out["config"]["exec"] = args.exec
     out["config"]["batch_order"] = args.batch_order
     out["config"]["wave_shots"] = "tuned" if args.autotune else args.wave_shots
-    out["config"]["group_layout"] = "tuned" if args.autotune else (
+    out["config"]["group_layout"] = "tuned" if args.autotune else "tiles" if not strips else (
         "8 strips x 1 shot" if args.layout == 0 else "%d strips x %d shots" % (8 // (8 if args.layout == 1 else args.layout),
                                                                           8 if args.layout == 1 else args.layout))
     if args.compare_sequential:
         # the same gradient with one shot per batch: the per-shot sequential
         # GPU loop the batched launch replaces (the reference's shot loop,
-        # denise.c:875), with the default launch shape for one shot (eight
-        # strips per workgroup, one shot per wave; a layout tuned for the
-        # batch could leave waves idle here)
+        # denise.c:875), with the default launch shape for one shot (tiles, or
+        # with --rows eight strips per workgroup; a layout tuned for the batch
+        # could leave waves idle here)
         ctx.set_batch(1, args.rows)
         ctx.set_group_layout(0)
         ctx.set_wave_shots(1)

@@ -354,7 +354,8 @@ class Context:
         self._chk(lib().dn_set_group_layout(self._h, mode))
 
     def launch_shape(self):
-        """(rows per segment (0: cost model), graph steps, shots per wave, shots per workgroup)."""
+        """(rows per segment, graph steps, shots per wave, shots per workgroup); 0, _, 1, 1: the automatic
+        choice (tiles, or several steps per launch on small grids), otherwise strips."""
         v = [C.c_int() for _ in range(4)]
         lib().dn_get_launch_shape.argtypes = [C.c_void_p] + [C.POINTER(C.c_int)] * 4
         self._chk(lib().dn_get_launch_shape(self._h, *[C.byref(x) for x in v]))

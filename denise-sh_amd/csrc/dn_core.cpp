@@ -711,16 +711,23 @@ extern "C" int dn_autotune(dn_ctx *c, int nshots, int nsteps, int *rows_out, int
 // Microseconds per step, tiles / several steps, forward and gradient, by
 // workgroups (1: 400x120, 255; 2: two such shots, 510):
 // FDORDER 2       1 5.4 / 1.5, 6.3 / 2.1   800x480 (2040) 7.7 / 4.9, 10.7 / 8.5
+//   with L 1      1 5.7 / 1.6, 6.3 / 2.1   800x480 8.5 / 5.2, 11.9 / 8.9
+//   with L 2                               800x480 8.8 / 5.6, 10.6 / 8.2
 //   with L 3                               800x480 9.4 / 6.0, 12.4 / 9.5
 // FDORDER 4       1 5.5 / 2.5, 6.6 / 3.2   2 5.7 / 3.3, 6.9 / 5.0
 //   750 (700x200) 5.8 / 4.5, 7.3 / 6.7     1020 6.5 / 5.2, 8.1 / 8.3
 //   with L 2      1 5.7 / 2.7, 6.5 / 3.5   2 5.8 / 4.7, 6.9 / 5.9
 //   with L 2, 625 (600x200) 5.7 / 6.2, 6.9 / 8.0
+//   with L 1      1 5.7 / 2.6, 6.7 / 3.4   2 5.9 / 3.5, 7.3 / 5.9
+//   with L 3      1 5.6 / 2.9, 6.4 / 3.5   2 5.8 / 5.0, 6.9 / 6.1
 // FDORDER 6       1 5.6 / 3.3, 6.5 / 4.0   420 (500x160) 5.6 / 4.3, 6.6 / 6.8
 //   with L 2      1 5.9 / 3.6, 6.8 / 4.4   420, two steps 5.9 / 6.2, 7.0 / 7.8
+//   with L 1, 3   1 5.6 / 3.4, 6.5 / 4.2   1 5.8 / 3.8, 6.7 / 4.6
 // FDORDER 8       1 5.8 / 4.0, 6.6 / 5.0   2 5.9 / 5.4, 6.9 / 8.6
 //   with L 2      1 6.0 / 4.4, 6.9 / 5.4   420 6.0 / 7.5, 7.1 / 9.1
-// Beyond FDORDER 8 a second step reaches too many cells.
+//   with L 1, 3   1 5.7 / 4.2, 6.5 / 5.2   1 6.0 / 4.6, 6.7 / 5.6
+// Beyond FDORDER 8 a second step reaches too many cells; for L 4 the kernel is
+// neither built nor measured.
 static int multi_limit(const dn_ctx *c, bool extra)
 {
     if (c->K > kMultiMaxK || c->p.L > kMultiMaxL) return 0;

@@ -10,13 +10,19 @@ namespace dn {
 constexpr int kWave = 64;      // CDNA wavefront width: one wave per strip
 constexpr int kStripsPerGroup = 8;   // waves (adjacent strips) per workgroup of the time step
 constexpr int kMaxL = 4;       // relaxation mechanisms supported
-// Zero frame around the interior of every padded field.  The fused step
+constexpr int kMaxK = 6;       // stencil half-orders 1..6 (FDORDER 2..12)
+// Zero frame around the interior of every padded field.  The strip step
 // reads up to 2K-1 rows above/below the interior, 2K-1 columns left of it
-// and 63 right of it (the last strip's wave), K <= 6.
+// and 63 right of it (the last strip's wave).  A tile reads 2K-1 rows and
+// columns around its 64 columns x 8 or 16 rows: up to 64 + 2K - 2 columns past
+// its first, which may be nx; rows end on 128-byte lines, so they hold them.
+// Rows beyond the frame are clamped to its last but one.
 constexpr int kPadX = 32;      // columns left of i = 1 (rows start on a 128-byte line)
 constexpr int kPadR = 64;      // columns right of i = nx (at least)
 constexpr int kPadY = 12;      // rows above j = 1 and below j = ny
-
+// nx = 1 (or 64 m + 1) leaves the least room behind the last tile's first column
+static_assert(kPadX + 1 + kWave + 2 * kMaxK - 2 <= (1 + kPadX + kPadR + 31) / 32 * 32, "a tile's columns lie in the row");
+static_assert(kPadY >= 2 * kMaxK && kPadX >= 2 * kMaxK, "the frame holds a stencil's reach above and to the left");
 
 // Padded, x-fastest layout of one 2-D field.  Element (j,i) of the
 // reference's index space (1-based interior) lives at

@@ -24,8 +24,10 @@
 // 1.64, 1.46, 1.57 us per step; FDORDER 6 with 2, 3 3.44, 3.29.  The CPML
 // profiles lie in LDS, not in registers, and the elastic kernels of FDORDER 2
 // and 4 are held to 80 registers: two workgroups share a CU (500 x 160: 4.09
-// -> 3.22 us per step, gradient 5.31 -> 4.86); not the correlating one, which
-// spilled at that limit (+12 % at 400 x 120).
+// -> 3.22 us per step, gradient 5.31 -> 4.86).  At that limit the storing one
+// of FDORDER 4 spills one vector register (8 bytes) and 40 scalar ones into
+// lanes of vector registers; the correlating one spilled 23 (+12 % at 400 x
+// 120) and is not held to it.
 //
 // Everything the cells around the tile read is double-buffered (here also the
 // stress CPML memory and the relaxation variables, which the single steps

@@ -314,13 +314,15 @@ int dn_set_group_layout(dn_ctx *ctx, int mode);
  * workgroup layouts (at the cost model's, half, equal and double the rows)
  * and graph replay (kept unless eager launches are more than 2 % faster),
  * each the faster of two timed passes; keeps the fastest setting and
- * returns rows (0: the cost model's) and graph use. */
+ * returns rows (0: the automatic choice) and graph use. */
 int dn_autotune(dn_ctx *ctx, int nshots, int nsteps, int *rows_per_segment, int *graph_steps);
 /* The launch shape in use (set by dn_set_batch / dn_set_exec /
  * dn_set_wave_shots / dn_set_group_layout or chosen by dn_autotune): rows per
- * segment (0: the cost model's choice per batch), graph steps, shots per wave
- * and shots per workgroup (1: eight adjacent strips of one shot).  No
- * counterpart in the reference. */
+ * segment, graph steps, shots per wave and shots per workgroup.  Rows 0 with
+ * one shot per wave and per workgroup: the automatic choice per batch, tiles
+ * or, on small grids, several steps per launch (strips on narrow periodic
+ * grids); otherwise strips (rows 0: the cost model's; one shot per workgroup:
+ * eight adjacent strips of it).  No counterpart in the reference. */
 int dn_get_launch_shape(const dn_ctx *ctx, int *rows_per_segment, int *graph_steps, int *wave_shots,
                         int *group_shots);
 
